@@ -11,8 +11,8 @@ objects (state-dict keys and weight tying unchanged):
 
 * ``FusedEmbedding`` — forward ``fh_embedding_fwd`` (row gather; ids outside
   [0, vocab) give zero rows, as VocabParallelEmbedding at one rank does),
-  backward ``fh_embedding_bwd`` (deterministic scatter-add: stable radix sort
-  of the ids, fp32 sums in token order, no floating-point atomics; skips
+  backward ``fh_embedding_bwd`` (deterministic scatter-add: tokens grouped by
+  id, fp32 sums in token order, no floating-point atomics; skips
   nn.Embedding's ``padding_idx``).
 * ``FusedRMSNorm`` — the same ``fh_rmsnorm_fwd`` / ``fh_rmsnorm_bwd`` kernels
   the checkpointed layers use, saving only the input.

@@ -327,8 +327,8 @@ size_t fh_embedding_bwd_workspace_size(int64_t n_tokens, int64_t vocab);
  * dy[t, :], accumulated in fp32 in ascending t and rounded once; every row of
  * dweight [vocab, hidden] is written (zeros for ids no token uses).  Tokens
  * whose id is outside [0, vocab) or equals padding_idx (nn.Embedding's; pass
- * -1 for none) contribute nothing.  Deterministic: a stable radix sort of the
- * ids, no floating-point atomics; n_tokens, vocab < 2^31.
+ * -1 for none) contribute nothing.  Deterministic: the tokens are grouped by id
+ * in token order, no floating-point atomics; n_tokens, vocab < 2^31.
  */
 int fh_embedding_bwd(fh_dtype dt, const void* dy, const int64_t* ids, void* dweight,
                      int64_t n_tokens, int64_t vocab, int64_t hidden, int64_t padding_idx,

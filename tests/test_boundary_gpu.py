@@ -66,6 +66,28 @@ def test_embedding_bwd_ordered_exact(dtype, T, V, H, pad, bad, hot):
     assert torch.equal(got, want32.to(dtype))
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("T,V,H", [
+    (7, 5, 8), (8, 1, 136), (9, 1, 128),        # either side of the frequent-id split, one id
+    (1023, 513, 264), (1025, 512, 8),           # waves with a ragged or an empty share of the tokens
+    (65536, 600, 8), (65537, 600, 8),           # the last size grouped in one launch, the first sorted
+    (2000, 524288, 8), (2000, 524296, 8),       # the same for the vocabulary
+])
+def test_embedding_bwd_zipf_ids_ordered_exact(dtype, T, V, H):
+    """Text-like ids (P(rank r) ~ 1/r, a few ids in much of the batch), some out of
+    range, one padded: bit-exact against the fp32 sums in token order."""
+    from femtotron_amd import ops
+    g = np.random.default_rng(T + V)
+    ids = np.minimum(np.exp(g.random(T) * np.log(V + 1.0)).astype(np.int64), V) - 1
+    ids[g.random(T) < 0.02] = -1
+    ids[g.random(T) < 0.02] = V
+    pad = None if V == 1 else V // 2
+    dy = torch.randn(T, H, generator=torch.Generator().manual_seed(T)).to(dtype)
+    got = ops.embedding_bwd(dy.to(DEV), torch.from_numpy(ids).to(DEV), V, pad).cpu()
+    want32 = torch.from_numpy(oe.embedding_bwd_ordered(dy.float().numpy(), ids, V, pad))
+    assert torch.equal(got, want32.to(dtype))
+
+
 def test_embedding_bwd_tinyllama_vs_torch_and_deterministic():
     """TinyLlama step shape (16384 tokens, V = 32000, H = 2048, bf16): within one
     bf16 ulp of torch's F.embedding backward on the GPU and of the fp64 sums;
