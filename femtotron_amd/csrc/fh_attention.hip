@@ -477,31 +477,6 @@ __global__ __launch_bounds__(256 * HPB) __attribute__((amdgpu_waves_per_eu(2))) 
   }
 }
 
-// --------------------------------------- backward: delta = rowsum(dO*O), fp32
-template <typename T>
-__global__ __launch_bounds__(256) void k_attn_delta(const T* __restrict__ o, int64_t ldo,
-                                                    const T* __restrict__ dO, int64_t lddo,
-                                                    float* __restrict__ delta, int S, int nh,
-                                                    int hd, int64_t tokens) {
-  const int64_t idx = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (idx >= tokens * nh) return;
-  const int64_t t = idx / nh;
-  const int h = static_cast<int>(idx - t * nh);
-  const T* orow = o + t * ldo + static_cast<int64_t>(h) * hd;
-  const T* grow = dO + t * lddo + static_cast<int64_t>(h) * hd;
-  float acc = 0.f;
-  for (int d = 0; d < hd; d += 8) {
-    float a[8], g[8];
-    Elem<T>::load8(orow + d, a);
-    Elem<T>::load8(grow + d, g);
-#pragma unroll
-    for (int j = 0; j < 8; ++j) acc = fmaf(a[j], g[j], acc);
-  }
-  const int64_t b = t / S;
-  const int s = static_cast<int>(t - b * S);
-  delta[(b * nh + h) * S + s] = acc;
-}
-
 // ------------------------------------------------------- backward: dQ (bf16)
 // Same tiling as the forward with one 32-query tile per wave:
 //   S^T = K Q^T, P^T = exp(S^T - lse), dP^T = V dO^T,
@@ -1061,152 +1036,403 @@ __global__ __launch_bounds__(DkdvTiles<HD>::NT) __attribute__((amdgpu_waves_per_
   }
 }
 
-// --------------------------------------------------------- fp32 reference-precision kernels
-// Plain fp32 FMA kernels (one thread per output row) for fp32 models; the same
-// algorithm (online softmax forward with lse, delta-based backward) as above.
+// ------------------------------------------------------------- fp32 kernels
+// fp32 models: the same algorithm (online softmax forward with lse, delta-based
+// backward) on v_mfma_f32_16x16x4_f32, whose products and sums are fp32.
+//
+// Lane i of an operand holds row / column r = i%16 and k index c = i/16 of
+// four; lane i of the accumulator holds column r and rows 4c .. 4c+3.  Two
+// operand forms, both read straight from global memory (a tile's rows come
+// from L2 / L1; LDS only combines the waves' results):
+//   * contraction over head dims ("frag"): lane (r, c) loads float4s of row r at
+//     dims 16u + 4c, i.e. product (u, e) contracts dims 16u + 4c + e, c = 0..3:
+//     the k order is permuted alike in both operands;
+//   * contraction over rows ("wsum": P V, dS K, P^T dO, dS^T Q): the weights are
+//     accumulator entries, so product (t, e) contracts rows 16t + 4c + e; lane
+//     (r, c) loads dims ND*r .. ND*r + ND-1 (ND = HD/16) of that row, one dim
+//     for each of the ND accumulators.
+// The forward and dQ take 16 queries of one head per workgroup, their key
+// blocks of 32 shared out over 4 waves; dK/dV takes 16 keys of one kv head, the
+// (query block of 32, query head) items shared out over 8 or 16 waves.  So even
+// one short sequence is many waves: one thread per query (or key) row, each
+// walking its keys (or all the group's queries) alone, took 804 / 569 / 15081 us
+// (forward / dQ / dK+dV) at 1 x 512 tokens, 32 / 4 heads of 64, and 180 / 101 /
+// 170 us at 2 x 128 tokens, 8 / 4 heads of 32; these take 34 / 53 / 133 and 6 / 6 /
+// 11 us.
+__device__ __forceinline__ f32x4 mfma_f32(float a, float b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
 
-// out[d] = acc[d] * mul, followed by the RoPE backward of the row when
-// rope.cos is set (the fp32 counterpart of store_grad_row).
+__device__ __forceinline__ f32x4 zero4() { return f32x4{0.f, 0.f, 0.f, 0.f}; }
+
+// max / sum over the four lanes that share a column (same r, c = 0..3).
+__device__ __forceinline__ float col_max(float v) {
+  v = fmaxf(v, __shfl_xor(v, 16, kWave));
+  return fmaxf(v, __shfl_xor(v, 32, kWave));
+}
+__device__ __forceinline__ float col_sum(float v) {
+  v += __shfl_xor(v, 16, kWave);
+  return v + __shfl_xor(v, 32, kWave);
+}
+
 template <int HD>
-__device__ __forceinline__ void store_row_f32(float* out, const float (&acc)[HD], float mul,
-                                              const RopeRows<float>& rope, int64_t tok0, int pos) {
-  if (!rope.cos) {
-    for (int d = 0; d < HD; ++d) out[d] = acc[d] * mul;
-    return;
-  }
-  const int64_t r = rope.row(tok0, pos) * HD;
-  const float* cs = rope.cos + r;
-  const float* sn = rope.sin + r;
-  for (int d = 0; d < HD / 2; ++d) {
-    float o0, o1;
-    rope_pair<float, true>(acc[d] * mul, acc[d + HD / 2] * mul, cs[d], cs[d + HD / 2], sn[d], sn[d + HD / 2],
-                           o0, o1);
-    out[d] = o0;
-    out[d + HD / 2] = o1;
+using FragF32 = f32x4[HD / 16];
+
+template <int HD>
+__device__ __forceinline__ void load_frag_f32(FragF32<HD>& f, const float* row, int c) {
+#pragma unroll
+  for (int u = 0; u < HD / 16; ++u) f[u] = *reinterpret_cast<const f32x4*>(row + 16 * u + 4 * c);
+}
+
+// a b^T over the head dims: accumulator rows = a's rows, columns = b's rows.
+template <int HD>
+__device__ __forceinline__ f32x4 dot_f32(const FragF32<HD>& a, const FragF32<HD>& b) {
+  f32x4 acc = zero4();
+#pragma unroll
+  for (int u = 0; u < HD / 16; ++u)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) acc = mfma_f32(a[u][e], b[u][e], acc);
+  return acc;
+}
+
+// acc[dt] (rows m: dim ND*m + dt, columns as w's) += sum over the block's 32 rows
+// of row[.][dim] * w[row][column]; row n of the block is rows + min(n, last) * ld.
+// Rows with n outside [lo, hi) of this lane's column are masked (their w is 0).
+// `partial`: some row is masked for some column.  There a row that holds an
+// infinity or a NaN must not reach the columns that do not see it (0 * inf), so
+// 16 rows with one are summed row by row on the vector unit.
+template <int HD>
+__device__ __forceinline__ void wsum_f32(f32x4 (&acc)[HD / 16], const f32x4 (&w)[2], const float* rows, int64_t ld,
+                                         int last, bool partial, int lo, int hi, int r, int c) {
+  constexpr int ND = HD / 16;
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    float v[4][ND];
+    bool bad = false;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float* src = rows + min(16 * t + 4 * c + e, last) * ld + ND * r;
+#pragma unroll
+      for (int d = 0; d < ND; d += 2) {
+        const float2 p = *reinterpret_cast<const float2*>(src + d);
+        v[e][d] = p.x;
+        v[e][d + 1] = p.y;
+        bad |= !(fabsf(p.x) < INFINITY) || !(fabsf(p.y) < INFINITY);
+      }
+    }
+    if (partial && wave_any(bad)) {
+      for (int n = 0; n < 16; ++n) {
+        const int e = n & 3;
+        const float mine = e == 0 ? w[t][0] : e == 1 ? w[t][1] : e == 2 ? w[t][2] : w[t][3];
+        const float p = __shfl(mine, r + 16 * (n >> 2), kWave);
+        if (16 * t + n < lo || 16 * t + n >= hi) continue;
+        const float* src = rows + min(16 * t + n, last) * ld + 4 * ND * c;
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+#pragma unroll
+          for (int dt = 0; dt < ND; ++dt) acc[dt][g] = fmaf(p, src[ND * g + dt], acc[dt][g]);
+      }
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int dt = 0; dt < ND; ++dt) acc[dt] = mfma_f32(v[e][dt], w[t][e], acc[dt]);
+    }
   }
 }
+
+// A wave's accumulators into an LDS tile [16 columns][HD + 4] (one row per
+// accumulator column).
 template <int HD>
-__global__ __launch_bounds__(128) void k_attn_fwd_f32(
+__device__ __forceinline__ void put_tile_f32(float* tile, const f32x4 (&acc)[HD / 16], int r, int c) {
+  constexpr int ND = HD / 16;
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+#pragma unroll
+    for (int dt = 0; dt < ND; ++dt) tile[r * (HD + 4) + ND * (4 * c + e) + dt] = acc[dt][e];
+}
+
+template <int HD>
+__device__ __forceinline__ void add_tile_f32(f32x4 (&acc)[HD / 16], const float* tile, int r, int c) {
+  constexpr int ND = HD / 16;
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+#pragma unroll
+    for (int dt = 0; dt < ND; ++dt) acc[dt][e] += tile[r * (HD + 4) + ND * (4 * c + e) + dt];
+}
+
+// Sums the NW waves' accumulators into wave 0's, pairs of waves in a fixed order.
+template <int HD, int NW>
+__device__ __forceinline__ void sum_waves_f32(f32x4 (&acc)[HD / 16], float* tiles, int wave, int r, int c) {
+  constexpr int TILE = 16 * (HD + 4);
+#pragma unroll
+  for (int half = NW / 2; half > 0; half >>= 1) {
+    if (wave >= half && wave < 2 * half) put_tile_f32<HD>(tiles + (wave - half) * TILE, acc, r, c);
+    __syncthreads();
+    if (wave < half) add_tile_f32<HD>(acc, tiles + wave * TILE, r, c);
+    __syncthreads();
+  }
+}
+
+// Rows pos0 .. pos0 + 15 (those before S) of an output from an LDS tile, times
+// mul, followed by the RoPE backward of each row when rope.cos is set.
+template <int HD, int NT>
+__device__ __forceinline__ void store_tile_f32(float* out, int64_t ld, const float* tile, int pos0, int S, float mul,
+                                               const RopeRows<float>& rope, int64_t tok0) {
+  for (int i = threadIdx.x; i < 16 * (HD / 2); i += NT) {
+    const int row = i / (HD / 2), d = i % (HD / 2), pos = pos0 + row;
+    if (pos >= S) break;  // rows ascend with i
+    float o0 = tile[row * (HD + 4) + d] * mul, o1 = tile[row * (HD + 4) + d + HD / 2] * mul;
+    if (rope.cos) {
+      const int64_t t = rope.row(tok0, pos) * HD + d;
+      rope_pair<float, true>(o0, o1, rope.cos[t], rope.cos[t + HD / 2], rope.sin[t], rope.sin[t + HD / 2], o0, o1);
+    }
+    float* dst = out + (tok0 + pos) * ld + d;
+    dst[0] = o0;
+    dst[HD / 2] = o1;
+  }
+}
+
+// q and qout may be the same buffer: every wave has read the workgroup's
+// queries before wave 0 writes them back.
+template <int HD>
+__global__ __launch_bounds__(256) void k_attn_fwd_f32(
     const float* q, int64_t ldq, const float* __restrict__ k, int64_t ldk,
     const float* __restrict__ v, int64_t ldv, float* __restrict__ o, int64_t ldo,
-    float* __restrict__ lse, int S, int nh, int group, float scale, int64_t rows, RopeRows<float> rope,
-    float* qout, int64_t ldqo) {  // q and qout may alias (in-place rotated q)
-  const int64_t idx = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (idx >= rows) return;  // rows = B*nh*S, idx = (b*nh + h)*S + s
-  const int s = static_cast<int>(idx % S);
-  const int64_t bh = idx / S;
-  const int h = static_cast<int>(bh % nh);
-  const int64_t b = bh / nh;
-  const int kvh = h / group;
-  const float* qr = q + (b * S + s) * ldq + static_cast<int64_t>(h) * HD;
-  float qv[HD], acc[HD];
-  for (int d = 0; d < HD; ++d) { qv[d] = qr[d]; acc[d] = 0.f; }
-  if (rope.cos) {  // q rotated on load (RoPE forward), optionally written back
-    const int64_t r = rope.row(b * S, s) * HD;
-    float* qo = qout ? qout + (b * S + s) * ldqo + static_cast<int64_t>(h) * HD : nullptr;
-    for (int d = 0; d < HD / 2; ++d) {
-      float o0, o1;
-      rope_pair<float, false>(qv[d], qv[d + HD / 2], rope.cos[r + d], rope.cos[r + d + HD / 2], rope.sin[r + d],
-                              rope.sin[r + d + HD / 2], o0, o1);
-      qv[d] = o0;
-      qv[d + HD / 2] = o1;
-      if (qo) {
-        qo[d] = o0;
-        qo[d + HD / 2] = o1;
+    float* __restrict__ lse, int S, int nh, int group, float scale_log2, RopeRows<float> rope,
+    float* qout, int64_t ldqo) {
+  constexpr int NU = HD / 16, TILE = 16 * (HD + 4);
+  __shared__ __align__(16) float tiles[2 * TILE];
+  __shared__ float sm[4][16], sl[4][16];
+  const int lane = threadIdx.x & 63, r = lane & 15, c = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int bh = blockIdx.y, b = bh / nh, h = bh - b * nh, kvh = h / group;
+  const int q0 = static_cast<int>(gridDim.x - 1 - blockIdx.x) * 16, qi = q0 + r;  // latest queries (most keys) first
+  const int64_t tok0 = static_cast<int64_t>(b) * S;
+  const int qc = min(qi, S - 1);
+
+  FragF32<HD> qf;
+  load_frag_f32<HD>(qf, q + (tok0 + qc) * ldq + static_cast<int64_t>(h) * HD, c);
+  if (rope.cos) {
+    const int64_t t = rope.row(tok0, qc) * HD + 4 * c;
+#pragma unroll
+    for (int u = 0; u < NU / 2; ++u)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int64_t d = t + 16 * u + e;
+        float o0, o1;
+        rope_pair<float, false>(qf[u][e], qf[u + NU / 2][e], rope.cos[d], rope.cos[d + HD / 2], rope.sin[d],
+                                rope.sin[d + HD / 2], o0, o1);
+        qf[u][e] = o0;
+        qf[u + NU / 2][e] = o1;
       }
+    __syncthreads();
+    if (qout != nullptr && wave == 0 && qi < S) {
+      float* dst = qout + (tok0 + qi) * ldqo + static_cast<int64_t>(h) * HD + 4 * c;
+#pragma unroll
+      for (int u = 0; u < NU; ++u) *reinterpret_cast<f32x4*>(dst + 16 * u) = qf[u];
     }
   }
+  f32x4 oacc[NU];
+#pragma unroll
+  for (int dt = 0; dt < NU; ++dt) oacc[dt] = zero4();
   float m = -INFINITY, l = 0.f;
-  for (int j = 0; j <= s; ++j) {
-    const float* kr = k + (b * S + j) * ldk + static_cast<int64_t>(kvh) * HD;
-    const float* vr = v + (b * S + j) * ldv + static_cast<int64_t>(kvh) * HD;
-    float x = 0.f;
-    for (int d = 0; d < HD; ++d) x = fmaf(qv[d], kr[d], x);
-    x *= scale;
-    const float mn = fmaxf(m, x);
-    const float a = expf(m - mn), p = expf(x - mn);
-    l = l * a + p;
-    for (int d = 0; d < HD; ++d) acc[d] = acc[d] * a + p * vr[d];
+  const int kend = min(S, q0 + 16), nkb = (kend + 31) / 32;
+  const float* kp = k + tok0 * ldk + static_cast<int64_t>(kvh) * HD;
+  const float* vp = v + tok0 * ldv + static_cast<int64_t>(kvh) * HD;
+  for (int kb = wave; kb < nkb; kb += 4) {
+    const int k0 = kb * 32;
+    f32x4 x[2];  // rows = keys, column = query
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      FragF32<HD> kf;
+      load_frag_f32<HD>(kf, kp + static_cast<int64_t>(min(k0 + 16 * t + r, S - 1)) * ldk, c);
+      x[t] = dot_f32<HD>(kf, qf);
+    }
+    const int hi = min(qi, S - 1) + 1 - k0;  // keys n of the block with n < hi are seen by this query
+    float mloc = -INFINITY;
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (16 * t + 4 * c + e < hi) mloc = fmaxf(mloc, x[t][e] * scale_log2);
+    const float mn = fmaxf(m, col_max(mloc));
+    const float alpha = fast_exp2(m - mn);
     m = mn;
+    l *= alpha;
+#pragma unroll
+    for (int dt = 0; dt < NU; ++dt) oacc[dt] *= alpha;
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        x[t][e] = 16 * t + 4 * c + e < hi ? fast_exp2(fmaf(x[t][e], scale_log2, -mn)) : 0.f;
+        l += x[t][e];
+      }
+    wsum_f32<HD>(oacc, x, vp + static_cast<int64_t>(k0) * ldv, ldv, S - 1 - k0, k0 + 31 > q0, 0, hi, r, c);
   }
-  float* orow = o + (b * S + s) * ldo + static_cast<int64_t>(h) * HD;
-  for (int d = 0; d < HD; ++d) orow[d] = acc[d] / l;
-  if (lse != nullptr) lse[idx] = m + logf(l);
+  // The waves' results meet: weights 2^(m_w - m), zero for a wave without keys.
+  l = col_sum(l);
+  if (c == 0) {
+    sm[wave][r] = m;
+    sl[wave][r] = l;
+  }
+  __syncthreads();
+  const float mt = fmaxf(fmaxf(sm[0][r], sm[1][r]), fmaxf(sm[2][r], sm[3][r]));
+  float lt = 0.f;
+#pragma unroll
+  for (int w = 0; w < 4; ++w) lt += sl[w][r] * fast_exp2(sm[w][r] - mt);
+  const float mul = fast_exp2(m - mt) / lt;
+#pragma unroll
+  for (int dt = 0; dt < NU; ++dt) oacc[dt] *= mul;
+  sum_waves_f32<HD, 4>(oacc, tiles, wave, r, c);
+  if (wave == 0) {
+    put_tile_f32<HD>(tiles, oacc, r, c);
+    if (lse != nullptr && c == 0 && qi < S) lse[static_cast<int64_t>(bh) * S + qi] = (mt + log2f(lt)) * kLn2;
+  }
+  __syncthreads();
+  store_tile_f32<HD, 256>(o + static_cast<int64_t>(h) * HD, ldo, tiles, q0, S, 1.f, RopeRows<float>{nullptr, nullptr, 0},
+                          tok0);
 }
 
+// Also writes delta = rowsum(dO * O) and -lse * log2(e) of its queries for the
+// dK/dV kernel, which runs next on the same stream.
 template <int HD>
-__global__ __launch_bounds__(128) void k_attn_bwd_dq_f32(
+__global__ __launch_bounds__(256) void k_attn_bwd_dq_f32(
     const float* __restrict__ q, int64_t ldq, const float* __restrict__ k, int64_t ldk,
-    const float* __restrict__ v, int64_t ldv, const float* __restrict__ dO, int64_t lddo,
-    const float* __restrict__ lse, const float* __restrict__ delta, float* __restrict__ dq,
-    int64_t lddq, int S, int nh, int group, float scale, int64_t rows, RopeRows<float> rope) {
-  const int64_t idx = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (idx >= rows) return;
-  const int s = static_cast<int>(idx % S);
-  const int64_t bh = idx / S;
-  const int h = static_cast<int>(bh % nh);
-  const int64_t b = bh / nh;
-  const int kvh = h / group;
-  const float* qr = q + (b * S + s) * ldq + static_cast<int64_t>(h) * HD;
-  const float* gr = dO + (b * S + s) * lddo + static_cast<int64_t>(h) * HD;
-  float qv[HD], gv[HD], acc[HD];
-  for (int d = 0; d < HD; ++d) { qv[d] = qr[d]; gv[d] = gr[d]; acc[d] = 0.f; }
-  const float L = lse[idx], D = delta[idx];
-  for (int j = 0; j <= s; ++j) {
-    const float* kr = k + (b * S + j) * ldk + static_cast<int64_t>(kvh) * HD;
-    const float* vr = v + (b * S + j) * ldv + static_cast<int64_t>(kvh) * HD;
-    float x = 0.f, dp = 0.f;
-    for (int d = 0; d < HD; ++d) {
-      x = fmaf(qv[d], kr[d], x);
-      dp = fmaf(gv[d], vr[d], dp);
+    const float* __restrict__ v, int64_t ldv, const float* __restrict__ o, int64_t ldo,
+    const float* __restrict__ dO, int64_t lddo, const float* __restrict__ lse, float* __restrict__ delta,
+    float* __restrict__ nl2, float* __restrict__ dq, int64_t lddq, int S, int nh, int group, float scale_log2,
+    float scale, RopeRows<float> rope) {
+  constexpr int NU = HD / 16, TILE = 16 * (HD + 4);
+  __shared__ __align__(16) float tiles[2 * TILE];
+  const int lane = threadIdx.x & 63, r = lane & 15, c = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int bh = blockIdx.y, b = bh / nh, h = bh - b * nh, kvh = h / group;
+  const int q0 = static_cast<int>(gridDim.x - 1 - blockIdx.x) * 16, qi = q0 + r;
+  const int64_t tok0 = static_cast<int64_t>(b) * S;
+  const int qc = min(qi, S - 1);
+  const int64_t hcol = static_cast<int64_t>(h) * HD;
+
+  FragF32<HD> qf, gf;
+  float dl = 0.f;
+  {
+    FragF32<HD> of;
+    load_frag_f32<HD>(qf, q + (tok0 + qc) * ldq + hcol, c);
+    load_frag_f32<HD>(gf, dO + (tok0 + qc) * lddo + hcol, c);
+    load_frag_f32<HD>(of, o + (tok0 + qc) * ldo + hcol, c);
+#pragma unroll
+    for (int u = 0; u < NU; ++u)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) dl = fmaf(gf[u][e], of[u][e], dl);
+  }
+  dl = col_sum(dl);
+  const int64_t srow = static_cast<int64_t>(bh) * S + qc;
+  const float nlse2 = -lse[srow] * kLog2e;
+  if (wave == 0 && c == 0 && qi < S) {
+    delta[srow] = dl;
+    nl2[srow] = nlse2;
+  }
+  f32x4 acc[NU];
+#pragma unroll
+  for (int dt = 0; dt < NU; ++dt) acc[dt] = zero4();
+  const int kend = min(S, q0 + 16), nkb = (kend + 31) / 32;
+  const float* kp = k + tok0 * ldk + static_cast<int64_t>(kvh) * HD;
+  const float* vp = v + tok0 * ldv + static_cast<int64_t>(kvh) * HD;
+  for (int kb = wave; kb < nkb; kb += 4) {
+    const int k0 = kb * 32;
+    const int hi = min(qi, S - 1) + 1 - k0;
+    f32x4 x[2];  // dS^T: rows = keys, column = query
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const int64_t row = min(k0 + 16 * t + r, S - 1);
+      FragF32<HD> f;
+      load_frag_f32<HD>(f, kp + row * ldk, c);
+      x[t] = dot_f32<HD>(f, qf);
+      load_frag_f32<HD>(f, vp + row * ldv, c);
+      const f32x4 y = dot_f32<HD>(f, gf);  // dP^T
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        x[t][e] = 16 * t + 4 * c + e < hi ? fast_exp2(fmaf(x[t][e], scale_log2, nlse2)) * (y[e] - dl) : 0.f;
     }
-    const float ds = expf(x * scale - L) * (dp - D);
-    for (int d = 0; d < HD; ++d) acc[d] = fmaf(ds, kr[d], acc[d]);
+    wsum_f32<HD>(acc, x, kp + static_cast<int64_t>(k0) * ldk, ldk, S - 1 - k0, k0 + 31 > q0, 0, hi, r, c);
   }
-  float* out = dq + (b * S + s) * lddq + static_cast<int64_t>(h) * HD;
-  store_row_f32<HD>(out, acc, scale, rope, b * S, s);
+  sum_waves_f32<HD, 4>(acc, tiles, wave, r, c);
+  if (wave == 0) put_tile_f32<HD>(tiles, acc, r, c);
+  __syncthreads();
+  store_tile_f32<HD, 256>(dq + hcol, lddq, tiles, q0, S, scale, rope, tok0);
 }
 
+// Waves of a dK/dV workgroup: 16 where the registers allow four per SIMD.
 template <int HD>
-__global__ __launch_bounds__(128) void k_attn_bwd_dkdv_f32(
+constexpr int kDkdvWavesF32 = HD == 32 ? 16 : 8;
+
+template <int HD>
+__global__ __launch_bounds__(64 * kDkdvWavesF32<HD>) void k_attn_bwd_dkdv_f32(
     const float* __restrict__ q, int64_t ldq, const float* __restrict__ k, int64_t ldk,
     const float* __restrict__ v, int64_t ldv, const float* __restrict__ dO, int64_t lddo,
-    const float* __restrict__ lse, const float* __restrict__ delta, float* __restrict__ dk,
+    const float* __restrict__ nl2, const float* __restrict__ delta, float* __restrict__ dk,
     int64_t lddk, float* __restrict__ dv, int64_t lddv, int S, int nh, int nkv, int group,
-    float scale, int64_t rows, RopeRows<float> rope) {
-  const int64_t idx = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (idx >= rows) return;  // rows = B*nkv*S, idx = (b*nkv + kvh)*S + j
-  const int j = static_cast<int>(idx % S);
-  const int64_t bk = idx / S;
-  const int kvh = static_cast<int>(bk % nkv);
-  const int64_t b = bk / nkv;
-  const float* kr = k + (b * S + j) * ldk + static_cast<int64_t>(kvh) * HD;
-  const float* vr = v + (b * S + j) * ldv + static_cast<int64_t>(kvh) * HD;
-  float kv[HD], vv[HD], ak[HD], av[HD];
-  for (int d = 0; d < HD; ++d) { kv[d] = kr[d]; vv[d] = vr[d]; ak[d] = 0.f; av[d] = 0.f; }
-  for (int hh = 0; hh < group; ++hh) {
+    float scale_log2, float scale, RopeRows<float> rope) {
+  constexpr int NU = HD / 16, TILE = 16 * (HD + 4), NW = kDkdvWavesF32<HD>;
+  __shared__ __align__(16) float tiles[NW / 2 * TILE];
+  const int lane = threadIdx.x & 63, r = lane & 15, c = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int bk = blockIdx.y, b = bk / nkv, kvh = bk - b * nkv;
+  const int k0 = static_cast<int>(blockIdx.x) * 16, ki = k0 + r;  // earliest keys (most queries) first
+  const int64_t tok0 = static_cast<int64_t>(b) * S;
+  const int kc = min(ki, S - 1);
+
+  FragF32<HD> kf, vf;
+  load_frag_f32<HD>(kf, k + (tok0 + kc) * ldk + static_cast<int64_t>(kvh) * HD, c);
+  load_frag_f32<HD>(vf, v + (tok0 + kc) * ldv + static_cast<int64_t>(kvh) * HD, c);
+  f32x4 ak[NU], av[NU];
+#pragma unroll
+  for (int dt = 0; dt < NU; ++dt) ak[dt] = av[dt] = zero4();
+
+  const int qb0 = k0 / 32, nqb = (S + 31) / 32 - qb0;  // query blocks that reach the keys
+  for (int it = wave; it < group * nqb; it += NW) {
+    const int hh = it / nqb, q0 = (qb0 + it - hh * nqb) * 32;
     const int h = kvh * group + hh;
-    const int64_t row = (b * nh + h) * S;
-    for (int s = j; s < S; ++s) {
-      const float* qr = q + (b * S + s) * ldq + static_cast<int64_t>(h) * HD;
-      const float* gr = dO + (b * S + s) * lddo + static_cast<int64_t>(h) * HD;
-      float x = 0.f, dp = 0.f;
-      for (int d = 0; d < HD; ++d) {
-        x = fmaf(qr[d], kv[d], x);
-        dp = fmaf(gr[d], vv[d], dp);
-      }
-      const float p = expf(x * scale - lse[row + s]);
-      const float ds = p * (dp - delta[row + s]);
-      for (int d = 0; d < HD; ++d) {
-        av[d] = fmaf(p, gr[d], av[d]);
-        ak[d] = fmaf(ds, qr[d], ak[d]);
+    const float* qp = q + (tok0 + q0) * ldq + static_cast<int64_t>(h) * HD;
+    const float* gp = dO + (tok0 + q0) * lddo + static_cast<int64_t>(h) * HD;
+    const int64_t srow = (static_cast<int64_t>(b) * nh + h) * S + q0;
+    const int last = S - 1 - q0;
+    // Queries n of the block with lo <= n < hi see this key (none when the key is past S).
+    const int lo = ki - q0, hi = ki < S ? S - q0 : lo;
+    f32x4 x[2], y[2];  // P, dS: rows = queries, column = key
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const int row = min(16 * t + r, last);
+      FragF32<HD> f;
+      load_frag_f32<HD>(f, qp + row * ldq, c);
+      x[t] = dot_f32<HD>(f, kf);
+      load_frag_f32<HD>(f, gp + row * lddo, c);
+      y[t] = dot_f32<HD>(f, vf);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int n = 16 * t + 4 * c + e;
+        const int64_t at = srow + min(n, last);
+        const bool live = n >= lo && n < hi;
+        const float p = fast_exp2(fmaf(x[t][e], scale_log2, nl2[at]));
+        x[t][e] = live ? p : 0.f;
+        y[t][e] = live ? p * (y[t][e] - delta[at]) : 0.f;
       }
     }
+    const bool partial = q0 < k0 + 15 || q0 + 32 > S || k0 + 16 > S;
+    wsum_f32<HD>(av, x, gp, lddo, last, partial, lo, hi, r, c);
+    wsum_f32<HD>(ak, y, qp, ldq, last, partial, lo, hi, r, c);
   }
-  float* ok = dk + (b * S + j) * lddk + static_cast<int64_t>(kvh) * HD;
-  float* ov = dv + (b * S + j) * lddv + static_cast<int64_t>(kvh) * HD;
-  for (int d = 0; d < HD; ++d) ov[d] = av[d];
-  store_row_f32<HD>(ok, ak, scale, rope, b * S, j);
+  sum_waves_f32<HD, NW>(av, tiles, wave, r, c);
+  if (wave == 0) put_tile_f32<HD>(tiles, av, r, c);
+  __syncthreads();
+  store_tile_f32<HD, 64 * NW>(dv + static_cast<int64_t>(kvh) * HD, lddv, tiles, k0, S, 1.f,
+                              RopeRows<float>{nullptr, nullptr, 0}, tok0);
+  __syncthreads();
+  sum_waves_f32<HD, NW>(ak, tiles, wave, r, c);
+  if (wave == 0) put_tile_f32<HD>(tiles, ak, r, c);
+  __syncthreads();
+  store_tile_f32<HD, 64 * NW>(dk + static_cast<int64_t>(kvh) * HD, lddk, tiles, k0, S, scale, rope, tok0);
 }
 
 // ------------------------------------------------------------------- host
@@ -1302,12 +1528,11 @@ int attn_fwd_impl(fh_dtype dt, const void* q, int64_t ldq, const void* k, int64_
     });
   } else {
     const RopeRows<float> rf{static_cast<const float*>(rp.cos), static_cast<const float*>(rp.sin), rp.per_token};
-    const int64_t rows = batch * n_heads * seq_len;
+    const dim3 grid(static_cast<unsigned>((seq_len + 15) / 16), static_cast<unsigned>(batch * n_heads));
     dispatch_hd(head_dim, [&](auto hdc) {
-      hipLaunchKernelGGL((k_attn_fwd_f32<hdc()>), dim3(static_cast<unsigned>((rows + 127) / 128)),
-                         dim3(128), 0, stream, static_cast<const float*>(q), ldq,
+      hipLaunchKernelGGL((k_attn_fwd_f32<hdc()>), grid, dim3(256), 0, stream, static_cast<const float*>(q), ldq,
                          static_cast<const float*>(k), ldk, static_cast<const float*>(v), ldv,
-                         static_cast<float*>(o), ldo, lse, S, nh, group, scale, rows, rf,
+                         static_cast<float*>(o), ldo, lse, S, nh, group, scale * kLog2e, rf,
                          static_cast<float*>(qout), ldqo);
       return 0;
     });
@@ -1403,24 +1628,20 @@ int attn_bwd_impl(fh_dtype dt, const void* q, int64_t ldq, const void* k, int64_
       return 0;
     });
   } else {
-    const int64_t tokens = batch * seq_len;
-    const unsigned dblocks = static_cast<unsigned>((tokens * n_heads + 255) / 256);
-    hipLaunchKernelGGL((k_attn_delta<float>), dim3(dblocks), dim3(256), 0, stream,
-                       static_cast<const float*>(o), ldo, static_cast<const float*>(dout), lddo,
-                       delta, S, nh, static_cast<int>(head_dim), tokens);
-    const int64_t qrows = batch * n_heads * seq_len, krows = batch * n_kv_heads * seq_len;
+    const unsigned tiles = static_cast<unsigned>((seq_len + 15) / 16);
     dispatch_hd(head_dim, [&](auto hdc) {
-      hipLaunchKernelGGL((k_attn_bwd_dq_f32<hdc()>), dim3(static_cast<unsigned>((qrows + 127) / 128)),
-                         dim3(128), 0, stream, static_cast<const float*>(q), ldq,
-                         static_cast<const float*>(k), ldk, static_cast<const float*>(v), ldv,
-                         static_cast<const float*>(dout), lddo, lse, delta, static_cast<float*>(dq),
-                         lddq, S, nh, group, scale, qrows, rf);
-      hipLaunchKernelGGL((k_attn_bwd_dkdv_f32<hdc()>), dim3(static_cast<unsigned>((krows + 127) / 128)),
-                         dim3(128), 0, stream, static_cast<const float*>(q), ldq,
-                         static_cast<const float*>(k), ldk, static_cast<const float*>(v), ldv,
-                         static_cast<const float*>(dout), lddo, lse, delta,
-                         static_cast<float*>(dk), lddk, static_cast<float*>(dv), lddv, S, nh, nkv,
-                         group, scale, krows, rf);
+      constexpr int HD = decltype(hdc)::value;
+      const auto kq = static_cast<const float*>(q);
+      const auto kk = static_cast<const float*>(k);
+      const auto kvp = static_cast<const float*>(v);
+      const auto kg = static_cast<const float*>(dout);
+      hipLaunchKernelGGL((k_attn_bwd_dq_f32<HD>), dim3(tiles, static_cast<unsigned>(batch * n_heads)), dim3(256), 0,
+                         stream, kq, ldq, kk, ldk, kvp, ldv, static_cast<const float*>(o), ldo, kg, lddo, lse, delta,
+                         nl2, static_cast<float*>(dq), lddq, S, nh, group, scale * kLog2e, scale, rf);
+      hipLaunchKernelGGL((k_attn_bwd_dkdv_f32<HD>), dim3(tiles, static_cast<unsigned>(batch * n_kv_heads)),
+                         dim3(64 * kDkdvWavesF32<HD>), 0, stream, kq, ldq, kk, ldk, kvp, ldv, kg, lddo, nl2, delta,
+                         static_cast<float*>(dk), lddk, static_cast<float*>(dv), lddv, S, nh, nkv, group,
+                         scale * kLog2e, scale, rf);
       return 0;
     });
   }

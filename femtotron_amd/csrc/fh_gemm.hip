@@ -138,8 +138,6 @@ __device__ __forceinline__ uint4 rope_fwd_chunk(uint4 x, uint4 p, uint4 c, uint4
   return Elem<uint16_t>::pack(o);
 }
 
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-
 // As inline asm with the accumulator tied in place ("+a"): through the
 // builtin, the register allocator gave 64 four-register accumulators
 // different source and destination tuples and shuffled them through VGPRs

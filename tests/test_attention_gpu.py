@@ -101,6 +101,58 @@ def test_attention_fp32_matches_closed_form_1e5(B, S, nh, nkv, hd):
     assert (got["lse"] - ref["lse"]).abs().max() < 1e-5
 
 
+@pytest.mark.parametrize("B,S,nh,nkv,hd", [
+    (1, 2, 2, 1, 32), (2, 15, 4, 4, 64), (1, 16, 2, 1, 128), (1, 17, 8, 1, 32),   # one query tile and its edges
+    (1, 31, 2, 2, 128), (2, 33, 6, 2, 32), (1, 65, 8, 1, 64),                     # one key block and its edges
+    (1, 129, 4, 1, 128), (1, 300, 16, 2, 64)])                                    # more key blocks / items than waves
+def test_attention_fp32_tile_edges(B, S, nh, nkv, hd):
+    """fp32 sums of at most S * group terms and a 2^x of relative error 2^-22: far inside 1e-5 of the peak.
+    (One token alone has dq = dk = 0 exactly, so no peak to measure against: two tokens are the smallest.)"""
+    got, ref = _run(B, S, nh, nkv, hd, torch.float32)
+    for name in ("o", "dq", "dk", "dv"):
+        e = _tensor_err(got[name], ref[name])
+        assert e < 1e-5, f"{name}: {e:.3e}"
+    assert (got["lse"] - ref["lse"]).abs().max() < 1e-5
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+@pytest.mark.parametrize("hd", [32, 64, 128])
+def test_attention_fp32_masked_rows_do_not_leak(hd, bad):
+    """Infinities and NaNs reach only what sees them: put into k and v from token
+    21 on, they leave outputs and dq of the tokens before unchanged; into q and dO
+    before token 21, dk and dv of the tokens from 21 on.  A tile with a bad row is
+    summed in another order, so equal within fp32 sums of at most 45 x 2 terms."""
+    ops = _ops()
+    S, nh, nkv, cut = 45, 4, 2, 21
+    hq, hkv = nh * hd, nkv * hd
+    buf, do = (t.to(DEV) for t in _inputs(1, S, nh, nkv, hd, torch.float32, 3))
+
+    def run(g, d, o=None, lse=None):
+        q, k, v = g[:, :hq], g[:, hq:hq + hkv], g[:, hq + hkv:]
+        if o is None:
+            o, lse = ops.attn_fwd(q, k, v, 1, S, nh, nkv, hd, hd ** -0.5)
+        dg = torch.empty_like(g)
+        ops.attn_bwd(q, k, v, o, d, lse, dg[:, :hq], dg[:, hq:hq + hkv], dg[:, hq + hkv:], 1, S, nh, nkv, hd,
+                     hd ** -0.5)
+        return o, lse, dg
+
+    def same(a, b):
+        assert torch.isfinite(a).all() and float((a - b).abs().max() / b.abs().max()) < 1e-5
+
+    o, lse, dg = run(buf, do)
+    late = buf.clone()
+    late[cut:, hq:] = bad
+    o2, lse2, dg2 = run(late, do)
+    same(o2[:cut], o[:cut])
+    same(lse2[..., :cut], lse[..., :cut])
+    same(dg2[:cut, :hq], dg[:cut, :hq])
+    early, d3 = buf.clone(), do.clone()
+    early[:cut, :hq] = bad
+    d3[:cut] = bad
+    _, _, dg3 = run(early, d3, o, lse)
+    same(dg3[cut:, hq:], dg[cut:, hq:])
+
+
 @pytest.mark.parametrize("hd", [32, 64, 128])
 def test_attention_ragged_tiles_stay_inside_their_sequence(hd):
     """Tiles that run past S load clamped rows of their own sequence, never the
