@@ -49,6 +49,14 @@
 // even share of the remaining tiles' k-steps, whose split tiles k_gemm_fixup
 // sums from fp32 segments in k order (deterministic, no inter-workgroup
 // waits).
+//
+// k that is no multiple of 64 (RAGGED): the last stage reads the last 64 k's
+// and zeroes in LDS those that the stage before covered, so no load leaves the
+// operands.  Weight gradients of ragged batches went to the library before
+// (28672 x 4096 and 4096 x 14336 over 2002 tokens: 806 -> 600 us together, 1.17
+// against 0.87 PFLOP/s; the four of a 2048-wide layer over 999 tokens: 193 ->
+// 136 us).  A template argument, as the multiples of 64 lost up to 1% to the
+// extra arithmetic per load.
 #include "fh_common.hpp"
 #include "fh_mfma.hpp"
 
@@ -102,6 +110,10 @@ struct GemmArgs {
   int m, n;
   int tiles_m, tiles_n, tiles;
   int steps_per_slice, total_steps;
+  // k_last: k of the last stage's first step, k - 64.  Where k is no multiple of
+  // 64 the last stage starts before a multiple and repeats the `repeat` = 64 -
+  // k % 64 k's of the stage before, which are zeroed in LDS (zero_repeat).
+  int k_last, repeat;
   int grid;  // logical blocks (tiles * slices; EPI_STREAM: the workgroups)
   // EPI_STREAM: full_rounds whole tiles per workgroup (tile r * grid + w),
   // then the remaining tail_tiles' tail_iters = tail_tiles * total_steps
@@ -252,6 +264,18 @@ __device__ __forceinline__ void bar() {
 constexpr int kSlot = 32768;  // one operand's stage: [256 x 64] bf16
 constexpr int kRing = 5;      // operand slots in LDS (160 KB)
 
+// Zeroes the first `n` of the 64 k's of this wave's quarter of an operand's
+// stage, which has landed (lane i filled 16-byte slot i of each 1 KB run, with
+// the k's of RunPlan's layout; n is a multiple of 8 for KC).
+template <bool KO>
+__device__ __forceinline__ void zero_repeat(char* quarter, int n, int lane) {
+#pragma unroll 1
+  for (int jj = 0; jj < 8; ++jj) {
+    const int k = KO ? 8 * jj + ((lane >> 1) & 7) : 8 * ((lane & 7) ^ swz<64>(8 * jj + (lane >> 3)));
+    if (k < n) *reinterpret_cast<uint4*>(quarter + jj * 1024 + lane * 16) = make_uint4(0, 0, 0, 0);
+  }
+}
+
 template <int N>
 __device__ __forceinline__ void wait_vm_n() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
@@ -301,7 +325,8 @@ __device__ __forceinline__ GemmArgs for_tile(const GemmArgs& g, int& t) {
 // (bf16, with the EPI epilogue) or, for EPI_PARTIAL and for EPI_STREAM with
 // to_part, as fp32 to pdst (the tile's origin, row stride pld).  EPI_STREAM
 // ends with a barrier, as the workgroup's next tile reuses the LDS ring.
-template <bool A_KO, bool B_KO, int EPI>
+// RAGGED: k may be no multiple of 64.
+template <bool A_KO, bool B_KO, int EPI, bool RAGGED>
 __device__ __forceinline__ void gemm_tile(const GemmArgs& g, char* ring, int t, int s_begin, int nst,
                                           float* pdst, int64_t pld, bool to_part) {
   const int tid = threadIdx.x, lane = tid & 63, hl = lane >> 5;
@@ -316,12 +341,16 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, char* ring, int t, 
   typedef __attribute__((address_space(3))) char* lptr;
   const uint32_t ring0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lptr)ring)) + wave * 8192;
 
+  auto k_of = [&](int step) __attribute__((always_inline)) {
+    const int64_t k0 = static_cast<int64_t>(s_begin + min(step, nst - 1)) * kTk;
+    return RAGGED ? min(k0, static_cast<int64_t>(g.k_last)) : k0;
+  };
   // Run jj of wave `wave`'s quarter of operand OP (0: A, 1: B) of stage
   // `step` into ring slot `slot`.  Stages past the slice's end re-load its
   // last stage (in bounds, never used): the loop has no branches.
   auto dma = [&](auto op_tag, int step, int slot, int jj) __attribute__((always_inline)) {
     constexpr int OP = decltype(op_tag)::value;
-    const int64_t k0 = static_cast<int64_t>(s_begin + min(step, nst - 1)) * kTk;
+    const int64_t k0 = k_of(step);
     const uint32_t lds_slot = ring0 + slot * kSlot + jj * 1024;
     if constexpr (OP == 0) pa.load(k0 * pa.k_bytes, jj, lds_slot);
     else pb.load(k0 * pb.k_bytes, jj, lds_slot);
@@ -329,7 +358,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, char* ring, int t, 
   // The loop's form: M0 set one MFMA earlier (set_m0), so the load needs no s_nop.
   auto dma_m0 = [&](auto op_tag, int step, int jj) __attribute__((always_inline)) {
     constexpr int OP = decltype(op_tag)::value;
-    const int64_t k0 = static_cast<int64_t>(s_begin + min(step, nst - 1)) * kTk;
+    const int64_t k0 = k_of(step);
     if constexpr (OP == 0) pa.load_m0(k0 * pa.k_bytes, jj);
     else pb.load_m0(k0 * pb.k_bytes, jj);
   };
@@ -377,6 +406,15 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, char* ring, int t, 
 #pragma unroll
   for (int jj = 0; jj < 8; ++jj) dma(OpB(), 1, 3, jj);
   wait_vm_n<16>();
+  // The stage that repeats k's, if this range ends with it (-1: none).
+  [[maybe_unused]] const int xr = g.repeat > 0 && s_begin + nst == g.total_steps ? nst - 1 : -1;
+  [[maybe_unused]] auto zero = [&](int sa, int sb) __attribute__((always_inline)) {
+    zero_repeat<A_KO>(ring + sa * kSlot + wave * 8192, g.repeat, lane);
+    zero_repeat<B_KO>(ring + sb * kSlot + wave * 8192, g.repeat, lane);
+    wait_lds();
+  };
+  if constexpr (RAGGED)
+    if (xr == 0) zero(0, 1);
   bar();
 #pragma unroll
   for (int r = 0; r < 16; ++r) {
@@ -408,6 +446,8 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, char* ring, int t, 
     }
     wait_lds();
     wait_vm_n<8>();
+    if constexpr (RAGGED)
+      if (x + 1 == xr) zero(nA, nB);
     bar();
 #pragma unroll
     for (int p = 0; p < 64; ++p) {
@@ -588,7 +628,7 @@ __device__ __forceinline__ const char* whole_base(const uint16_t* base, int64_t 
 // this saves, per tile, the prologue (two stages loaded and the first waited
 // for), the output's round trip through LDS with its barriers, and the gap
 // between a CU's consecutive workgroups.
-template <bool A_KO, bool B_KO, bool RESID>
+template <bool A_KO, bool B_KO, bool RESID, bool RAGGED>
 __device__ __forceinline__ void gemm_persist(const GemmArgs& g, char* ring, int lid) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -626,15 +666,19 @@ __device__ __forceinline__ void gemm_persist(const GemmArgs& g, char* ring, int 
     acc[i][j] = mfma16(fb[buf][i], fa[buf][j], acc[i][j]);
   };
 
+  auto k_of = [&](int step) __attribute__((always_inline)) {
+    const int64_t k0 = static_cast<int64_t>(step) * kTk;
+    return RAGGED ? min(k0, static_cast<int64_t>(g.k_last)) : k0;
+  };
   // Prologue of the first tile (as gemm_tile's).
 #pragma unroll
   for (int jj = 0; jj < 8; ++jj) dma16(offa[jj], ba, ring0 + 0 * kSlot + jj * 1024);
 #pragma unroll
   for (int jj = 0; jj < 8; ++jj) dma16(offb[jj], bb, ring0 + 1 * kSlot + jj * 1024);
 #pragma unroll
-  for (int jj = 0; jj < 8; ++jj) dma16(offa[jj], ba + kTk * kba, ring0 + 2 * kSlot + jj * 1024);
+  for (int jj = 0; jj < 8; ++jj) dma16(offa[jj], ba + k_of(1) * kba, ring0 + 2 * kSlot + jj * 1024);
 #pragma unroll
-  for (int jj = 0; jj < 8; ++jj) dma16(offb[jj], bb + kTk * kbb, ring0 + 3 * kSlot + jj * 1024);
+  for (int jj = 0; jj < 8; ++jj) dma16(offb[jj], bb + k_of(1) * kbb, ring0 + 3 * kSlot + jj * 1024);
   wait_vm_n<16>();
   bar();
 #pragma unroll
@@ -644,6 +688,7 @@ __device__ __forceinline__ void gemm_persist(const GemmArgs& g, char* ring, int 
   }
 
   int s = 0;  // ring slot of the current stage's A (stage x: A in s, B in s+1)
+  [[maybe_unused]] const int xr = g.repeat > 0 ? nst - 2 : -1;  // the stage before the one that repeats k's (nst >= 2)
   for (;;) {
     const int tn = t + g.grid;
     const bool more = tn < g.tiles;
@@ -661,7 +706,7 @@ __device__ __forceinline__ void gemm_persist(const GemmArgs& g, char* ring, int 
     for (int x = 0; x < nst; ++x) {
       const int sB = mod5(s + 1), nA = mod5(s + 2), nB = mod5(s + 3), fA = mod5(s + 4);
       const bool ahead = more && x + 2 >= nst;
-      const int64_t k2 = static_cast<int64_t>(ahead ? x + 2 - nst : min(x + 2, nst - 1)) * kTk;
+      const int64_t k2 = k_of(ahead ? x + 2 - nst : min(x + 2, nst - 1));
       const char* srcA = (ahead ? na : ba) + k2 * kba;
       const char* srcB = (ahead ? nb : bb) + k2 * kbb;
       const uint32_t dA = ring0 + fA * kSlot, dB = ring0 + s * kSlot;
@@ -676,6 +721,12 @@ __device__ __forceinline__ void gemm_persist(const GemmArgs& g, char* ring, int 
       }
       wait_lds();
       wait_vm_n<8>();
+      if constexpr (RAGGED)
+        if (x == xr) {
+          zero_repeat<A_KO>(ring + nA * kSlot + wave * 8192, g.repeat, lane);
+          zero_repeat<B_KO>(ring + nB * kSlot + wave * 8192, g.repeat, lane);
+          wait_lds();
+        }
       bar();
 #pragma unroll
       for (int p = 0; p < 64; ++p) {
@@ -746,7 +797,7 @@ __device__ __forceinline__ void gemm_persist(const GemmArgs& g, char* ring, int 
 // of the tail's k-steps as segments of one tile each.  A tail segment that is not a whole tile goes to
 // fp32 slot 2w (the workgroup's first tail segment) or 2w + 1 (its last);
 // k_gemm_fixup adds a split tile's segments in k order.
-template <bool A_KO, bool B_KO, int EPI>
+template <bool A_KO, bool B_KO, int EPI, bool RAGGED>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void k_gemm(GemmArgs g) {
   __shared__ __align__(16) char ring[kRing * kSlot];
   const int nb8 = gridDim.x >> 3;
@@ -785,7 +836,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
         break;
       }
       const GemmArgs pg = for_tile(g, t);
-      gemm_tile<A_KO, B_KO, EPI>(pg, ring, t, k0, len, slot, kTn, len < ki);
+      gemm_tile<A_KO, B_KO, EPI, RAGGED>(pg, ring, t, k0, len, slot, kTn, len < ki);
     }
   } else {
     const int slice = lid / g.tiles, t = lid - slice * g.tiles;
@@ -795,18 +846,18 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     float* pdst = EPI == EPI_PARTIAL
                       ? g.part + static_cast<int64_t>(slice) * g.m * g.n + static_cast<int64_t>(m0) * g.n + n0
                       : nullptr;
-    gemm_tile<A_KO, B_KO, EPI>(g, ring, t, s_begin, min(g.total_steps - s_begin, g.steps_per_slice), pdst,
+    gemm_tile<A_KO, B_KO, EPI, RAGGED>(g, ring, t, s_begin, min(g.total_steps - s_begin, g.steps_per_slice), pdst,
                                g.n, EPI == EPI_PARTIAL);
   }
 }
 
 // The persistent form (gemm_persist): G = gridDim.x workgroups, a multiple of
 // 8, at most the number of tiles.
-template <bool A_KO, bool B_KO, bool RESID>
+template <bool A_KO, bool B_KO, bool RESID, bool RAGGED>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void k_gemm_persist(GemmArgs g) {
   __shared__ __align__(16) char ring[kRing * kSlot];
   const int nb8 = gridDim.x >> 3;
-  gemm_persist<A_KO, B_KO, RESID>(g, ring, (blockIdx.x & 7) * nb8 + (blockIdx.x >> 3));
+  gemm_persist<A_KO, B_KO, RESID, RAGGED>(g, ring, (blockIdx.x & 7) * nb8 + (blockIdx.x >> 3));
 }
 
 // Rows blockIdx.y * 16 .. +15 of tail tile blockIdx.x of a stream GEMM: if
@@ -945,7 +996,7 @@ struct GemmPlan {
 };
 
 GemmPlan gemm_plan(int64_t m, int64_t n, int64_t k) {
-  const int64_t tiles = ((m + kTm - 1) / kTm) * ((n + kTn - 1) / kTn), steps = k / kTk;
+  const int64_t tiles = ((m + kTm - 1) / kTm) * ((n + kTn - 1) / kTn), steps = (k + kTk - 1) / kTk;
   const int cus = device_cus();
   const double per_slice = 48.0 * static_cast<double>(m) * n / (655360.0 * static_cast<double>(k));
   int best = 1;
@@ -973,22 +1024,49 @@ GemmPlan gemm_plan(int64_t m, int64_t n, int64_t k) {
 
 size_t stream_workspace_bytes() { return 2 * static_cast<size_t>(stream_grid()) * kTm * kTn * sizeof(float); }
 
-template <bool A_KO, bool B_KO>
+template <bool A_KO, bool B_KO, bool RAGGED>
 void launch(const GemmArgs& g, unsigned blocks, bool partial, bool resid, hipStream_t stream) {
-  if constexpr (!A_KO && !B_KO) {  // the rotated forward projection is NT only
+  if constexpr (!A_KO && !B_KO && !RAGGED) {  // the rotated forward projection: NT, k % 64 == 0
     if (g.rope.cos) {
-      hipLaunchKernelGGL((k_gemm<false, false, EPI_ROPE>), dim3(blocks), dim3(256), 0, stream, g);
+      hipLaunchKernelGGL((k_gemm<false, false, EPI_ROPE, false>), dim3(blocks), dim3(256), 0, stream, g);
       return;
     }
   }
-  if (g.tail_iters > 0)
-    hipLaunchKernelGGL((k_gemm<A_KO, B_KO, EPI_STREAM>), dim3(blocks), dim3(256), 0, stream, g);
+  if (g.full_rounds > 0)  // the stream form: at least one whole round
+    hipLaunchKernelGGL((k_gemm<A_KO, B_KO, EPI_STREAM, RAGGED>), dim3(blocks), dim3(256), 0, stream, g);
   else if (partial)
-    hipLaunchKernelGGL((k_gemm<A_KO, B_KO, EPI_PARTIAL>), dim3(blocks), dim3(256), 0, stream, g);
+    hipLaunchKernelGGL((k_gemm<A_KO, B_KO, EPI_PARTIAL, RAGGED>), dim3(blocks), dim3(256), 0, stream, g);
   else if (resid)
-    hipLaunchKernelGGL((k_gemm<A_KO, B_KO, EPI_RESIDUAL>), dim3(blocks), dim3(256), 0, stream, g);
+    hipLaunchKernelGGL((k_gemm<A_KO, B_KO, EPI_RESIDUAL, RAGGED>), dim3(blocks), dim3(256), 0, stream, g);
   else
-    hipLaunchKernelGGL((k_gemm<A_KO, B_KO, EPI_STORE>), dim3(blocks), dim3(256), 0, stream, g);
+    hipLaunchKernelGGL((k_gemm<A_KO, B_KO, EPI_STORE, RAGGED>), dim3(blocks), dim3(256), 0, stream, g);
+}
+
+template <bool RAGGED>
+void launch_op(int op, const GemmArgs& g, unsigned blocks, bool partial, bool resid, hipStream_t stream) {
+  switch (op) {
+    case FH_GEMM_NT: launch<false, false, RAGGED>(g, blocks, partial, resid, stream); break;
+    case FH_GEMM_NN: launch<false, true, RAGGED>(g, blocks, partial, resid, stream); break;
+    default: launch<true, true, RAGGED>(g, blocks, partial, resid, stream); break;
+  }
+}
+
+void launch_op(int op, const GemmArgs& g, unsigned blocks, bool partial, bool resid, hipStream_t stream) {
+  if (g.repeat > 0) launch_op<true>(op, g, blocks, partial, resid, stream);
+  else launch_op<false>(op, g, blocks, partial, resid, stream);
+}
+
+template <bool RAGGED>
+void launch_persist(int op, const GemmArgs& g, hipStream_t stream) {
+  const dim3 grid(g.grid), block(256);
+  if (g.r != nullptr)  // the forward (NT) layout only
+    hipLaunchKernelGGL((k_gemm_persist<false, false, true, RAGGED>), grid, block, 0, stream, g);
+  else if (op == FH_GEMM_NT)
+    hipLaunchKernelGGL((k_gemm_persist<false, false, false, RAGGED>), grid, block, 0, stream, g);
+  else if (op == FH_GEMM_NN)
+    hipLaunchKernelGGL((k_gemm_persist<false, true, false, RAGGED>), grid, block, 0, stream, g);
+  else
+    hipLaunchKernelGGL((k_gemm_persist<true, true, false, RAGGED>), grid, block, 0, stream, g);
 }
 
 bool valid_op(int op) { return op == FH_GEMM_NT || op == FH_GEMM_NN || op == FH_GEMM_TN; }
@@ -998,22 +1076,41 @@ bool valid_op(int op) { return op == FH_GEMM_NT || op == FH_GEMM_NN || op == FH_
 
 using namespace fh;
 
-extern "C" size_t fh_gemm_bf16_workspace_size(int op, int64_t m, int64_t n, int64_t k) {
-  if (!valid_op(op) || m <= 0 || n <= 0 || k <= 0 || k % 64) return 0;
-  // the stream form's segment slots, or the split form's partials
+namespace {
+
+// The stream form's segment slots, or the split form's partials.
+size_t gemm_workspace(int64_t m, int64_t n, int64_t k) {
   const GemmPlan p = gemm_plan(m, n, k);
   if (p.stream) return stream_workspace_bytes();
   return p.slices > 1 ? static_cast<size_t>(p.slices) * m * n * sizeof(float) : 0;
+}
+
+// k of the any-k entry points: at least one whole stage; where an operand has k
+// contiguous the last stage's start k - 64 must keep 16-byte alignment.
+bool any_k_ok(int op, int64_t k) { return k >= kTk && (op == FH_GEMM_TN || k % 8 == 0); }
+
+}  // namespace
+
+extern "C" size_t fh_gemm_bf16_workspace_size(int op, int64_t m, int64_t n, int64_t k) {
+  if (!valid_op(op) || m <= 0 || n <= 0 || k <= 0 || k % 64) return 0;
+  return gemm_workspace(m, n, k);
+}
+
+extern "C" size_t fh_gemm_bf16_any_k_workspace_size(int op, int64_t m, int64_t n, int64_t k) {
+  if (!valid_op(op) || m <= 0 || n <= 0 || !any_k_ok(op, k)) return 0;
+  return gemm_workspace(m, n, k);
 }
 
 namespace {
 
 // Checks the operands of one GEMM and fills g (tiling for `slices` K slices).
 int gemm_setup(int op, const void* a, int64_t lda, const void* b, int64_t ldb, void* c, int64_t ldc,
-               const void* residual, int64_t ldr, int64_t m, int64_t n, int64_t k, GemmArgs& g) {
+               const void* residual, int64_t ldr, int64_t m, int64_t n, int64_t k, bool any_k, GemmArgs& g) {
   FH_REQUIRE(valid_op(op), "gemm_bf16: op must be FH_GEMM_NT, FH_GEMM_NN or FH_GEMM_TN");
   FH_REQUIRE(m > 0 && n > 0 && k > 0, "gemm_bf16: sizes must be positive");
-  FH_REQUIRE(k % 64 == 0, "gemm_bf16: k must be a multiple of 64");
+  FH_REQUIRE(any_k || k % 64 == 0, "gemm_bf16: k must be a multiple of 64");
+  FH_REQUIRE(!any_k || any_k_ok(op, k),
+             "gemm_bf16_any_k: k must be at least 64, and a multiple of 8 unless the op is FH_GEMM_TN");
   FH_REQUIRE(n % 8 == 0, "gemm_bf16: n must be a multiple of 8");
   FH_REQUIRE(op != FH_GEMM_TN || m % 8 == 0, "gemm_bf16: m must be a multiple of 8 for FH_GEMM_TN");
   FH_REQUIRE(m < (int64_t(1) << 30) && n < (int64_t(1) << 30) && k < (int64_t(1) << 30),
@@ -1045,7 +1142,9 @@ int gemm_setup(int op, const void* a, int64_t lda, const void* b, int64_t ldb, v
   g.tiles_m = static_cast<int>((m + kTm - 1) / kTm);
   g.tiles_n = static_cast<int>((n + kTn - 1) / kTn);
   g.tiles = g.tiles_m * g.tiles_n;
-  g.total_steps = static_cast<int>(k / kTk);
+  g.total_steps = static_cast<int>((k + kTk - 1) / kTk);
+  g.k_last = static_cast<int>(k) - kTk;
+  g.repeat = g.total_steps * kTk - static_cast<int>(k);
   g.ngroup = 1;
   g.grp[0] = GemmProblem{g.a, g.b, g.c, g.r, lda, ldb, ldc, ldr, g.m, g.n, g.tiles_m, g.tiles_n, 0};
   return FH_OK;
@@ -1064,11 +1163,7 @@ int gemm_run(int op, GemmArgs& g, int slices, bool stream_form, void* workspace,
     g.tail_iters = static_cast<int64_t>(g.tail_tiles) * g.total_steps;
     g.steps_per_slice = g.total_steps;
     g.slab_chunks = g.tail_tiles % (sg / 8) == 0 ? g.tail_tiles / (sg / 8) : 0;
-    switch (op) {
-      case FH_GEMM_NT: launch<false, false>(g, sg, false, false, stream); break;
-      case FH_GEMM_NN: launch<false, true>(g, sg, false, false, stream); break;
-      default: launch<true, true>(g, sg, false, false, stream); break;
-    }
+    launch_op(op, g, sg, false, false, stream);
     if (g.tail_tiles > 0)
       hipLaunchKernelGGL(k_gemm_fixup, dim3(g.tail_tiles, kTm / kFixRows), dim3(256), 0, stream, g);
     return FH_OK;
@@ -1080,15 +1175,8 @@ int gemm_run(int op, GemmArgs& g, int slices, bool stream_form, void* workspace,
       g.m % kTm == 0 && g.n % kTn == 0 && g.lda < (int64_t(1) << 24) && g.ldb < (int64_t(1) << 24) &&
       g.tiles > stream_grid()) {
     g.grid = stream_grid();
-    if (g.r != nullptr) {
-      hipLaunchKernelGGL((k_gemm_persist<false, false, true>), dim3(g.grid), dim3(256), 0, stream, g);
-      return FH_OK;
-    }
-    switch (op) {
-      case FH_GEMM_NT: hipLaunchKernelGGL((k_gemm_persist<false, false, false>), dim3(g.grid), dim3(256), 0, stream, g); break;
-      case FH_GEMM_NN: hipLaunchKernelGGL((k_gemm_persist<false, true, false>), dim3(g.grid), dim3(256), 0, stream, g); break;
-      default: hipLaunchKernelGGL((k_gemm_persist<true, true, false>), dim3(g.grid), dim3(256), 0, stream, g); break;
-    }
+    if (g.repeat > 0) launch_persist<true>(op, g, stream);
+    else launch_persist<false>(op, g, stream);
     return FH_OK;
   }
 #endif
@@ -1097,11 +1185,7 @@ int gemm_run(int op, GemmArgs& g, int slices, bool stream_form, void* workspace,
   g.grid = static_cast<int>(logical);
   const unsigned blocks = static_cast<unsigned>((logical + 7) / 8 * 8);
   const bool partial = slices > 1, resid = g.r != nullptr;
-  switch (op) {
-    case FH_GEMM_NT: launch<false, false>(g, blocks, partial, resid, stream); break;
-    case FH_GEMM_NN: launch<false, true>(g, blocks, partial, resid, stream); break;
-    default: launch<true, true>(g, blocks, partial, resid, stream); break;
-  }
+  launch_op(op, g, blocks, partial, resid, stream);
   if (partial) {
     const int64_t mn = static_cast<int64_t>(g.m) * g.n;
     const unsigned rb = static_cast<unsigned>((mn / 4 + 255) / 256);
@@ -1117,16 +1201,32 @@ int gemm_run(int op, GemmArgs& g, int slices, bool stream_form, void* workspace,
 
 }  // namespace
 
+namespace {
+
+int gemm_impl(int op, const void* a, int64_t lda, const void* b, int64_t ldb, void* c, int64_t ldc,
+              const void* residual, int64_t ldr, int64_t m, int64_t n, int64_t k, bool any_k, void* workspace,
+              hipStream_t stream, const char* name) {
+  GemmArgs g;
+  if (int e = gemm_setup(op, a, lda, b, ldb, c, ldc, residual, ldr, m, n, k, any_k, g)) return e;
+  const GemmPlan p = gemm_plan(m, n, k);
+  FH_REQUIRE((p.slices == 1 && !p.stream) || (workspace && aligned16(workspace)),
+             std::string(name + 3) + ": workspace (" + name + "_workspace_size bytes) required");
+  if (int e = gemm_run(op, g, p.slices, p.stream, workspace, stream)) return e;
+  return check_launch(name);
+}
+
+}  // namespace
+
 extern "C" int fh_gemm_bf16(int op, const void* a, int64_t lda, const void* b, int64_t ldb, void* c,
                             int64_t ldc, const void* residual, int64_t ldr, int64_t m, int64_t n,
                             int64_t k, void* workspace, hipStream_t stream) {
-  GemmArgs g;
-  if (int e = gemm_setup(op, a, lda, b, ldb, c, ldc, residual, ldr, m, n, k, g)) return e;
-  const GemmPlan p = gemm_plan(m, n, k);
-  FH_REQUIRE((p.slices == 1 && !p.stream) || (workspace && aligned16(workspace)),
-             "gemm_bf16: workspace (fh_gemm_bf16_workspace_size bytes) required");
-  if (int e = gemm_run(op, g, p.slices, p.stream, workspace, stream)) return e;
-  return check_launch("fh_gemm_bf16");
+  return gemm_impl(op, a, lda, b, ldb, c, ldc, residual, ldr, m, n, k, false, workspace, stream, "fh_gemm_bf16");
+}
+
+extern "C" int fh_gemm_bf16_any_k(int op, const void* a, int64_t lda, const void* b, int64_t ldb, void* c,
+                                  int64_t ldc, const void* residual, int64_t ldr, int64_t m, int64_t n,
+                                  int64_t k, void* workspace, hipStream_t stream) {
+  return gemm_impl(op, a, lda, b, ldb, c, ldc, residual, ldr, m, n, k, true, workspace, stream, "fh_gemm_bf16_any_k");
 }
 
 namespace {
@@ -1138,14 +1238,15 @@ bool group_stream(int64_t tiles, int64_t steps) { return tiles > stream_grid() &
 
 // Checks every problem of a group and fills g with the group's table (tiles
 // numbered problem by problem).
-int group_setup(int op, int count, const fh_gemm_problem* probs, int64_t k, GemmArgs& g) {
+int group_setup(int op, int count, const fh_gemm_problem* probs, int64_t k, bool any_k, GemmArgs& g) {
   FH_REQUIRE(count >= 1 && count <= kMaxGroup && probs != nullptr,
              "gemm_bf16_grouped: between 1 and 3 problems required");
   int tile0 = 0;
   for (int i = 0; i < count; ++i) {
     const fh_gemm_problem& p = probs[i];
     GemmArgs gi;
-    if (int e = gemm_setup(op, p.a, p.lda, p.b, p.ldb, p.c, p.ldc, p.residual, p.ldr, p.m, p.n, k, gi)) return e;
+    if (int e = gemm_setup(op, p.a, p.lda, p.b, p.ldb, p.c, p.ldc, p.residual, p.ldr, p.m, p.n, k, any_k, gi))
+      return e;
     if (i == 0) g = gi;
     g.grp[i] = gi.grp[0];
     g.grp[i].tile0 = tile0;
@@ -1156,31 +1257,27 @@ int group_setup(int op, int count, const fh_gemm_problem* probs, int64_t k, Gemm
   return FH_OK;
 }
 
-}  // namespace
-
-extern "C" size_t fh_gemm_bf16_grouped_workspace_size(int op, int count, const fh_gemm_problem* problems,
-                                                      int64_t k) {
-  if (!valid_op(op) || count < 1 || count > kMaxGroup || problems == nullptr || k <= 0 || k % kTk) return 0;
+size_t group_workspace(int count, const fh_gemm_problem* problems, int64_t k) {
   int64_t tiles = 0;
   size_t most = 0;
   for (int i = 0; i < count; ++i) {
     const int64_t m = problems[i].m, n = problems[i].n;
     if (m <= 0 || n <= 0) return 0;
     tiles += ((m + kTm - 1) / kTm) * ((n + kTn - 1) / kTn);
-    most = std::max(most, fh_gemm_bf16_workspace_size(op, m, n, k));
+    most = std::max(most, gemm_workspace(m, n, k));
   }
-  return group_stream(tiles, k / kTk) ? stream_workspace_bytes() : most;
+  return group_stream(tiles, (k + kTk - 1) / kTk) ? stream_workspace_bytes() : most;
 }
 
-extern "C" int fh_gemm_bf16_grouped(int op, int count, const fh_gemm_problem* problems, int64_t k,
-                                    void* workspace, hipStream_t stream) {
+int group_impl(int op, int count, const fh_gemm_problem* problems, int64_t k, bool any_k, void* workspace,
+               hipStream_t stream) {
   GemmArgs g;
-  if (int e = group_setup(op, count, problems, k, g)) return e;
+  if (int e = group_setup(op, count, problems, k, any_k, g)) return e;
   if (!group_stream(g.tiles, g.total_steps)) {
     for (int i = 0; i < count; ++i) {
       const fh_gemm_problem& p = problems[i];
-      if (int e = fh_gemm_bf16(op, p.a, p.lda, p.b, p.ldb, p.c, p.ldc, p.residual, p.ldr, p.m, p.n, k,
-                               workspace, stream))
+      if (int e = gemm_impl(op, p.a, p.lda, p.b, p.ldb, p.c, p.ldc, p.residual, p.ldr, p.m, p.n, k, any_k,
+                            workspace, stream, any_k ? "fh_gemm_bf16_any_k" : "fh_gemm_bf16"))
         return e;
     }
     return FH_OK;
@@ -1195,14 +1292,34 @@ extern "C" int fh_gemm_bf16_grouped(int op, int count, const fh_gemm_problem* pr
   g.tail_iters = static_cast<int64_t>(g.tail_tiles) * g.total_steps;
   g.steps_per_slice = g.total_steps;
   g.slab_chunks = g.tail_tiles % (sg / 8) == 0 ? g.tail_tiles / (sg / 8) : 0;
-  switch (op) {
-    case FH_GEMM_NT: hipLaunchKernelGGL((k_gemm<false, false, EPI_STREAM>), dim3(sg), dim3(256), 0, stream, g); break;
-    case FH_GEMM_NN: hipLaunchKernelGGL((k_gemm<false, true, EPI_STREAM>), dim3(sg), dim3(256), 0, stream, g); break;
-    default: hipLaunchKernelGGL((k_gemm<true, true, EPI_STREAM>), dim3(sg), dim3(256), 0, stream, g); break;
-  }
+  launch_op(op, g, sg, false, false, stream);
   if (g.tail_tiles > 0)
     hipLaunchKernelGGL(k_gemm_fixup, dim3(g.tail_tiles, kTm / kFixRows), dim3(256), 0, stream, g);
   return check_launch("fh_gemm_bf16_grouped");
+}
+
+}  // namespace
+
+extern "C" size_t fh_gemm_bf16_grouped_workspace_size(int op, int count, const fh_gemm_problem* problems,
+                                                      int64_t k) {
+  if (!valid_op(op) || count < 1 || count > kMaxGroup || problems == nullptr || k <= 0 || k % kTk) return 0;
+  return group_workspace(count, problems, k);
+}
+
+extern "C" int fh_gemm_bf16_grouped(int op, int count, const fh_gemm_problem* problems, int64_t k,
+                                    void* workspace, hipStream_t stream) {
+  return group_impl(op, count, problems, k, false, workspace, stream);
+}
+
+extern "C" size_t fh_gemm_bf16_grouped_any_k_workspace_size(int op, int count, const fh_gemm_problem* problems,
+                                                            int64_t k) {
+  if (!valid_op(op) || count < 1 || count > kMaxGroup || problems == nullptr || !any_k_ok(op, k)) return 0;
+  return group_workspace(count, problems, k);
+}
+
+extern "C" int fh_gemm_bf16_grouped_any_k(int op, int count, const fh_gemm_problem* problems, int64_t k,
+                                          void* workspace, hipStream_t stream) {
+  return group_impl(op, count, problems, k, true, workspace, stream);
 }
 
 extern "C" int fh_gemm_bf16_rope(const void* a, int64_t lda, const void* b, int64_t ldb, void* c, int64_t ldc,
@@ -1210,7 +1327,7 @@ extern "C" int fh_gemm_bf16_rope(const void* a, int64_t lda, const void* b, int6
                                  int64_t seq_len, const void* cos, const void* sin, int cos_per_token,
                                  hipStream_t stream) {
   GemmArgs g;
-  if (int e = gemm_setup(FH_GEMM_NT, a, lda, b, ldb, c, ldc, nullptr, 0, m, n, k, g)) return e;
+  if (int e = gemm_setup(FH_GEMM_NT, a, lda, b, ldb, c, ldc, nullptr, 0, m, n, k, false, g)) return e;
   FH_REQUIRE(head_dim == 32 || head_dim == 64 || head_dim == 128, "gemm_bf16_rope: head_dim must be 32, 64 or 128");
   FH_REQUIRE(rot_cols > 0 && rot_cols <= n && rot_cols % head_dim == 0,
              "gemm_bf16_rope: rot_cols must be a positive multiple of head_dim, at most n");

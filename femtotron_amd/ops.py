@@ -390,13 +390,25 @@ def gemm_supported(op: str, a: torch.Tensor, b: torch.Tensor) -> bool:
     """Whether fh_gemm_bf16 takes these operands: bf16 on one HIP device, 2-D
     with a contiguous last dim, k a multiple of 64, n (and for 'tn' also m) a
     multiple of 8, row strides multiples of 8 and 16-byte aligned data."""
+    return _gemm_operands_ok(op, a, b, False)
+
+
+def gemm_any_k_supported(op: str, a: torch.Tensor, b: torch.Tensor) -> bool:
+    """Whether fh_gemm_bf16_any_k takes these operands: as gemm_supported, but
+    any k of at least 64 ('tn'), or its multiples of 8 ('nt', 'nn')."""
+    return _gemm_operands_ok(op, a, b, True)
+
+
+def _gemm_operands_ok(op: str, a: torch.Tensor, b: torch.Tensor, any_k: bool) -> bool:
     if not (a.is_cuda and b.is_cuda and a.device == b.device and a.dtype == b.dtype == torch.bfloat16):
         return False
     dims = gemm_dims(op, a, b)
     if dims is None:
         return False
     m, n, k = dims
-    if min(m, n, k) <= 0 or k % 64 or n % 8 or (op == "tn" and m % 8):
+    if min(m, n, k) <= 0 or n % 8 or (op == "tn" and m % 8):
+        return False
+    if k % 64 and not (any_k and k >= 64 and (op == "tn" or k % 8 == 0)):
         return False
     for t in (a, b):
         if t.stride(1) != 1 or t.stride(0) % 8 or t.data_ptr() % 16:
@@ -405,14 +417,15 @@ def gemm_supported(op: str, a: torch.Tensor, b: torch.Tensor) -> bool:
 
 
 def gemm(op: str, a: torch.Tensor, b: torch.Tensor, *, residual: torch.Tensor | None = None,
-         out: torch.Tensor | None = None) -> torch.Tensor:
+         out: torch.Tensor | None = None, any_k: bool = False) -> torch.Tensor:
     """op(a) @ op(b) in bf16 with fp32 accumulation (fh_gemm_bf16):
     'nt': a [m,k] @ b[n,k]^T (nn.Linear forward), 'nn': a [m,k] @ b [k,n]
     (input gradient), 'tn': a[k,m]^T @ b [k,n] (weight gradient).  With
     `residual` ([m, n]) returns residual + to_bf16(product), rounded again;
-    `out` may be `residual` itself."""
+    `out` may be `residual` itself.  `any_k`: k need not be a multiple of 64
+    (fh_gemm_bf16_any_k, gemm_any_k_supported)."""
     _require_gpu(a, b, residual, out)
-    if not gemm_supported(op, a, b):
+    if not _gemm_operands_ok(op, a, b, any_k):
         raise ValueError(f"gemm({op}): unsupported operands {tuple(a.shape)} {a.stride()} x "
                          f"{tuple(b.shape)} {b.stride()} ({a.dtype}, {b.dtype})")
     m, n, k = gemm_dims(op, a, b)
@@ -425,25 +438,27 @@ def gemm(op: str, a: torch.Tensor, b: torch.Tensor, *, residual: torch.Tensor | 
         if t.stride(0) % 8 or t.data_ptr() % 16:
             raise ValueError(f"gemm({op}): {name} must be 16-byte aligned with a row stride % 8 == 0")
     code = _GEMM_OPS[op]
-    nbytes = _lib.lib().fh_gemm_bf16_workspace_size(code, m, n, k)
+    name = "fh_gemm_bf16_any_k" if any_k else "fh_gemm_bf16"
+    nbytes = getattr(_lib.lib(), name + "_workspace_size")(code, m, n, k)
     ws = torch.empty(nbytes, dtype=torch.uint8, device=a.device) if nbytes else None
-    _lib.call("fh_gemm_bf16", code, _ptr(a), a.stride(0), _ptr(b), b.stride(0), _ptr(c), c.stride(0),
+    _lib.call(name, code, _ptr(a), a.stride(0), _ptr(b), b.stride(0), _ptr(c), c.stride(0),
               _ptr(residual), 0 if residual is None else residual.stride(0), m, n, k, _ptr(ws),
               _stream(a))
     return c
 
 
-def gemm_grouped(op: str, items: list) -> list:
+def gemm_grouped(op: str, items: list, *, any_k: bool = False) -> list:
     """Up to three GEMMs of layout `op` with one k in one fh_gemm_bf16_grouped
     call: each item is (a, b, residual, out) with gemm()'s meaning (residual
-    and out may be None; out may be residual itself).  Returns the outputs."""
+    and out may be None; out may be residual itself), `any_k` too.  Returns the
+    outputs."""
     if not 1 <= len(items) <= 3:
         raise ValueError(f"gemm_grouped({op}): between 1 and 3 problems, got {len(items)}")
     probs = (_lib.FhGemmProblem * len(items))()
     outs, ks = [], set()
     for i, (a, b, residual, out) in enumerate(items):
         _require_gpu(a, b, residual, out)
-        if not gemm_supported(op, a, b):
+        if not _gemm_operands_ok(op, a, b, any_k):
             raise ValueError(f"gemm_grouped({op}): unsupported operands {tuple(a.shape)} {a.stride()} x "
                              f"{tuple(b.shape)} {b.stride()} ({a.dtype}, {b.dtype})")
         m, n, k = gemm_dims(op, a, b)
@@ -467,9 +482,10 @@ def gemm_grouped(op: str, items: list) -> list:
     if any(t is not None and t.device != a0.device for item in items for t in item) or \
             any(o.device != a0.device for o in outs):
         raise ValueError(f"gemm_grouped({op}): every operand and output must be on {a0.device}")
-    nbytes = _lib.lib().fh_gemm_bf16_grouped_workspace_size(code, len(items), probs, k)
+    name = "fh_gemm_bf16_grouped_any_k" if any_k else "fh_gemm_bf16_grouped"
+    nbytes = getattr(_lib.lib(), name + "_workspace_size")(code, len(items), probs, k)
     ws = torch.empty(nbytes, dtype=torch.uint8, device=a0.device) if nbytes else None
-    _lib.call("fh_gemm_bf16_grouped", code, len(items), probs, k, _ptr(ws), _stream(a0))
+    _lib.call(name, code, len(items), probs, k, _ptr(ws), _stream(a0))
     return outs
 
 

@@ -33,8 +33,9 @@ GEMM (``torch.mm`` on hipBLASLt/rocBLAS), by policy:
   kernels measured 3-7% faster; a TinyLlama step runs ~2% faster with them;
 * ``"library"``: always the library.
 
-Operands the kernel does not take (fp32, k not a multiple of 64, ...) go to
-the library under every policy.  ``gemm_dispatch_counts()`` tells tests and
+k need not be a multiple of 64 (fh_gemm_bf16_any_k: a weight gradient's k is the
+token count of a batch, of any length).  Operands the kernel does not take
+(fp32, k below 64, ...) go to the library under every policy.  ``gemm_dispatch_counts()`` tells tests and
 the benchmark which path ran.
 """
 from __future__ import annotations
@@ -97,7 +98,7 @@ def _library_shapes() -> dict[str, set]:
 
 def _choose_hand(op: str, a: torch.Tensor, b: torch.Tensor, table: str | None = None) -> bool:
     pol = _policy[0]
-    use = pol != "library" and ops.gemm_supported(op, a, b)
+    use = pol != "library" and (ops.gemm_supported(op, a, b) or ops.gemm_any_k_supported(op, a, b))
     if use and pol == "auto":
         use = ops.gemm_dims(op, a, b) not in _library_shapes()[table or op]
     return use
@@ -117,7 +118,7 @@ def _use_hand(op: str, a: torch.Tensor, b: torch.Tensor) -> bool:
 def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """x [T, in] @ w[out, in]^T."""
     if _use_hand("nt", x, w):
-        return ops.gemm("nt", x, w)
+        return ops.gemm("nt", x, w, any_k=True)
     return torch.mm(x, w.t())
 
 
@@ -139,7 +140,7 @@ def linear_residual(x: torch.Tensor, w: torch.Tensor, residual: torch.Tensor) ->
     hand-written GEMM's residual epilogue; otherwise the library GEMM followed
     by fh_add into `residual`)."""
     if _count(residual.is_contiguous() and _choose_hand("nt", x, w, "nt_res")):
-        return ops.gemm("nt", x, w, residual=residual, out=residual)
+        return ops.gemm("nt", x, w, residual=residual, out=residual, any_k=True)
     m = torch.mm(x, w.t())
     if not residual.is_contiguous():
         return residual.add_(m)  # one fp32 add, one rounding, as fh_add
@@ -149,14 +150,14 @@ def linear_residual(x: torch.Tensor, w: torch.Tensor, residual: torch.Tensor) ->
 def linear_dgrad(dy: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """dy [T, out] @ w [out, in]."""
     if _use_hand("nn", dy, w):
-        return ops.gemm("nn", dy, w)
+        return ops.gemm("nn", dy, w, any_k=True)
     return torch.mm(dy, w)
 
 
 def linear_wgrad(dy: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
     """dy [T, out]^T @ x [T, in]: the [out, in] weight gradient."""
     if _use_hand("tn", dy, x):
-        return ops.gemm("tn", dy, x)
+        return ops.gemm("tn", dy, x, any_k=True)
     return torch.mm(dy.t(), x)
 
 
@@ -171,7 +172,7 @@ def linear_wgrad_into(dy: torch.Tensor, x: torch.Tensor, grad: torch.Tensor) -> 
     if not _choose_hand("tn", dy, x):
         return False
     _count(True)
-    ops.gemm("tn", dy, x, residual=grad, out=grad)
+    ops.gemm("tn", dy, x, residual=grad, out=grad, any_k=True)
     return True
 
 
@@ -198,7 +199,7 @@ def linear_wgrad_group(items: list) -> list | None:
         return None
     for _ in items:
         _count(True)
-    outs = ops.gemm_grouped("tn", [(dy, x, g, g) for dy, x, g in items])
+    outs = ops.gemm_grouped("tn", [(dy, x, g, g) for dy, x, g in items], any_k=True)
     return [None if g is not None else o for (_, _, g), o in zip(items, outs)]
 
 

@@ -375,6 +375,16 @@ int fh_gemm_bf16(int op, const void* a, int64_t lda, const void* b, int64_t ldb,
                  int64_t ldc, const void* residual, int64_t ldr, int64_t m, int64_t n,
                  int64_t k, void* workspace, hipStream_t stream);
 
+/* fh_gemm_bf16 for any k >= 64: any k for FH_GEMM_TN, multiples of 8 for the
+ * other layouts (a weight gradient's k is the token count, which a batch of
+ * ragged sequences leaves odd; an ffn width of 688 is k of the down
+ * projection).  Where k is no multiple of 64 the last 64 k's are read as one
+ * stage whose repeated part counts as zeros.  Otherwise as fh_gemm_bf16. */
+size_t fh_gemm_bf16_any_k_workspace_size(int op, int64_t m, int64_t n, int64_t k);
+int fh_gemm_bf16_any_k(int op, const void* a, int64_t lda, const void* b, int64_t ldb, void* c,
+                       int64_t ldc, const void* residual, int64_t ldr, int64_t m, int64_t n,
+                       int64_t k, void* workspace, hipStream_t stream);
+
 /* Up to three GEMMs of one layout and one k in one launch: problem i is
  * fh_gemm_bf16(op, a, lda, b, ldb, c, ldc, residual, ldr, m, n, k) of its
  * fields, with the same roundings, requirements and residual rules.  The
@@ -410,6 +420,11 @@ typedef struct fh_gemm_problem {
 size_t fh_gemm_bf16_grouped_workspace_size(int op, int count, const fh_gemm_problem* problems, int64_t k);
 int fh_gemm_bf16_grouped(int op, int count, const fh_gemm_problem* problems, int64_t k, void* workspace,
                          hipStream_t stream);
+
+/* fh_gemm_bf16_grouped with the k of fh_gemm_bf16_any_k. */
+size_t fh_gemm_bf16_grouped_any_k_workspace_size(int op, int count, const fh_gemm_problem* problems, int64_t k);
+int fh_gemm_bf16_grouped_any_k(int op, int count, const fh_gemm_problem* problems, int64_t k, void* workspace,
+                               hipStream_t stream);
 
 /* The q/k/v projection with the rotary embedding in its epilogue: C = A B^T
  * (FH_GEMM_NT, no residual) and then, on columns [0, rot_cols) of C (the q and

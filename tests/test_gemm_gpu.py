@@ -270,6 +270,64 @@ def test_gemm_rejects_unsupported_operands():
         ops.gemm("nt", x, x, out=wide[:, :128])
 
 
+def _guarded(rows, cols, g):
+    """A [rows, cols] operand inside a larger NaN-filled buffer: what a read past it would meet."""
+    buf = torch.full((rows + 64, cols + 64), float("nan"), device=DEV, dtype=BF)
+    buf[:rows, :cols] = torch.randn(rows, cols, device=DEV, generator=g).to(BF)
+    return buf[:rows, :cols]
+
+
+@pytest.mark.parametrize("op", ["nt", "nn", "tn"])
+@pytest.mark.parametrize("m,n,k,form", [
+    (264, 520, 72, "tile"), (512, 768, 120, "tile"), (264, 264, 200, "tile"),  # two to four stages
+    (512, 768, 2056, "split"), (256, 512, 328, "split"),                       # the last slice ends ragged
+    (4352, 4096, 72, "persist"), (4352, 4096, 184, "persist"),                 # the next tile's stages loaded ahead
+    (4104, 4088, 2056, "stream"), (10240, 2048, 1000, "stream"),               # a segment ends ragged
+])
+@pytest.mark.parametrize("resid", [False, True])
+def test_any_k_matches_fp64_product(op, m, n, k, form, resid):
+    """k not a multiple of 64 (a multiple of 8, and for 'tn' an odd one): every form of the kernel, operands
+    followed by NaNs, against the fp64 product within the rounding bound; with a residual bit-identical to the
+    rounded product plus the residual."""
+    for kk in ((k, k + 1, k - 7) if op == "tn" else (k,)):
+        g = torch.Generator(device=DEV).manual_seed(m + kk)
+        shapes = {"nt": ((m, kk), (n, kk)), "nn": ((m, kk), (kk, n)), "tn": ((kk, m), (kk, n))}[op]
+        a, b = (_guarded(*s, g) for s in shapes)
+        assert not ops.gemm_supported(op, a, b) and ops.gemm_any_k_supported(op, a, b)
+        with pytest.raises(ValueError):
+            ops.gemm(op, a, b)
+        c = ops.gemm(op, a, b, any_k=True)
+        _check(op, a, b, c)
+        assert torch.equal(c, ops.gemm(op, a, b, any_k=True))
+        if resid:
+            r = torch.randn(m, n, device=DEV, generator=g).to(BF)
+            want = (r.float() + c.float()).to(BF)
+            assert torch.equal(ops.gemm(op, a, b, residual=r, out=r, any_k=True), want)
+
+
+@pytest.mark.parametrize("k", [65, 127, 999, 2002])
+@pytest.mark.parametrize("shapes", [[(2560, 2048), (2048, 2048), (2048, 5632)], [(512, 256), (256, 256)]])
+def test_grouped_any_k_matches_each_product(shapes, k):
+    g = torch.Generator(device=DEV).manual_seed(k)
+    items = [(_guarded(k, m, g), _guarded(k, n, g), None, None) for m, n in shapes]
+    with pytest.raises(ValueError):
+        ops.gemm_grouped("tn", items)
+    for (a, b, _, _), c in zip(items, ops.gemm_grouped("tn", items, any_k=True)):
+        _check("tn", a, b, c)
+
+
+def test_any_k_rejects_what_it_cannot_read():
+    x = torch.randn(256, 256, device=DEV).to(BF)
+    assert not ops.gemm_any_k_supported("tn", x[:63], x[:63])       # less than one stage
+    assert not ops.gemm_any_k_supported("nt", x[:, :100], x[:, :100])  # k contiguous: multiples of 8
+    L = _lib.lib()
+    for op, k in ((_lib.FH_GEMM_TN, 63), (_lib.FH_GEMM_NT, 100), (_lib.FH_GEMM_NN, 100)):
+        assert L.fh_gemm_bf16_any_k_workspace_size(op, 256, 256, k) == 0
+        st = L.fh_gemm_bf16_any_k(op, x.data_ptr(), 256, x.data_ptr(), 256, x.data_ptr(), 256, None, 0, 64, 64, k,
+                                  None, None)
+        assert st == 1 and b"at least 64" in L.fh_last_error()
+
+
 @pytest.mark.parametrize("m,seq,nh,nkv,hd,k,per_token", [
     (16384, 2048, 32, 4, 64, 2048, False),  # the TinyLlama q/k/v projection
     (600, 200, 8, 2, 64, 256, False),       # ragged m (not a multiple of the 256-row tile), 3 sequences
