@@ -36,6 +36,11 @@
 //     rate: 4 cycles per read and wave, against 4.8 with the 64-column rows
 //     XOR-swizzled), and a fragment's address is one per-lane offset plus
 //     immediates.
+// Outputs that 256 x 256 tiles would spread over few CUs run in 128 x 128 tiles
+// (k_gemm_mid, chosen by gemm_plan): the same stages and ring with a quarter of
+// the wave's outputs, 80 KB of LDS and two workgroups per CU.  The GEMMs of a
+// 2048-wide layer at 256 tokens 430 -> 265 us of kernel time, at 999 tokens 606 ->
+// 476 us.
 // The MFMA is issued as (B fragment, A fragment), so each lane's four
 // accumulator values are consecutive along n (C's contiguous index).  The finished tile goes through LDS so that
 // every global store writes whole rows.
@@ -74,7 +79,7 @@ namespace {
 constexpr int kTm = 256, kTn = 256, kTk = 64;  // block tile and stage depth
 constexpr int kSubBytes = kTk * 128;           // KO sub-tile: [64 k x 64] bf16
 
-enum Epi { EPI_STORE = 0, EPI_RESIDUAL = 1, EPI_PARTIAL = 2, EPI_ROPE = 3, EPI_STREAM = 4 };
+enum Epi { EPI_STORE = 0, EPI_RESIDUAL = 1, EPI_PARTIAL = 2, EPI_ROPE = 3, EPI_STREAM = 4, EPI_GROUP = 5 };
 
 // The rotary embedding of EPI_ROPE: columns [0, rot_cols) of C are heads of
 // hd columns (hd a power of two dividing the 256-column tile, so no head
@@ -123,9 +128,10 @@ struct GemmArgs {
   // > 0: the tail in XCD slabs (tail_tiles = slab_chunks * grid / 8; see k_gemm)
   int slab_chunks;
   GemmRope rope;
-  // EPI_STREAM: the problems (one, or several of the same op and k that share
-  // the launch), tiles numbered problem by problem
+  // EPI_STREAM, EPI_GROUP: the problems (one, or several of the same op and k
+  // that share the launch), tiles numbered problem by problem
   int ngroup;
+  int grouped;  // a call of the grouped entry points
   GemmProblem grp[kMaxGroup];
 };
 
@@ -156,7 +162,9 @@ __device__ __forceinline__ uint4 rope_fwd_chunk(uint4 x, uint4 p, uint4 c, uint4
 // (~130 extra moves per stage).  The compiler's hazard checks do not see an
 // asm MFMA: the kernel pads the two hazards this code has itself (an
 // accumulator zeroed just before its first MFMA; MFMA results read right
-// after the last one) with s_nop.
+// after the last one) with s_nop.  The 16 accumulators of the 128 x 128 tile go
+// through the builtin: the allocator keeps them in place, and where it copies
+// one (it peels the last stage of that loop) the compiler's checks apply.
 __device__ __forceinline__ f32x4 mfma16(bf16x8 a, bf16x8 b, f32x4 c) {
   asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
   return c;
@@ -199,11 +207,12 @@ __device__ __forceinline__ bf16x8 frag_ko16(const char* tile, int t0, int o, int
 // any LDS read); the kernel waits for its loads itself (s_waitcnt vmcnt) before
 // the barrier that hands a stage to the other waves.
 
-// Wave q's quarter of one operand's stage is 8 runs jj, each one 1 KB load
-// into slot (8q + jj) of the stage's tile.  KC: tile rows 64q + 8jj .. +7
-// (clamped to `last`), k0 .. k0+63: lane i fills 16-byte slot i%8 of row i/8,
-// i.e. it loads the chunk the swizzle puts there.  KO: unit jj of sub-tile q,
-// k rows k0 + 8jj .. +7, columns o0 + 64q .. +63 (chunks clamped to `last`,
+// Wave q's quarter of one operand's stage (2 W rows or columns, W = 128 or 64) is
+// W / 16 runs jj, each one 1 KB load into slot (q W / 16 + jj) of the stage's
+// tile.  KC: tile rows W/2 q + 8jj .. +7 (clamped to `last`), k0 .. k0+63: lane i
+// fills 16-byte slot i%8 of row i/8, i.e. it loads the chunk the swizzle puts
+// there.  KO: unit u of a sub-tile (W = 128: unit jj of sub-tile q; 64: unit
+// 4 (q%2) + jj of sub-tile q/2), k rows k0 + 8u .. +7, the sub-tile's 64 columns (chunks clamped to `last`,
 // the last 8-column chunk start): lane i fills 16-byte slot i%16 of block
 // i/16, i.e. chunk i%2 of that block's 32 bytes of row (i%16)/2.  A load's address is a wave-uniform 64-bit base
 // (clamped too, so the lane offset is never negative) plus a 32-bit lane offset
@@ -213,29 +222,31 @@ __device__ __forceinline__ bf16x8 frag_ko16(const char* tile, int t0, int o, int
 // rows for KO); recomputing (k0 + 8jj) * ld for every KO load put a 64-bit
 // scalar multiply chain in front of each one, ~180 cycles per stage and KO
 // operand.  A KO lane offset is the same for every run.
-template <bool KO>
+template <bool KO, int W>
 struct RunPlan {
-  const char* run[8];
-  uint32_t off[KO ? 1 : 8];
+  static constexpr int RUNS = W / 16;  // runs of a wave per operand and stage
+  const char* run[RUNS];
+  uint32_t off[KO ? 1 : RUNS];
   int64_t k_bytes;  // bytes per k (KO: a row, ld elements; KC: one element)
 
   __device__ __forceinline__ void init(const uint16_t* base, int64_t ld, int o0, int last, int q, int lane) {
     if constexpr (KO) {
-      const int col0 = min(o0 + 64 * q, last);
+      const int sub = o0 + 64 * (q * W / 128), unit0 = q * (W / 16) % 8;
+      const int col0 = min(sub, last);
 #pragma unroll
-      for (int jj = 0; jj < 8; ++jj)
-        run[jj] = reinterpret_cast<const char*>(base + static_cast<int64_t>(8 * jj) * ld + col0);
+      for (int jj = 0; jj < RUNS; ++jj)
+        run[jj] = reinterpret_cast<const char*>(base + static_cast<int64_t>(8 * (unit0 + jj)) * ld + col0);
       const int r = (lane >> 1) & 7, c = 2 * (lane >> 4) + (lane & 1);
-      off[0] = static_cast<uint32_t>(r * static_cast<int>(ld) + min(o0 + 64 * q + 8 * c, last) - col0) * 2u;
+      off[0] = static_cast<uint32_t>(r * static_cast<int>(ld) + min(sub + 8 * c, last) - col0) * 2u;
       k_bytes = ld * 2;
     } else {
       const int lr = lane >> 3;
 #pragma unroll
-      for (int jj = 0; jj < 8; ++jj) {
-        const int row0 = min(o0 + 64 * q + 8 * jj, last);
+      for (int jj = 0; jj < RUNS; ++jj) {
+        const int row0 = min(o0 + W / 2 * q + 8 * jj, last);
         const int c = (lane & 7) ^ swz<64>(8 * jj + lr);
         run[jj] = reinterpret_cast<const char*>(base + static_cast<int64_t>(row0) * ld);
-        off[jj] = static_cast<uint32_t>((min(o0 + 64 * q + 8 * jj + lr, last) - row0) * static_cast<int>(ld) + 8 * c) * 2u;
+        off[jj] = static_cast<uint32_t>((min(o0 + W / 2 * q + 8 * jj + lr, last) - row0) * static_cast<int>(ld) + 8 * c) * 2u;
       }
       k_bytes = 2;
     }
@@ -261,17 +272,21 @@ __device__ __forceinline__ void bar() {
   __builtin_amdgcn_sched_barrier(0);
 }
 
-constexpr int kSlot = 32768;  // one operand's stage: [256 x 64] bf16
-constexpr int kRing = 5;      // operand slots in LDS (160 KB)
+// One operand's stage: [2 W x 64] bf16.
+template <int W>
+constexpr int kSlotOf = 2 * W * 128;
+constexpr int kSlot = kSlotOf<128>;
+constexpr int kRing = 5;  // operand slots in LDS (160 KB, or 80 KB for W = 64)
 
 // Zeroes the first `n` of the 64 k's of this wave's quarter of an operand's
 // stage, which has landed (lane i filled 16-byte slot i of each 1 KB run, with
 // the k's of RunPlan's layout; n is a multiple of 8 for KC).
-template <bool KO>
-__device__ __forceinline__ void zero_repeat(char* quarter, int n, int lane) {
+template <bool KO, int W>
+__device__ __forceinline__ void zero_repeat(char* quarter, int n, int wave, int lane) {
 #pragma unroll 1
-  for (int jj = 0; jj < 8; ++jj) {
-    const int k = KO ? 8 * jj + ((lane >> 1) & 7) : 8 * ((lane & 7) ^ swz<64>(8 * jj + (lane >> 3)));
+  for (int jj = 0; jj < W / 16; ++jj) {
+    const int k = KO ? 8 * (wave * (W / 16) % 8 + jj) + ((lane >> 1) & 7)
+                     : 8 * ((lane & 7) ^ swz<64>(8 * jj + (lane >> 3)));
     if (k < n) *reinterpret_cast<uint4*>(quarter + jj * 1024 + lane * 16) = make_uint4(0, 0, 0, 0);
   }
 }
@@ -283,17 +298,18 @@ __device__ __forceinline__ void wait_vm_n() {
 
 __device__ __forceinline__ int mod5(int v) { return v >= 5 ? v - 5 : v; }
 
-// Origin of tile t: tiles run in groups of GM = 4 m-tiles, n-major inside a
+// Origin of tile t: tiles run in groups of 1024 rows (GM m-tiles), n-major inside a
 // group, so consecutive tiles (and the workgroups of one XCD) share B columns
 // and A rows in L2.
+template <int W = 128>
 __device__ __forceinline__ void tile_origin(const GemmArgs& g, int t, int& m0, int& n0) {
-  constexpr int GM = 4;
+  constexpr int GM = 512 / W;
   const int width = GM * g.tiles_n;
   const int gi = t / width, first_m = gi * GM;
   const int gm = min(g.tiles_m - first_m, GM);
   const int tw = t - gi * width;
-  m0 = (first_m + tw % gm) * kTm;
-  n0 = (tw / gm) * kTn;
+  m0 = (first_m + tw % gm) * (2 * W);
+  n0 = (tw / gm) * (2 * W);
 }
 
 // The arguments of the problem that holds tile t of a stream GEMM's tile
@@ -326,20 +342,22 @@ __device__ __forceinline__ GemmArgs for_tile(const GemmArgs& g, int& t) {
 // to_part, as fp32 to pdst (the tile's origin, row stride pld).  EPI_STREAM
 // ends with a barrier, as the workgroup's next tile reuses the LDS ring.
 // RAGGED: k may be no multiple of 64.
-template <bool A_KO, bool B_KO, int EPI, bool RAGGED>
+template <bool A_KO, bool B_KO, int EPI, bool RAGGED, int W>
 __device__ __forceinline__ void gemm_tile(const GemmArgs& g, char* ring, int t, int s_begin, int nst,
                                           float* pdst, int64_t pld, bool to_part) {
-  const int tid = threadIdx.x, lane = tid & 63, hl = lane >> 5;
+  constexpr int F = W / 16, RUNS = W / 16;  // fragments per operand and k32 step; loads per operand and stage
+  constexpr int SLOT = kSlotOf<W>, QUARTER = SLOT / 4;
+  const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   int m0, n0;
-  tile_origin(g, t, m0, n0);
+  tile_origin<W>(g, t, m0, n0);
 
-  RunPlan<A_KO> pa;
-  RunPlan<B_KO> pb;
+  RunPlan<A_KO, W> pa;
+  RunPlan<B_KO, W> pb;
   pa.init(g.a, g.lda, m0, A_KO ? g.m - 8 : g.m - 1, wave, lane);
   pb.init(g.b, g.ldb, n0, B_KO ? g.n - 8 : g.n - 1, wave, lane);
   typedef __attribute__((address_space(3))) char* lptr;
-  const uint32_t ring0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lptr)ring)) + wave * 8192;
+  const uint32_t ring0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lptr)ring)) + wave * QUARTER;
 
   auto k_of = [&](int step) __attribute__((always_inline)) {
     const int64_t k0 = static_cast<int64_t>(s_begin + min(step, nst - 1)) * kTk;
@@ -351,7 +369,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, char* ring, int t, 
   auto dma = [&](auto op_tag, int step, int slot, int jj) __attribute__((always_inline)) {
     constexpr int OP = decltype(op_tag)::value;
     const int64_t k0 = k_of(step);
-    const uint32_t lds_slot = ring0 + slot * kSlot + jj * 1024;
+    const uint32_t lds_slot = ring0 + slot * SLOT + jj * 1024;
     if constexpr (OP == 0) pa.load(k0 * pa.k_bytes, jj, lds_slot);
     else pb.load(k0 * pb.k_bytes, jj, lds_slot);
   };
@@ -366,94 +384,95 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, char* ring, int t, 
   using OpB = std::integral_constant<int, 1>;
 
   const int wm = wave & 1, wn = wave >> 1;
-  // v_mfma_f32_16x16x32_bf16: the wave's 128 x 128 outputs are 8 (n) x 8 (m)
-  // accumulators of 16 x 16; a stage is two k32 steps of 64 MFMAs.  Operand
+  // v_mfma_f32_16x16x32_bf16: the wave's W x W outputs are F (n) x F (m)
+  // accumulators of 16 x 16; a stage is two k32 steps of F * F MFMAs.  Operand
   // lane i holds row/column i%16 and k 8*(i/16) .. +7 of the step.
   const int a_off = lane_off_kc16(lane);
   const int t0 = lane_off_tr16(lane);
-  bf16x8 fa[2][8], fb[2][8];
-  // Fragment r = 0..15 of k32 step ks (order B0, A0..A7, B1..B7: the order
+  bf16x8 fa[2][F], fb[2][F];
+  // Fragment r = 0..2F-1 of k32 step ks (order B0, A0.., B1..: the order
   // the MFMAs first use them) from slots sa (A) and sb (B).
   auto rd1 = [&](int sa, int sb, int ks, int buf, int r) __attribute__((always_inline)) {
-    if (r >= 1 && r <= 8) {
-      const char* tile = ring + sa * kSlot;
-      const int j = r - 1, o = 128 * wm + 16 * j;
+    if (r >= 1 && r <= F) {
+      const char* tile = ring + sa * SLOT;
+      const int j = r - 1, o = W * wm + 16 * j;
       fa[buf][j] = A_KO ? frag_ko16(tile, t0, o, ks) : frag_kc16(tile, a_off, o, ks);
     } else {
-      const char* tile = ring + sb * kSlot;
-      const int i = r == 0 ? 0 : r - 8, o = 128 * wn + 16 * i;
+      const char* tile = ring + sb * SLOT;
+      const int i = r == 0 ? 0 : r - F, o = W * wn + 16 * i;
       fb[buf][i] = B_KO ? frag_ko16(tile, t0, o, ks) : frag_kc16(tile, a_off, o, ks);
     }
   };
-  f32x4 acc[8][8];
+  f32x4 acc[F][F];
 #pragma unroll
-  for (int i = 0; i < 8; ++i)
+  for (int i = 0; i < F; ++i)
 #pragma unroll
-    for (int j = 0; j < 8; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < F; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
   auto mf1 = [&](int buf, int nn) __attribute__((always_inline)) {
-    const int i = nn >> 3, j = nn & 7;
-    acc[i][j] = mfma16(fb[buf][i], fa[buf][j], acc[i][j]);
+    const int i = nn / F, j = nn % F;
+    if constexpr (W == 128) acc[i][j] = mfma16(fb[buf][i], fa[buf][j], acc[i][j]);
+    else acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[buf][i], fa[buf][j], acc[i][j], 0, 0, 0);
   };
 
   // Operand u (A of stage x: u = 2x, B: 2x+1) lives in ring slot u % 5.
   // Prologue: stages 0 and 1, wait for stage 0, read its step-0 fragments.
 #pragma unroll
-  for (int jj = 0; jj < 8; ++jj) dma(OpA(), 0, 0, jj);
+  for (int jj = 0; jj < RUNS; ++jj) dma(OpA(), 0, 0, jj);
 #pragma unroll
-  for (int jj = 0; jj < 8; ++jj) dma(OpB(), 0, 1, jj);
+  for (int jj = 0; jj < RUNS; ++jj) dma(OpB(), 0, 1, jj);
 #pragma unroll
-  for (int jj = 0; jj < 8; ++jj) dma(OpA(), 1, 2, jj);
+  for (int jj = 0; jj < RUNS; ++jj) dma(OpA(), 1, 2, jj);
 #pragma unroll
-  for (int jj = 0; jj < 8; ++jj) dma(OpB(), 1, 3, jj);
-  wait_vm_n<16>();
+  for (int jj = 0; jj < RUNS; ++jj) dma(OpB(), 1, 3, jj);
+  wait_vm_n<2 * RUNS>();
   // The stage that repeats k's, if this range ends with it (-1: none).
   [[maybe_unused]] const int xr = g.repeat > 0 && s_begin + nst == g.total_steps ? nst - 1 : -1;
   [[maybe_unused]] auto zero = [&](int sa, int sb) __attribute__((always_inline)) {
-    zero_repeat<A_KO>(ring + sa * kSlot + wave * 8192, g.repeat, lane);
-    zero_repeat<B_KO>(ring + sb * kSlot + wave * 8192, g.repeat, lane);
+    zero_repeat<A_KO, W>(ring + sa * SLOT + wave * QUARTER, g.repeat, wave, lane);
+    zero_repeat<B_KO, W>(ring + sb * SLOT + wave * QUARTER, g.repeat, wave, lane);
     wait_lds();
   };
   if constexpr (RAGGED)
     if (xr == 0) zero(0, 1);
   bar();
 #pragma unroll
-  for (int r = 0; r < 16; ++r) {
+  for (int r = 0; r < 2 * F; ++r) {
     rd1(0, 1, 0, 0, r);
     __builtin_amdgcn_sched_barrier(0);
   }
 
   // Stage x (A in slot s, B in s+1; stage x+1 in s+2, s+3; s+4 free):
-  //   step 0: 64 MFMAs on buffer 0 while step 1's fragments are read into
-  //     buffer 1 (one read per 4 MFMAs) and A(x+2) is loaded into s+4;
+  //   step 0: its MFMAs on buffer 0 while step 1's fragments are read into
+  //     buffer 1 (one read per F / 2 MFMAs) and A(x+2) is loaded into s+4;
   //   then each wave waits for its reads and for every load but A(x+2)'s
   //   (stage x+1 complete in LDS), and the barrier: stage x's slots are
   //   read no more;
-  //   step 1: 64 MFMAs on buffer 1 while the next stage's step-0 fragments
+  //   step 1: its MFMAs on buffer 1 while the next stage's step-0 fragments
   //     are read into buffer 0 and B(x+2) is loaded into slot s.
   int s = 0;
   for (int x = 0; x < nst; ++x) {
     const int sB = mod5(s + 1), nA = mod5(s + 2), nB = mod5(s + 3), fA = mod5(s + 4);
     // VALU writes of an accumulator (the zeroing before the loop) need wait
     // states before an MFMA reads it.
-    asm volatile("s_nop 4");
+    if constexpr (W == 128) asm volatile("s_nop 4");
 #pragma unroll
-    for (int p = 0; p < 64; ++p) {
-      if ((p & 3) == 0) rd1(s, sB, 1, 1, p >> 2);
-      if ((p & 7) == 1) set_m0(ring0 + fA * kSlot + (p >> 3) * 1024);
-      if ((p & 7) == 2) dma_m0(OpA(), x + 2, p >> 3);
+    for (int p = 0; p < F * F; ++p) {
+      if (p % (F / 2) == 0) rd1(s, sB, 1, 1, p / (F / 2));
+      if (p % F == 1) set_m0(ring0 + fA * SLOT + (p / F) * 1024);
+      if (p % F == 2) dma_m0(OpA(), x + 2, p / F);
       mf1(0, p);
       __builtin_amdgcn_sched_barrier(0);
     }
     wait_lds();
-    wait_vm_n<8>();
+    wait_vm_n<RUNS>();
     if constexpr (RAGGED)
       if (x + 1 == xr) zero(nA, nB);
     bar();
 #pragma unroll
-    for (int p = 0; p < 64; ++p) {
-      if ((p & 3) == 0) rd1(nA, nB, 0, 0, p >> 2);
-      if ((p & 7) == 1) set_m0(ring0 + s * kSlot + (p >> 3) * 1024);
-      if ((p & 7) == 2) dma_m0(OpB(), x + 2, p >> 3);
+    for (int p = 0; p < F * F; ++p) {
+      if (p % (F / 2) == 0) rd1(nA, nB, 0, 0, p / (F / 2));
+      if (p % F == 1) set_m0(ring0 + s * SLOT + (p / F) * 1024);
+      if (p % F == 2) dma_m0(OpB(), x + 2, p / F);
       mf1(1, p);
       __builtin_amdgcn_sched_barrier(0);
     }
@@ -462,7 +481,8 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, char* ring, int t, 
     // (at most 18): after the last stage, before anything (the staging
     // below, or a copy the register allocator places at the loop's exit)
     // reads the accumulators.
-    if (x == nst - 1) asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7");
+    if constexpr (W == 128)
+      if (x == nst - 1) asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7");
   }
   __builtin_amdgcn_sched_barrier(0);
   // The re-loads past the end and the last stale fragment reads complete
@@ -472,62 +492,66 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, char* ring, int t, 
   bar();
 
   if (EPI == EPI_PARTIAL || (EPI == EPI_STREAM && to_part)) {
-    // The fp32 tile goes through LDS in two halves of 128 rows ([128 rows x
-    // 256 columns], 16-byte chunk c of row r stored at chunk c ^ (r % 16));
-    // lane i of a wave then stores chunk i of a 1 KB row.
+    // The fp32 tile goes through LDS in two halves of W rows ([W rows x 2 W
+    // columns], 16-byte chunk c of row r stored at chunk c ^ (r % 16)); the
+    // lanes of a wave then store the chunks of 128 / W whole rows.
+    constexpr int RB = 8 * W, CH = W / 2, RI = 128 / W;  // bytes and chunks of a row, rows per store
 #pragma unroll
     for (int half = 0; half < 2; ++half) {
       if (wm == half) {
         // lane i of accumulator (i, j): row 16 j + i%16, columns
-        // 128 wn + 16 i + 4 (i/16) .. +3 (one 16-byte chunk)
+        // W wn + 16 i + 4 (i/16) .. +3 (one 16-byte chunk)
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
+        for (int j = 0; j < F; ++j) {
           const int r = 16 * j + (lane & 15);
 #pragma unroll
-          for (int i = 0; i < 8; ++i) {
-            const int chunk = 32 * wn + 4 * i + (lane >> 4);
+          for (int i = 0; i < F; ++i) {
+            const int chunk = W / 4 * wn + 4 * i + (lane >> 4);
             const f32x4& v = acc[i][j];
-            *reinterpret_cast<float4*>(ring + r * 1024 + ((chunk ^ (r & 15)) << 4)) =
+            *reinterpret_cast<float4*>(ring + r * RB + ((chunk ^ (r & 15)) << 4)) =
                 make_float4(v[0], v[1], v[2], v[3]);
           }
         }
       }
       wait_lds();
       bar();
-      const int col = n0 + 4 * lane;
+      const int chunk = lane % CH, col = n0 + 4 * chunk;
 #pragma unroll 4
-      for (int q2 = 0; q2 < 32; ++q2) {
-        const int r = 32 * wave + q2;
-        const float4 v = *reinterpret_cast<const float4*>(ring + r * 1024 + ((lane ^ (r & 15)) << 4));
-        const int mrow = m0 + 128 * half + r;
+      for (int q2 = 0; q2 < W / 4 / RI; ++q2) {
+        const int r = W / 4 * wave + RI * q2 + lane / CH;
+        const float4 v = *reinterpret_cast<const float4*>(ring + r * RB + ((chunk ^ (r & 15)) << 4));
+        const int mrow = m0 + W * half + r;
         if (mrow < g.m && col < g.n)
-          *reinterpret_cast<float4*>(pdst + static_cast<int64_t>(128 * half + r) * pld + 4 * lane) = v;
+          *reinterpret_cast<float4*>(pdst + static_cast<int64_t>(W * half + r) * pld + 4 * chunk) = v;
       }
       wait_lds();
       bar();
     }
   } else {
-    // The bf16 tile goes through LDS ([256 rows x 256 columns], 16-byte chunk
+    // The bf16 tile goes through LDS ([2 W rows x 2 W columns], 16-byte chunk
     // c of row r stored at chunk c ^ (r % 16)) so that every global store
-    // writes whole rows: lane i of a wave stores chunk i % 32 of row 2q + i / 32.
-    // lane i of accumulator (i, j): row 128 wm + 16 j + i%16, columns
-    // 128 wn + 16 i + 4 (i/16) .. +3 (half a 16-byte chunk)
+    // writes whole rows: the lanes of a wave store the chunks of 256 / W rows.
+    // lane i of accumulator (i, j): row W wm + 16 j + i%16, columns
+    // W wn + 16 i + 4 (i/16) .. +3 (half a 16-byte chunk)
+    constexpr int RB = 4 * W, CH = W / 4, RI = 256 / W;  // bytes and chunks of a row, rows per store
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const int r = 128 * wm + 16 * j + (lane & 15);
+    for (int j = 0; j < F; ++j) {
+      const int r = W * wm + 16 * j + (lane & 15);
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const int chunk = 16 * wn + 2 * i + (lane >> 5);
+      for (int i = 0; i < F; ++i) {
+        const int chunk = W / 8 * wn + 2 * i + (lane >> 5);
         const f32x4& v = acc[i][j];
-        *reinterpret_cast<uint2*>(ring + r * 512 + ((chunk ^ (r & 15)) << 4) + 8 * ((lane >> 4) & 1)) =
+        *reinterpret_cast<uint2*>(ring + r * RB + ((chunk ^ (r & 15)) << 4) + 8 * ((lane >> 4) & 1)) =
             make_uint2(pk_bf16(v[0], v[1]), pk_bf16(v[2], v[3]));
       }
     }
     wait_lds();
     bar();
-    const int chunk = lane & 31;
+    const int chunk = lane % CH;
     const int col = n0 + 8 * chunk;
     if constexpr (EPI == EPI_ROPE) {
+      static_assert(EPI != EPI_ROPE || W == 128, "the rotation runs in the 256-wide tile");
+      const int hl = lane >> 5;
       // Rotated columns read their partner chunk (hd/2 columns away, same
       // head, same row) from the staged tile and the cos / sin chunks of
       // their own columns; eight rows' loads are issued before their math.
@@ -564,12 +588,12 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, char* ring, int t, 
       return;
     }
 #pragma unroll 4
-    for (int q2 = 0; q2 < 32; ++q2) {
-      const int r = 64 * wave + 2 * q2 + hl;
-      const uint4 v = *reinterpret_cast<const uint4*>(ring + r * 512 + ((chunk ^ (r & 15)) << 4));
+    for (int q2 = 0; q2 < W / 2 / RI; ++q2) {
+      const int r = W / 2 * wave + RI * q2 + lane / CH;
+      const uint4 v = *reinterpret_cast<const uint4*>(ring + r * RB + ((chunk ^ (r & 15)) << 4));
       const int mrow = m0 + r;
       if (mrow >= g.m || col >= g.n) continue;
-      if (EPI == EPI_RESIDUAL || (EPI == EPI_STREAM && g.r != nullptr)) {
+      if (EPI == EPI_RESIDUAL || ((EPI == EPI_STREAM || EPI == EPI_GROUP) && g.r != nullptr)) {
         const uint4 rv = *reinterpret_cast<const uint4*>(g.r + mrow * g.ldr + col);
         *reinterpret_cast<uint4*>(g.c + mrow * g.ldc + col) = make_uint4(
             add_bf16x2(rv.x, v.x), add_bf16x2(rv.y, v.y), add_bf16x2(rv.z, v.z), add_bf16x2(rv.w, v.w));
@@ -723,8 +747,8 @@ __device__ __forceinline__ void gemm_persist(const GemmArgs& g, char* ring, int 
       wait_vm_n<8>();
       if constexpr (RAGGED)
         if (x == xr) {
-          zero_repeat<A_KO>(ring + nA * kSlot + wave * 8192, g.repeat, lane);
-          zero_repeat<B_KO>(ring + nB * kSlot + wave * 8192, g.repeat, lane);
+          zero_repeat<A_KO, 128>(ring + nA * kSlot + wave * 8192, g.repeat, wave, lane);
+          zero_repeat<B_KO, 128>(ring + nB * kSlot + wave * 8192, g.repeat, wave, lane);
           wait_lds();
         }
       bar();
@@ -836,7 +860,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
         break;
       }
       const GemmArgs pg = for_tile(g, t);
-      gemm_tile<A_KO, B_KO, EPI, RAGGED>(pg, ring, t, k0, len, slot, kTn, len < ki);
+      gemm_tile<A_KO, B_KO, EPI, RAGGED, 128>(pg, ring, t, k0, len, slot, kTn, len < ki);
     }
   } else {
     const int slice = lid / g.tiles, t = lid - slice * g.tiles;
@@ -846,8 +870,34 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     float* pdst = EPI == EPI_PARTIAL
                       ? g.part + static_cast<int64_t>(slice) * g.m * g.n + static_cast<int64_t>(m0) * g.n + n0
                       : nullptr;
-    gemm_tile<A_KO, B_KO, EPI, RAGGED>(g, ring, t, s_begin, min(g.total_steps - s_begin, g.steps_per_slice), pdst,
+    gemm_tile<A_KO, B_KO, EPI, RAGGED, 128>(g, ring, t, s_begin, min(g.total_steps - s_begin, g.steps_per_slice), pdst,
                                g.n, EPI == EPI_PARTIAL);
+  }
+}
+
+// The 128 x 128 tile: W = 64, so a workgroup needs 80 KB of LDS and half the
+// registers, and two run on a CU.  One tile, or one K slice of it
+// (EPI_PARTIAL), per workgroup; EPI_GROUP: the tiles of a group's problems.
+template <bool A_KO, bool B_KO, int EPI, bool RAGGED>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_gemm_mid(GemmArgs g) {
+  __shared__ __align__(16) char ring[kRing * kSlotOf<64>];
+  const int nb8 = gridDim.x >> 3;
+  const int lid = (blockIdx.x & 7) * nb8 + (blockIdx.x >> 3);
+  if (lid >= g.grid) return;
+  if constexpr (EPI == EPI_GROUP) {
+    int t = lid;
+    const GemmArgs pg = for_tile(g, t);
+    gemm_tile<A_KO, B_KO, EPI, RAGGED, 64>(pg, ring, t, 0, g.total_steps, nullptr, 0, false);
+  } else {
+    const int slice = lid / g.tiles, t = lid - slice * g.tiles;
+    const int s_begin = slice * g.steps_per_slice;
+    int m0, n0;
+    tile_origin<64>(g, t, m0, n0);
+    float* pdst = EPI == EPI_PARTIAL
+                      ? g.part + static_cast<int64_t>(slice) * g.m * g.n + static_cast<int64_t>(m0) * g.n + n0
+                      : nullptr;
+    gemm_tile<A_KO, B_KO, EPI, RAGGED, 64>(g, ring, t, s_begin, min(g.total_steps - s_begin, g.steps_per_slice), pdst,
+                                           g.n, EPI == EPI_PARTIAL);
   }
 }
 
@@ -993,9 +1043,40 @@ int stream_grid() { return std::max(8, device_cus() / 8 * 8); }
 struct GemmPlan {
   int slices;   // K slices of the split form
   bool stream;  // the stream form models faster
+  bool mid;     // in 128 x 128 tiles (never the stream form)
+  double us;    // modelled time
 };
 
-GemmPlan gemm_plan(int64_t m, int64_t n, int64_t k) {
+constexpr int kMid = 128;  // tile of k_gemm_mid
+
+// Modelled microseconds of the two tile sizes, fitted to 370 products (NT, NN
+// and TN of three widths, 16 to 4096 tokens, each timed in 256 x 256 tiles and in
+// 128 x 128 tiles over 1 to 8 slices): stages per CU times a stage's time, a
+// cost per tile and per launch, and for K slices writing and re-reading the
+// partials.  A 128 x 128 stage takes 0.41-0.56 us for a quarter of the work of
+// the 256 x 256 stage's 1.18 (LDS reads per MFMA double), so the small tiles win
+// only where the large ones leave CUs idle or split K: 256 x 11264 x 2048 32 ->
+// 20 us, 512 x 2048 x 2048 28 -> 14, 999 x 2048 x 2048 31 -> 19, 256 x 2048 x
+// 5632 30 -> 18 (8 slices), 2002 x 2048 x 2048 37 -> 21; 4096 x 11264 x 2048
+// would lose (148 -> 161).  Over those products the choice is within 1% of the
+// better one on average and at most 5% behind the 256 x 256 form.
+constexpr double kBigStage = 1.18, kBigTile = 2.65, kBigFixed = 5.5, kStreamFixed = 6.0;
+constexpr double kMidFixed = 4.0, kMidTile = 0.9, kReduceFixed = 5.0, kReducePerMB = 0.27;
+constexpr double kMidStage[3] = {0.41, 0.54, 0.56};  // NT, NN, TN
+constexpr double kMidMargin = 0.97;                  // the small tiles must model this much faster
+
+int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
+
+double reduce_us(int64_t m, int64_t n, int64_t slices) {
+  return slices > 1 ? kReduceFixed + kReducePerMB * static_cast<double>(slices) * m * n * 4e-6 : 0.0;
+}
+
+double mid_us(int op, int64_t tiles, int64_t m, int64_t n, int64_t per, int64_t slices, int cus) {
+  return static_cast<double>(ceil_div(tiles * slices, cus)) * per * kMidStage[op] + kMidFixed +
+         kMidTile * static_cast<double>(tiles * slices) / cus + reduce_us(m, n, slices);
+}
+
+GemmPlan gemm_plan(int op, int64_t m, int64_t n, int64_t k) {
   const int64_t tiles = ((m + kTm - 1) / kTm) * ((n + kTn - 1) / kTn), steps = (k + kTk - 1) / kTk;
   const int cus = device_cus();
   const double per_slice = 48.0 * static_cast<double>(m) * n / (655360.0 * static_cast<double>(k));
@@ -1011,13 +1092,26 @@ GemmPlan gemm_plan(int64_t m, int64_t n, int64_t k) {
   }
   // Slices of ceil(steps / S) stages; fewer if that leaves the last one empty.
   const int64_t per = (steps + best - 1) / best;
-  GemmPlan p{static_cast<int>((steps + per - 1) / per), false};
+  GemmPlan p{static_cast<int>((steps + per - 1) / per), false, false, 0.0};
   const int64_t sg = stream_grid(), tail = tiles % sg;
   if (tiles > sg && tail > 0 && steps >= 4) {
     const double segs = static_cast<double>(std::min<int64_t>(2 * sg, sg + tail));
     const double cost = static_cast<double>(tiles / sg) + static_cast<double>(tail) / sg +
                         per_slice * segs * (kTm * kTn) / (static_cast<double>(m) * n);
     p.stream = cost < 0.97 * best_cost;
+  }
+  p.us = p.stream ? static_cast<double>(tiles) / cus * (steps * kBigStage + kBigTile) + kBigFixed + kStreamFixed
+                  : static_cast<double>(ceil_div(tiles * p.slices, cus)) * (per * kBigStage + kBigTile) + kBigFixed +
+                        reduce_us(m, n, p.slices);
+  const int64_t mid_tiles = ceil_div(m, kMid) * ceil_div(n, kMid);
+  double bound = kMidMargin * p.us;
+  for (int s = 1; s <= 8 && (s == 1 || s <= k / 256); ++s) {
+    const int64_t mper = ceil_div(steps, s), ms = ceil_div(steps, mper);
+    const double us = mid_us(op, mid_tiles, m, n, mper, ms, cus);
+    if (us < bound - 1e-9) {
+      bound = us;
+      p = GemmPlan{static_cast<int>(ms), false, true, us};
+    }
   }
   return p;
 }
@@ -1069,6 +1163,33 @@ void launch_persist(int op, const GemmArgs& g, hipStream_t stream) {
     hipLaunchKernelGGL((k_gemm_persist<true, true, false, RAGGED>), grid, block, 0, stream, g);
 }
 
+template <bool A_KO, bool B_KO, bool RAGGED>
+void launch_mid(const GemmArgs& g, unsigned blocks, bool partial, hipStream_t stream) {
+  const dim3 grid(blocks), block(256);
+  if (g.grouped)
+    hipLaunchKernelGGL((k_gemm_mid<A_KO, B_KO, EPI_GROUP, RAGGED>), grid, block, 0, stream, g);
+  else if (partial)
+    hipLaunchKernelGGL((k_gemm_mid<A_KO, B_KO, EPI_PARTIAL, RAGGED>), grid, block, 0, stream, g);
+  else if (g.r != nullptr)
+    hipLaunchKernelGGL((k_gemm_mid<A_KO, B_KO, EPI_RESIDUAL, RAGGED>), grid, block, 0, stream, g);
+  else
+    hipLaunchKernelGGL((k_gemm_mid<A_KO, B_KO, EPI_STORE, RAGGED>), grid, block, 0, stream, g);
+}
+
+template <bool RAGGED>
+void launch_mid_op(int op, const GemmArgs& g, unsigned blocks, bool partial, hipStream_t stream) {
+  switch (op) {
+    case FH_GEMM_NT: launch_mid<false, false, RAGGED>(g, blocks, partial, stream); break;
+    case FH_GEMM_NN: launch_mid<false, true, RAGGED>(g, blocks, partial, stream); break;
+    default: launch_mid<true, true, RAGGED>(g, blocks, partial, stream); break;
+  }
+}
+
+void launch_mid_op(int op, const GemmArgs& g, unsigned blocks, bool partial, hipStream_t stream) {
+  if (g.repeat > 0) launch_mid_op<true>(op, g, blocks, partial, stream);
+  else launch_mid_op<false>(op, g, blocks, partial, stream);
+}
+
 bool valid_op(int op) { return op == FH_GEMM_NT || op == FH_GEMM_NN || op == FH_GEMM_TN; }
 
 }  // namespace
@@ -1079,8 +1200,8 @@ using namespace fh;
 namespace {
 
 // The stream form's segment slots, or the split form's partials.
-size_t gemm_workspace(int64_t m, int64_t n, int64_t k) {
-  const GemmPlan p = gemm_plan(m, n, k);
+size_t gemm_workspace(int op, int64_t m, int64_t n, int64_t k) {
+  const GemmPlan p = gemm_plan(op, m, n, k);
   if (p.stream) return stream_workspace_bytes();
   return p.slices > 1 ? static_cast<size_t>(p.slices) * m * n * sizeof(float) : 0;
 }
@@ -1093,12 +1214,12 @@ bool any_k_ok(int op, int64_t k) { return k >= kTk && (op == FH_GEMM_TN || k % 8
 
 extern "C" size_t fh_gemm_bf16_workspace_size(int op, int64_t m, int64_t n, int64_t k) {
   if (!valid_op(op) || m <= 0 || n <= 0 || k <= 0 || k % 64) return 0;
-  return gemm_workspace(m, n, k);
+  return gemm_workspace(op, m, n, k);
 }
 
 extern "C" size_t fh_gemm_bf16_any_k_workspace_size(int op, int64_t m, int64_t n, int64_t k) {
   if (!valid_op(op) || m <= 0 || n <= 0 || !any_k_ok(op, k)) return 0;
-  return gemm_workspace(m, n, k);
+  return gemm_workspace(op, m, n, k);
 }
 
 namespace {
@@ -1150,12 +1271,29 @@ int gemm_setup(int op, const void* a, int64_t lda, const void* b, int64_t ldb, v
   return FH_OK;
 }
 
-// Launches the GEMM of g in the stream form (stream: segment slots in
-// `workspace`, split tiles summed by k_gemm_fixup) or over `slices` K slices
-// (partials in `workspace`, summed by k_gemm_reduce, when slices > 1).
-int gemm_run(int op, GemmArgs& g, int slices, bool stream_form, void* workspace, hipStream_t stream) {
+// Makes every tile count of g that of 128 x 128 tiles.
+void use_mid_tiles(GemmArgs& g) {
+  int tile0 = 0;
+  for (int i = 0; i < g.ngroup; ++i) {
+    GemmProblem& p = g.grp[i];
+    p.tiles_m = (p.m + kMid - 1) / kMid;
+    p.tiles_n = (p.n + kMid - 1) / kMid;
+    p.tile0 = tile0;
+    tile0 += p.tiles_m * p.tiles_n;
+  }
+  g.tiles_m = g.grp[0].tiles_m;
+  g.tiles_n = g.grp[0].tiles_n;
+  g.tiles = tile0;
+}
+
+// Launches the GEMM of g in the stream form (segment slots in `workspace`,
+// split tiles summed by k_gemm_fixup) or over the plan's K slices (partials in
+// `workspace`, summed by k_gemm_reduce, when there is more than one).
+int gemm_run(int op, GemmArgs& g, const GemmPlan& plan, void* workspace, hipStream_t stream) {
+  const int slices = plan.slices;
   g.part = static_cast<float*>(workspace);
-  if (stream_form) {
+  if (plan.mid) use_mid_tiles(g);
+  if (plan.stream) {
     const int sg = stream_grid();
     g.grid = sg;
     g.full_rounds = g.tiles / sg;
@@ -1171,7 +1309,7 @@ int gemm_run(int op, GemmArgs& g, int slices, bool stream_form, void* workspace,
   g.steps_per_slice = (g.total_steps + slices - 1) / slices;
 #if FH_GEMM_PERSIST
   // The residual epilogue in this form: the forward (NT) layout only.
-  if (slices == 1 && (g.r == nullptr || op == FH_GEMM_NT) && g.rope.cos == nullptr && g.total_steps >= 2 &&
+  if (!plan.mid && slices == 1 && (g.r == nullptr || op == FH_GEMM_NT) && g.rope.cos == nullptr && g.total_steps >= 2 &&
       g.m % kTm == 0 && g.n % kTn == 0 && g.lda < (int64_t(1) << 24) && g.ldb < (int64_t(1) << 24) &&
       g.tiles > stream_grid()) {
     g.grid = stream_grid();
@@ -1185,7 +1323,8 @@ int gemm_run(int op, GemmArgs& g, int slices, bool stream_form, void* workspace,
   g.grid = static_cast<int>(logical);
   const unsigned blocks = static_cast<unsigned>((logical + 7) / 8 * 8);
   const bool partial = slices > 1, resid = g.r != nullptr;
-  launch_op(op, g, blocks, partial, resid, stream);
+  if (plan.mid) launch_mid_op(op, g, blocks, partial, stream);
+  else launch_op(op, g, blocks, partial, resid, stream);
   if (partial) {
     const int64_t mn = static_cast<int64_t>(g.m) * g.n;
     const unsigned rb = static_cast<unsigned>((mn / 4 + 255) / 256);
@@ -1208,10 +1347,10 @@ int gemm_impl(int op, const void* a, int64_t lda, const void* b, int64_t ldb, vo
               hipStream_t stream, const char* name) {
   GemmArgs g;
   if (int e = gemm_setup(op, a, lda, b, ldb, c, ldc, residual, ldr, m, n, k, any_k, g)) return e;
-  const GemmPlan p = gemm_plan(m, n, k);
+  const GemmPlan p = gemm_plan(op, m, n, k);
   FH_REQUIRE((p.slices == 1 && !p.stream) || (workspace && aligned16(workspace)),
              std::string(name + 3) + ": workspace (" + name + "_workspace_size bytes) required");
-  if (int e = gemm_run(op, g, p.slices, p.stream, workspace, stream)) return e;
+  if (int e = gemm_run(op, g, p, workspace, stream)) return e;
   return check_launch(name);
 }
 
@@ -1231,10 +1370,45 @@ extern "C" int fh_gemm_bf16_any_k(int op, const void* a, int64_t lda, const void
 
 namespace {
 
-// A group runs as one stream launch when its tiles fill more than a round of
-// the CUs (the tail, if any, in XCD slabs when it is a whole number of
-// 32-tile chunks); otherwise its problems run one by one, each by its own plan.
-bool group_stream(int64_t tiles, int64_t steps) { return tiles > stream_grid() && steps >= 4; }
+// How a group runs: one stream launch (only with more than a round of 256 x 256
+// tiles; the tail, if any, in XCD slabs when it is a whole number of 32-tile
+// chunks), one launch of 128 x 128 tiles, or its problems one by one, each by
+// its own plan.  Modelled times fitted to the weight gradients of four widths
+// over 64 to 8192 tokens.  Few k-steps leave the stream form little to set
+// against its segments and their sum (2048-wide: 46 -> 23 us at 256 tokens, 69 ->
+// 60 at 999; the debug model's three, 2 tiles each: 34 -> 6 us at 256), many
+// tiles leave little to share (4096-wide MHA, 1712 tiles: 178 -> 130 us one by
+// one at 512 tokens); at 4096 tokens it is the fastest of the three (2048-wide:
+// 152 us against 180 and 189).  The other layouts, which no layer groups, run as
+// one stream launch wherever that is allowed.
+enum class GroupForm { kStream, kMid, kSeparate };
+
+bool stream_allowed(int64_t tiles, int64_t steps) { return tiles > stream_grid() && steps >= 4; }
+
+GroupForm group_form(int op, int count, const fh_gemm_problem* problems, int64_t k) {
+  const int64_t steps = ceil_div(k, kTk), sg = stream_grid();
+  int64_t tiles = 0, mid_tiles = 0;
+  double separate = 0.0;
+  for (int i = 0; i < count; ++i) {
+    const int64_t m = problems[i].m, n = problems[i].n;
+    tiles += ceil_div(m, kTm) * ceil_div(n, kTn);
+    mid_tiles += ceil_div(m, kMid) * ceil_div(n, kMid);
+    separate += gemm_plan(op, m, n, k).us;
+  }
+  if (op != FH_GEMM_TN) return stream_allowed(tiles, steps) ? GroupForm::kStream : GroupForm::kSeparate;
+  GroupForm form = GroupForm::kSeparate;
+  double us = separate;
+  if (stream_allowed(tiles, steps)) {
+    const int64_t tail = tiles % sg;
+    const double stream = static_cast<double>(tiles) / sg * (1.37 * steps + 6.5) + (tail ? 22.0 + 0.12 * tail : 0.0);
+    if (0.95 * stream <= separate) {
+      form = GroupForm::kStream;
+      us = 0.95 * stream;
+    }
+  }
+  const double mid = static_cast<double>(ceil_div(mid_tiles, device_cus())) * (0.55 * steps + 1.6) + kMidFixed;
+  return mid < us ? GroupForm::kMid : form;
+}
 
 // Checks every problem of a group and fills g with the group's table (tiles
 // numbered problem by problem).
@@ -1253,27 +1427,39 @@ int group_setup(int op, int count, const fh_gemm_problem* probs, int64_t k, bool
     tile0 += gi.tiles;
   }
   g.ngroup = count;
+  g.grouped = 1;
   g.tiles = tile0;
   return FH_OK;
 }
 
-size_t group_workspace(int count, const fh_gemm_problem* problems, int64_t k) {
+// The problems' own workspace where they run one by one; else the stream form's
+// segment slots where its tiles allow it (the 128 x 128 tiles need none, but the
+// size stays one of a group's sizes).
+size_t group_workspace(int op, int count, const fh_gemm_problem* problems, int64_t k) {
   int64_t tiles = 0;
   size_t most = 0;
   for (int i = 0; i < count; ++i) {
     const int64_t m = problems[i].m, n = problems[i].n;
     if (m <= 0 || n <= 0) return 0;
-    tiles += ((m + kTm - 1) / kTm) * ((n + kTn - 1) / kTn);
-    most = std::max(most, gemm_workspace(m, n, k));
+    tiles += ceil_div(m, kTm) * ceil_div(n, kTn);
+    most = std::max(most, gemm_workspace(op, m, n, k));
   }
-  return group_stream(tiles, (k + kTk - 1) / kTk) ? stream_workspace_bytes() : most;
+  if (group_form(op, count, problems, k) == GroupForm::kSeparate) return most;
+  return stream_allowed(tiles, ceil_div(k, kTk)) ? stream_workspace_bytes() : 0;
 }
 
 int group_impl(int op, int count, const fh_gemm_problem* problems, int64_t k, bool any_k, void* workspace,
                hipStream_t stream) {
   GemmArgs g;
   if (int e = group_setup(op, count, problems, k, any_k, g)) return e;
-  if (!group_stream(g.tiles, g.total_steps)) {
+  const GroupForm form = group_form(op, count, problems, k);
+  if (form == GroupForm::kMid) {
+    use_mid_tiles(g);
+    g.grid = g.tiles;
+    launch_mid_op(op, g, static_cast<unsigned>((g.tiles + 7) / 8 * 8), false, stream);
+    return check_launch("fh_gemm_bf16_grouped");
+  }
+  if (form == GroupForm::kSeparate) {
     for (int i = 0; i < count; ++i) {
       const fh_gemm_problem& p = problems[i];
       if (int e = gemm_impl(op, p.a, p.lda, p.b, p.ldb, p.c, p.ldc, p.residual, p.ldr, p.m, p.n, k, any_k,
@@ -1303,7 +1489,7 @@ int group_impl(int op, int count, const fh_gemm_problem* problems, int64_t k, bo
 extern "C" size_t fh_gemm_bf16_grouped_workspace_size(int op, int count, const fh_gemm_problem* problems,
                                                       int64_t k) {
   if (!valid_op(op) || count < 1 || count > kMaxGroup || problems == nullptr || k <= 0 || k % kTk) return 0;
-  return group_workspace(count, problems, k);
+  return group_workspace(op, count, problems, k);
 }
 
 extern "C" int fh_gemm_bf16_grouped(int op, int count, const fh_gemm_problem* problems, int64_t k,
@@ -1314,7 +1500,7 @@ extern "C" int fh_gemm_bf16_grouped(int op, int count, const fh_gemm_problem* pr
 extern "C" size_t fh_gemm_bf16_grouped_any_k_workspace_size(int op, int count, const fh_gemm_problem* problems,
                                                             int64_t k) {
   if (!valid_op(op) || count < 1 || count > kMaxGroup || problems == nullptr || !any_k_ok(op, k)) return 0;
-  return group_workspace(count, problems, k);
+  return group_workspace(op, count, problems, k);
 }
 
 extern "C" int fh_gemm_bf16_grouped_any_k(int op, int count, const fh_gemm_problem* problems, int64_t k,
@@ -1341,6 +1527,6 @@ extern "C" int fh_gemm_bf16_rope(const void* a, int64_t lda, const void* b, int6
   g.rope.per_token = cos_per_token ? 1 : 0;
   g.rope.seq_len = static_cast<int>(seq_len);
   g.rope.seq = FastDiv(static_cast<uint32_t>(seq_len));
-  if (int e = gemm_run(FH_GEMM_NT, g, 1, false, nullptr, stream)) return e;  // whole K: the epilogue sees final sums
+  if (int e = gemm_run(FH_GEMM_NT, g, GemmPlan{1, false, false, 0.0}, nullptr, stream)) return e;  // whole K: the epilogue sees final sums
   return check_launch("fh_gemm_bf16_rope");
 }

@@ -356,7 +356,8 @@ int fh_embedding_bwd(fh_dtype dt, const void* dy, const int64_t* ids, void* dwei
  * Requirements: k % 64 == 0; n % 8 == 0 (and m % 8 == 0 for FH_GEMM_TN);
  * lda, ldb, ldc and ldr multiples of 8 (< 2^26 for lda, ldb); A, B, C and the
  * residual 16-byte aligned; m, n, k < 2^30.
- * When the output has few 256 x 256 tiles the k range is split into slices
+ * Where 256 x 256 tiles would leave compute units idle the output runs in
+ * 128 x 128 tiles.  When the output has few tiles the k range is split into slices
  * whose fp32 partial sums go to `workspace` (fh_gemm_bf16_workspace_size bytes;
  * 0 = none needed) and are added in slice order; when its tiles leave the
  * last round of CUs partly idle, each CU instead takes an equal share of the
@@ -395,7 +396,9 @@ int fh_gemm_bf16_any_k(int op, const void* a, int64_t lda, const void* b, int64_
  * together fill more than one round of the CUs they share one launch in the
  * stream form (every CU an equal share of the group's k-steps, problem by
  * problem; split tiles summed in k order from fp32 segments in `workspace`);
- * otherwise each runs as its own fh_gemm_bf16 call.  Bitwise deterministic
+ * otherwise each runs as its own fh_gemm_bf16 call.  FH_GEMM_TN groups of few
+ * tokens instead run as one launch of smaller whole tiles, or one by one, where
+ * that models faster.  Bitwise deterministic
  * (the form depends only on the problems' sizes, k and the CU count); a
  * problem's result may differ in the last bit from its own fh_gemm_bf16 call,
  * whose form may split k differently.  The problems' outputs must not overlap

@@ -270,6 +270,26 @@ def test_gemm_rejects_unsupported_operands():
         ops.gemm("nt", x, x, out=wide[:, :128])
 
 
+@pytest.mark.parametrize("op", ["nt", "nn", "tn"])
+@pytest.mark.parametrize("m,n,k,pad", [
+    (128, 128, 64, 0), (8, 128, 128, 8), (136, 120, 192, 0),     # one 128 x 128 tile and its edges, one to three stages
+    (256, 11264, 2048, 0), (1000, 2048, 2048, 0),                # whole K, two workgroups on some CUs
+    (256, 2048, 5632, 0), (16, 2048, 11264, 64), (512, 264, 16384, 0),  # K slices
+])
+def test_mid_tiles_match_and_add_the_residual(op, m, n, k, pad):
+    """Sizes that run in 128 x 128 tiles: the product within its bound, repeatable, the residual bit-identical to
+    the rounded product plus the residual, in place too."""
+    g = torch.Generator(device=DEV).manual_seed(m + 3 * n + 7 * k)
+    a, b = _operands(op, m, n, k, g, pad)
+    c = ops.gemm(op, a, b)
+    _check(op, a, b, c)
+    assert torch.equal(c, ops.gemm(op, a, b))
+    r = torch.randn(m, n, device=DEV, generator=g).to(BF)
+    want = (r.float() + c.float()).to(BF)
+    assert torch.equal(ops.gemm(op, a, b, residual=r), want)
+    assert torch.equal(ops.gemm(op, a, b, residual=r, out=r), want)
+
+
 def _guarded(rows, cols, g):
     """A [rows, cols] operand inside a larger NaN-filled buffer: what a read past it would meet."""
     buf = torch.full((rows + 64, cols + 64), float("nan"), device=DEV, dtype=BF)
@@ -279,15 +299,19 @@ def _guarded(rows, cols, g):
 
 @pytest.mark.parametrize("op", ["nt", "nn", "tn"])
 @pytest.mark.parametrize("m,n,k,form", [
-    (264, 520, 72, "tile"), (512, 768, 120, "tile"), (264, 264, 200, "tile"),  # two to four stages
-    (512, 768, 2056, "split"), (256, 512, 328, "split"),                       # the last slice ends ragged
-    (4352, 4096, 72, "persist"), (4352, 4096, 184, "persist"),                 # the next tile's stages loaded ahead
-    (4104, 4088, 2056, "stream"), (10240, 2048, 1000, "stream"),               # a segment ends ragged
+    # 128 x 128 tiles: two to four stages, K slices of which the last ends ragged
+    (264, 520, 72, "mid"), (512, 768, 120, "mid"), (4352, 4096, 184, "mid"), (512, 768, 2056, "mid split"),
+    (128, 136, 712, "mid split"), (8, 8, 72, "mid"),
+    # 256 x 256 tiles
+    (2000, 14336, 520, "tile"), (1000, 28672, 2056, "tile"),
+    (1000, 4096, 14344, "split"), (1032, 4104, 14344, "split"),           # the last slice ends ragged
+    (8192, 4096, 1032, "persist"), (10240, 2048, 1000, "persist"),        # the next tile's stages loaded ahead
+    (4104, 4088, 2056, "stream"), (10240, 2048, 4104, "stream"),          # a segment ends ragged
 ])
 @pytest.mark.parametrize("resid", [False, True])
 def test_any_k_matches_fp64_product(op, m, n, k, form, resid):
-    """k not a multiple of 64 (a multiple of 8, and for 'tn' an odd one): every form of the kernel, operands
-    followed by NaNs, against the fp64 product within the rounding bound; with a residual bit-identical to the
+    """k not a multiple of 64 (a multiple of 8, and for 'tn' an odd one): every form of the kernels (`form`: the
+    one that most layouts take at these sizes), operands followed by NaNs, against the fp64 product within the rounding bound; with a residual bit-identical to the
     rounded product plus the residual."""
     for kk in ((k, k + 1, k - 7) if op == "tn" else (k,)):
         g = torch.Generator(device=DEV).manual_seed(m + kk)
