@@ -643,6 +643,82 @@ struct QTileDma {
   }
 };
 
+// ------------------------------------------ backward: dK, dV (bf16), few workgroups
+// The dK/dV kernels give a workgroup a key block of one kv head and loop over
+// all of the group's query heads, so one short sequence with few kv heads is few
+// workgroups (1 x 256 tokens, 32 / 4 heads of 64: 4 of them on 256 CUs).  There
+// the group's heads are split over `n` workgroups (HeadSplit), each of which
+// writes its fp32 sums to `part`; k_attn_dkdv_sum adds them in head order and
+// stores dK and dV as the kernels do.  63 -> 12 + 6 us at that size, 81 -> 21 + 7 us at
+// 3 x 333.
+struct HeadSplit {
+  float* part;  // [n][2][B*S][nkv][HD] (dK, dV), n > 1
+  int n;
+  __device__ __forceinline__ float* row(int split, int which, int64_t tokens, int64_t tok, int nkv, int kvh,
+                                        int hd) const {
+    return part + (((static_cast<int64_t>(split) * 2 + which) * tokens + tok) * nkv + kvh) * hd;
+  }
+};
+
+// store_rows_T's elements as fp32.
+template <int HD>
+__device__ __forceinline__ void store_rows_T_f32(float* out_row, const f32x16 (&acc)[HD / 32], int hl) {
+#pragma unroll
+  for (int dt = 0; dt < HD / 32; ++dt)
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+      *reinterpret_cast<float4*>(out_row + dt * 32 + 8 * g + 4 * hl) =
+          make_float4(acc[dt][4 * g], acc[dt][4 * g + 1], acc[dt][4 * g + 2], acc[dt][4 * g + 3]);
+}
+
+// One thread: dims d .. d+3 and d + HD/2 .. of one (token, kv head) of dK and dV.
+template <int HD>
+__global__ __launch_bounds__(256) void k_attn_dkdv_sum(HeadSplit hs, uint16_t* __restrict__ dk, int64_t lddk,
+                                                       uint16_t* __restrict__ dv, int64_t lddv, int S,
+                                                       int64_t tokens, int nkv, float scale,
+                                                       RopeRows<uint16_t> rope) {
+  constexpr int C = HD / 8;
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  if (i >= tokens * nkv * C) return;
+  const int d = static_cast<int>(i % C) * 4;
+  const int64_t th = i / C, t = th / nkv;
+  const int kvh = static_cast<int>(th - t * nkv);
+#pragma unroll
+  for (int which = 0; which < 2; ++which) {
+    float a[8];
+    for (int sp = 0; sp < hs.n; ++sp) {
+      const float* p = hs.row(sp, which, tokens, t, nkv, kvh, HD) + d;
+      const float4 lo = *reinterpret_cast<const float4*>(p), hi = *reinterpret_cast<const float4*>(p + HD / 2);
+      const float v[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+#pragma unroll
+      for (int e = 0; e < 8; ++e) a[e] = sp == 0 ? v[e] : a[e] + v[e];
+    }
+    if (which == 0) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) a[e] *= scale;
+      if (rope.cos) {
+        const int64_t b = t / S, at = rope.row(b * S, static_cast<int>(t - b * S)) * HD + d;
+        float c0[4], c1[4], s0[4], s1[4];
+        unpack4_bf16(*reinterpret_cast<const uint2*>(rope.cos + at), c0);
+        unpack4_bf16(*reinterpret_cast<const uint2*>(rope.cos + at + HD / 2), c1);
+        unpack4_bf16(*reinterpret_cast<const uint2*>(rope.sin + at), s0);
+        unpack4_bf16(*reinterpret_cast<const uint2*>(rope.sin + at + HD / 2), s1);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          float o0, o1;
+          rope_pair<uint16_t, true>(round_bf(a[e]), round_bf(a[e + 4]), c0[e], c1[e], s0[e], s1[e], o0, o1);
+          a[e] = o0;
+          a[e + 4] = o1;
+        }
+      }
+    }
+    uint16_t* out = which == 0 ? dk + t * lddk : dv + t * lddv;
+    out += static_cast<int64_t>(kvh) * HD + d;
+    *reinterpret_cast<uint2*>(out) = make_uint2(pk_bf16(a[0], a[1]), pk_bf16(a[2], a[3]));
+    *reinterpret_cast<uint2*>(out + HD / 2) = make_uint2(pk_bf16(a[4], a[5]), pk_bf16(a[6], a[7]));
+  }
+}
+
 // ------------------------------------------ backward: dK, dV (bf16), fused roles
 // Used for head_dim <= 64.  Block = 8 waves for one (batch, kv head) and two
 // key blocks of 128 keys, j and nkb-1-j, taken one after the other (causal
@@ -732,7 +808,7 @@ __global__ __launch_bounds__(DkdvFusedTiles<HD>::NT) __attribute__((amdgpu_waves
     const uint16_t* __restrict__ v, int64_t ldv, const uint16_t* __restrict__ dO, int64_t lddo,
     const float* __restrict__ nl2, const float* __restrict__ delta, uint16_t* __restrict__ dk,
     int64_t lddk, uint16_t* __restrict__ dv, int64_t lddv, int S, int nh, int nkv, int group,
-    float scale_log2, float scale, RopeRows<uint16_t> rope) {
+    float scale_log2, float scale, RopeRows<uint16_t> rope, HeadSplit hs, bool paired) {
   constexpr int NWH = DkdvFusedTiles<HD>::NWH, NT = DkdvFusedTiles<HD>::NT;
   constexpr int BKN = NWH * 32, BQ = DkdvFusedTiles<HD>::BQ, NS = HD / 16, ND = HD / 32;
   constexpr int TILE = BQ * 2 * HD;
@@ -759,9 +835,10 @@ __global__ __launch_bounds__(DkdvFusedTiles<HD>::NT) __attribute__((amdgpu_waves
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform (scalar) index
   const int half = wave / NWH, wq = wave % NWH;
   const XcdOrder ord = xcd_order();
-  const int bk = ord.y, b = bk / nkv, kvh = bk - b * nkv;
+  const int bk = ord.y / hs.n, split = ord.y - bk * hs.n, b = bk / nkv, kvh = bk - b * nkv;
+  const int gs = group / hs.n;  // query heads of this workgroup
   const int nkb = (S + BKN - 1) / BKN;
-  const int jlo = ord.rank, jhi = nkb - 1 - ord.rank;
+  const int jlo = ord.rank, jhi = paired ? nkb - 1 - ord.rank : -1;
   const int64_t tok0 = static_cast<int64_t>(b) * S;
   const int hrow = 32 * half;  // this wave's first query row within a tile
   // The LDS read offsets include the wave's first row (its byte offset lies
@@ -770,7 +847,8 @@ __global__ __launch_bounds__(DkdvFusedTiles<HD>::NT) __attribute__((amdgpu_waves
   // additions in the loop (32 per query tile otherwise).
   int a_off = lane_off_a<HD>(lane) + hrow * 2 * HD;
   int b0 = lane_off_b<HD>(lane, 0) + hrow * 2 * HD, b8 = lane_off_b<HD>(lane, 8) + hrow * 2 * HD;
-  const int64_t h0 = static_cast<int64_t>(kvh) * group;
+  const int64_t h0 = static_cast<int64_t>(kvh) * group + split * gs;
+  const int64_t tokens = static_cast<int64_t>(gridDim.y / (nkv * hs.n)) * S;
   const uint16_t* qg = q + tok0 * ldq + h0 * HD;
   const uint16_t* gg = dO + tok0 * lddo + h0 * HD;
   const float* lg = nl2 + (static_cast<int64_t>(b) * nh + h0) * S;
@@ -804,12 +882,12 @@ __global__ __launch_bounds__(DkdvFusedTiles<HD>::NT) __attribute__((amdgpu_waves
     // loaded straight into the other LDS stage while item it is multiplied;
     // each wave waits for its own loads before the barrier that ends the item.
     const int qt0 = (jb * BKN) / BQ;
-    const int n_it = group * (qt_end - qt0);
+    const int n_it = gs * (qt_end - qt0);
     QTileDma<HD, BQ, NT> pre;
     pre.start(qt_end, ldq, lddo, wave, lane);
-    pre.fetch(qg, ldq, gg, lddo, lg, dg, S, qt0, group, lds.sq0a, lds.sg0a, lds.sl0a, lds.sd0a, wave, lane);
+    pre.fetch(qg, ldq, gg, lddo, lg, dg, S, qt0, gs, lds.sq0a, lds.sg0a, lds.sl0a, lds.sd0a, wave, lane);
     if (n_it > 1)
-      pre.fetch(qg, ldq, gg, lddo, lg, dg, S, qt0, group, lds.sq0b, lds.sg0b, lds.sl0b, lds.sd0b, wave, lane);
+      pre.fetch(qg, ldq, gg, lddo, lg, dg, S, qt0, gs, lds.sq0b, lds.sg0b, lds.sl0b, lds.sd0b, wave, lane);
     wait_loads();
     __syncthreads();
     int cqt = qt_end - 1, chh = 0;  // query tile and head of the current item
@@ -818,12 +896,12 @@ __global__ __launch_bounds__(DkdvFusedTiles<HD>::NT) __attribute__((amdgpu_waves
   {                                                                                               \
     refresh_offsets(a_off, b0, b8);                                                               \
     if ((IT) + 2 < n_it)                                                                          \
-      pre.fetch(qg, ldq, gg, lddo, lg, dg, S, qt0, group, QN, GN, LN, DN, wave, lane);            \
+      pre.fetch(qg, ldq, gg, lddo, lg, dg, S, qt0, gs, QN, GN, LN, DN, wave, lane);            \
     const int qh = cqt * BQ + hrow; /* first query of this wave's half */                         \
     if ((IT) < n_it && qh + 31 >= kw) /* some query of the half reaches this wave's keys */      \
       dkdv_tile<HD>(QC, GC, LC, DC, kf, vf, dkacc, dvacc, a_off, b0, b8, hrow, qh, kw, ki, S,      \
                     scale_log2, hl);                                                              \
-    if (++chh == group) {                                                                         \
+    if (++chh == gs) {                                                                         \
       chh = 0;                                                                                    \
       --cqt;                                                                                      \
     }                                                                                             \
@@ -856,13 +934,19 @@ __global__ __launch_bounds__(DkdvFusedTiles<HD>::NT) __attribute__((amdgpu_waves
       for (int dt = 0; dt < ND; ++dt)
 #pragma unroll
         for (int j = 0; j < 16; ++j) dkacc[dt][j] = dkacc[dt][j] + other[dt * 16 + j][lane];
-      if (ki < S) store_grad_row<HD>(dk + (tok0 + ki) * lddk + static_cast<int64_t>(kvh) * HD, dkacc, scale, hl, rope, tok0, ki);
+      if (ki < S) {
+        if (hs.n > 1) store_rows_T_f32<HD>(hs.row(split, 0, tokens, tok0 + ki, nkv, kvh, HD), dkacc, hl);
+        else store_grad_row<HD>(dk + (tok0 + ki) * lddk + static_cast<int64_t>(kvh) * HD, dkacc, scale, hl, rope, tok0, ki);
+      }
     } else {
 #pragma unroll
       for (int dt = 0; dt < ND; ++dt)
 #pragma unroll
         for (int j = 0; j < 16; ++j) dvacc[dt][j] = other[dt * 16 + j][lane] + dvacc[dt][j];
-      if (ki < S) store_rows_T<HD>(dv + (tok0 + ki) * lddv + static_cast<int64_t>(kvh) * HD, dvacc, 1.f, hl);
+      if (ki < S) {
+        if (hs.n > 1) store_rows_T_f32<HD>(hs.row(split, 1, tokens, tok0 + ki, nkv, kvh, HD), dvacc, hl);
+        else store_rows_T<HD>(dv + (tok0 + ki) * lddv + static_cast<int64_t>(kvh) * HD, dvacc, 1.f, hl);
+      }
     }
   }
 }
@@ -896,7 +980,7 @@ __global__ __launch_bounds__(DkdvTiles<HD>::NT) __attribute__((amdgpu_waves_per_
     const uint16_t* __restrict__ v, int64_t ldv, const uint16_t* __restrict__ dO, int64_t lddo,
     const float* __restrict__ nl2, const float* __restrict__ delta, uint16_t* __restrict__ dk,
     int64_t lddk, uint16_t* __restrict__ dv, int64_t lddv, int S, int nh, int nkv, int group,
-    float scale_log2, float scale, RopeRows<uint16_t> rope) {
+    float scale_log2, float scale, RopeRows<uint16_t> rope, HeadSplit hs) {
   constexpr int NKS = DkdvTiles<HD>::NKS, NT = DkdvTiles<HD>::NT, BQ = DkdvTiles<HD>::BQ;
   constexpr int BKN = NKS * 32, NS = HD / 16, ND = HD / 32, NQT = BQ / 32, TILE = BQ * 2 * HD;
   // Two LDS stages as separate arrays (the loop below is unrolled by two),
@@ -913,7 +997,8 @@ __global__ __launch_bounds__(DkdvTiles<HD>::NT) __attribute__((amdgpu_waves_per_
   const bool role_a = wave < NKS;
   const int sub = role_a ? wave : wave - NKS;
   const XcdOrder ord = xcd_order();
-  const int bk = ord.y, b = bk / nkv, kvh = bk - b * nkv;
+  const int bk = ord.y / hs.n, split = ord.y - bk * hs.n, b = bk / nkv, kvh = bk - b * nkv;
+  const int gs = group / hs.n;  // query heads of this workgroup
   const int kb0 = ord.rank * BKN;  // heaviest (earliest keys) first
   const int kw = kb0 + sub * 32, ki = kw + l32;
   const int64_t tok0 = static_cast<int64_t>(b) * S;
@@ -933,15 +1018,15 @@ __global__ __launch_bounds__(DkdvTiles<HD>::NT) __attribute__((amdgpu_waves_per_
 
   // iteration space: (query tiles from the block's first key, last first) x (query heads of the group)
   const int qt0 = kb0 / BQ, qt_end = (S + BQ - 1) / BQ;
-  const int n_it = group * (qt_end - qt0);
-  const int64_t h0 = static_cast<int64_t>(kvh) * group;
+  const int n_it = gs * (qt_end - qt0);
+  const int64_t h0 = static_cast<int64_t>(kvh) * group + split * gs;
   const uint16_t* qg = q + tok0 * ldq + h0 * HD;
   const uint16_t* gg = dO + tok0 * lddo + h0 * HD;
   const float* lg = nl2 + (static_cast<int64_t>(b) * nh + h0) * S;
   const float* dg = delta + (static_cast<int64_t>(b) * nh + h0) * S;
   QTileDma<HD, BQ, NT> pre;
   pre.start(qt_end, ldq, lddo, wave, lane);
-  if (n_it > 0) pre.fetch(qg, ldq, gg, lddo, lg, dg, S, qt0, group, st0, st0 + TILE, sl0, sd0, wave, lane);
+  if (n_it > 0) pre.fetch(qg, ldq, gg, lddo, lg, dg, S, qt0, gs, st0, st0 + TILE, sl0, sd0, wave, lane);
   wait_loads();
   __syncthreads();
   int cqt = qt_end - 1, chh = 0;  // query tile and head of the current item
@@ -950,7 +1035,7 @@ __global__ __launch_bounds__(DkdvTiles<HD>::NT) __attribute__((amdgpu_waves_per_
   auto step = [&](int it, const char* T, const float* L, const float* D, char* TN, float* LN, float* DN)
                   __attribute__((always_inline)) {
     refresh_offsets(a_off, b0, b8);
-    if (it + 1 < n_it) pre.fetch(qg, ldq, gg, lddo, lg, dg, S, qt0, group, TN, TN + TILE, LN, DN, wave, lane);
+    if (it + 1 < n_it) pre.fetch(qg, ldq, gg, lddo, lg, dg, S, qt0, gs, TN, TN + TILE, LN, DN, wave, lane);
     const int q0 = cqt * BQ;
     // some query of the tile reaches this sub-tile's keys (same answer for both roles)
     const bool active = it < n_it && kw < S && q0 + BQ - 1 >= kw;
@@ -1017,7 +1102,7 @@ __global__ __launch_bounds__(DkdvTiles<HD>::NT) __attribute__((amdgpu_waves_per_
             acc[dt] = mfma(lds_frag_tr<HD>(Y, b0, b8, 32 * u + 16 * s2, dt), f, acc[dt]);
         }
     }
-    if (++chh == group) {
+    if (++chh == gs) {
       chh = 0;
       --cqt;
     }
@@ -1029,7 +1114,10 @@ __global__ __launch_bounds__(DkdvTiles<HD>::NT) __attribute__((amdgpu_waves_per_
     step(it + 1, st1, sl1, sd1, st0, sl0, sd0);
   }
   if (ki < S) {
-    if (role_a)
+    if (hs.n > 1)
+      store_rows_T_f32<HD>(hs.row(split, role_a ? 1 : 0, static_cast<int64_t>(gridDim.y / (nkv * hs.n)) * S, tok0 + ki,
+                                  nkv, kvh, HD), acc, hl);
+    else if (role_a)
       store_rows_T<HD>(dv + (tok0 + ki) * lddv + static_cast<int64_t>(kvh) * HD, acc, 1.f, hl);
     else
       store_grad_row<HD>(dk + (tok0 + ki) * lddk + static_cast<int64_t>(kvh) * HD, acc, scale, hl, rope, tok0, ki);
@@ -1471,9 +1559,42 @@ int dispatch_hd(int64_t hd, F&& f) {
 
 using namespace fh;
 
+namespace {
+
+// Floats of workspace set aside for the head split's partial sums, known from
+// the size function's arguments alone: up to 256 per (token, query head), which
+// holds any split of heads of 128, at most 32 MB, and only where a model of at
+// most eight query heads per kv head could leave CUs without a workgroup.
+size_t split_floats(int64_t batch, int64_t seq_len, int64_t n_heads) {
+  const int64_t rows = batch * seq_len * n_heads;
+  if (rows > (int64_t(1) << 17) || batch * ((n_heads + 7) / 8) * ((seq_len + 255) / 256) >= 256) return 0;
+  const int64_t floats = 256 * rows, most = int64_t(8) << 20;
+  return static_cast<size_t>(floats < most ? floats : most);
+}
+
+// Where they start in the workspace: after delta and -lse*log2(e), 16-byte aligned.
+size_t split_offset(int64_t batch, int64_t seq_len, int64_t n_heads) {
+  return (2 * static_cast<size_t>(batch * seq_len * n_heads) + 3) / 4 * 4;
+}
+
+// Workgroups that fill the chip: one per CU of the head_dim <= 64 kernel (133 KB
+// of LDS), two of the head_dim-128 kernel.
+constexpr int64_t kDkdvBlocks = 256;
+
+// The smallest split of the group's heads (a divisor of the group) that gives
+// `want` workgroups, or the largest that the workspace holds.
+int head_split(int64_t blocks, int64_t want, int64_t group, int64_t floats_per_split, size_t room) {
+  int64_t n = 1;
+  for (int64_t d = 2; d <= group && blocks * n < want; ++d)
+    if (group % d == 0 && d * floats_per_split <= static_cast<int64_t>(room)) n = d;
+  return static_cast<int>(n);
+}
+
+}  // namespace
+
 extern "C" size_t fh_attn_bwd_workspace_size(int64_t batch, int64_t seq_len, int64_t n_heads) {
   if (batch <= 0 || seq_len <= 0 || n_heads <= 0) return 0;
-  return 2 * static_cast<size_t>(batch * seq_len * n_heads) * sizeof(float);
+  return (split_offset(batch, seq_len, n_heads) + split_floats(batch, seq_len, n_heads)) * sizeof(float);
 }
 
 namespace {
@@ -1610,20 +1731,33 @@ int attn_bwd_impl(fh_dtype dt, const void* q, int64_t ldq, const void* k, int64_
       const auto kg = static_cast<const uint16_t*>(dout);
       const auto kdk = static_cast<uint16_t*>(dk);
       const auto kdv = static_cast<uint16_t*>(dv);
+      // Few workgroups: the group's heads split over several (HeadSplit).
+      const int64_t per_split = 2 * batch * seq_len * n_kv_heads * HD, kvb = batch * n_kv_heads;
+      const size_t room = split_floats(batch, seq_len, n_heads);
+      HeadSplit hs{delta + split_offset(batch, seq_len, n_heads), 1};
       if constexpr (HD <= 64) {
         using DT = DkdvFusedTiles<HD>;
-        const int64_t nkb = (seq_len + DT::NWH * 32 - 1) / (DT::NWH * 32);
-        const dim3 gk(static_cast<unsigned>((nkb + 1) / 2), static_cast<unsigned>(batch * n_kv_heads));
+        const int64_t nkb = (seq_len + DT::NWH * 32 - 1) / (DT::NWH * 32), pairs = (nkb + 1) / 2;
+        hs.n = head_split(pairs * kvb, kDkdvBlocks, group, per_split, room);
+        // One key block per workgroup where all of them still run at once.
+        const bool paired = nkb * kvb * hs.n > kDkdvBlocks;
+        const dim3 gk(static_cast<unsigned>(paired ? pairs : nkb), static_cast<unsigned>(kvb * hs.n));
         hipLaunchKernelGGL((k_attn_bwd_dkdv_fused<HD>), gk, dim3(DT::NT), 0, stream, kq, ldq, kk,
                            ldk, kvp, ldv, kg, lddo, nl2, delta, kdk, lddk, kdv, lddv, S, nh, nkv,
-                           group, scale * kLog2e, scale, rb);
+                           group, scale * kLog2e, scale, rb, hs, paired);
       } else {
         using DT = DkdvTiles<HD>;
         const int64_t nkb = (seq_len + DT::NKS * 32 - 1) / (DT::NKS * 32);
-        const dim3 gk(static_cast<unsigned>(nkb), static_cast<unsigned>(batch * n_kv_heads));
+        hs.n = head_split(nkb * kvb, 2 * kDkdvBlocks, group, per_split, room);
+        const dim3 gk(static_cast<unsigned>(nkb), static_cast<unsigned>(kvb * hs.n));
         hipLaunchKernelGGL((k_attn_bwd_dkdv<HD>), gk, dim3(DT::NT), 0, stream, kq, ldq, kk, ldk,
                            kvp, ldv, kg, lddo, nl2, delta, kdk, lddk, kdv, lddv, S, nh, nkv, group,
-                           scale * kLog2e, scale, rb);
+                           scale * kLog2e, scale, rb, hs);
+      }
+      if (hs.n > 1) {
+        const int64_t tokens = batch * seq_len, threads = tokens * n_kv_heads * (HD / 8);
+        hipLaunchKernelGGL((k_attn_dkdv_sum<HD>), dim3(static_cast<unsigned>((threads + 255) / 256)), dim3(256), 0,
+                           stream, hs, kdk, lddk, kdv, lddv, S, tokens, nkv, scale, rb);
       }
       return 0;
     });

@@ -92,6 +92,23 @@ def test_attention_bf16_matches_closed_form(B, S, nh, nkv, hd):
         assert err <= 2e-2 * float(ref[name].abs().max()) + 1e-3, f"{name}: {err:.3e}"
 
 
+@pytest.mark.parametrize("B,S,nh,nkv,hd", [
+    (1, 33, 3, 1, 64), (1, 61, 5, 1, 128),      # prime groups; partial sums that start at an odd offset
+    (2, 129, 6, 1, 32), (1, 257, 24, 3, 64),    # one and two keys past a key block
+    (1, 1000, 16, 2, 64), (1, 520, 32, 4, 128),  # not every head on its own
+    (5, 700, 32, 4, 64),                        # blocks enough: no split
+])
+def test_attention_bwd_split_over_heads(B, S, nh, nkv, hd):
+    """Few key blocks: dK and dV summed over workgroups that take part of the group's heads each.  The bf16
+    bound of test_attention_bf16_matches_closed_form; two runs bitwise equal."""
+    got, ref = _run(B, S, nh, nkv, hd, torch.bfloat16)
+    again, _ = _run(B, S, nh, nkv, hd, torch.bfloat16)
+    for name in ("dq", "dk", "dv"):
+        assert torch.equal(got[name], again[name])
+        err = float((got[name] - ref[name]).abs().max())
+        assert err <= 2e-2 * float(ref[name].abs().max()) + 1e-3, f"{name}: {err:.3e}"
+
+
 @pytest.mark.parametrize("B,S,nh,nkv,hd", [(2, 128, 8, 4, 32), (1, 77, 4, 2, 64), (1, 40, 2, 1, 128)])
 def test_attention_fp32_matches_closed_form_1e5(B, S, nh, nkv, hd):
     got, ref = _run(B, S, nh, nkv, hd, torch.float32)
