@@ -447,6 +447,51 @@ def gemm(op: str, a: torch.Tensor, b: torch.Tensor, *, residual: torch.Tensor | 
     return c
 
 
+# fh_gemm_f32 takes products of at most this many outputs and k (weight
+# gradients: k of at most 256).  There the library runs some shapes as one tile
+# on one CU (256 x 256 x 688 160 us against 8, 256 x 256 x 512 'nn' 118 against 8)
+# and the others within 1 us of it (5-8 us); above, its choices are sound and its
+# tiles faster (512 x 1376 x 256 7.5 us against 9.9, 2048 x 256 x 688 12 against 14).
+F32_MAX_OUTPUTS = 98304
+F32_MAX_K = {"nt": 768, "nn": 768, "tn": 256}
+
+
+def gemm_f32_supported(op: str, a: torch.Tensor, b: torch.Tensor) -> bool:
+    """Whether a product runs on fh_gemm_f32: fp32 on one HIP device, 2-D with a
+    contiguous last dim, small (above), and where k is an operand's last dim,
+    multiples of 4 and 16-byte aligned rows."""
+    if not (a.is_cuda and b.is_cuda and a.device == b.device and a.dtype == b.dtype == torch.float32):
+        return False
+    dims = gemm_dims(op, a, b)
+    if dims is None:
+        return False
+    m, n, k = dims
+    if min(m, n, k) <= 0 or m * n > F32_MAX_OUTPUTS or k > F32_MAX_K[op]:
+        return False
+    for t, k_last in ((a, op != "tn"), (b, op == "nt")):
+        if t.stride(1) != 1 or t.stride(0) < t.size(1) or (k_last and (k % 4 or t.stride(0) % 4 or t.data_ptr() % 16)):
+            return False
+    return True
+
+
+def gemm_f32(op: str, a: torch.Tensor, b: torch.Tensor, *, residual: torch.Tensor | None = None,
+             out: torch.Tensor | None = None) -> torch.Tensor:
+    """gemm() in fp32 for small products (fh_gemm_f32): op(a) @ op(b), plus
+    `residual`, into `out` (which may be `residual` itself)."""
+    _require_gpu(a, b, residual, out)
+    if not gemm_f32_supported(op, a, b):
+        raise ValueError(f"gemm_f32({op}): unsupported operands {tuple(a.shape)} {a.stride()} x "
+                         f"{tuple(b.shape)} {b.stride()} ({a.dtype}, {b.dtype})")
+    m, n, k = gemm_dims(op, a, b)
+    c = torch.empty(m, n, dtype=a.dtype, device=a.device) if out is None else out
+    for t, name in ((c, "out"), (residual, "residual")):
+        if t is not None and (t.dtype != torch.float32 or tuple(t.shape) != (m, n) or t.stride(1) != 1):
+            raise ValueError(f"gemm_f32({op}): {name} must be an fp32 [{m}, {n}] row-major view")
+    _lib.call("fh_gemm_f32", _GEMM_OPS[op], _ptr(a), a.stride(0), _ptr(b), b.stride(0), _ptr(c), c.stride(0),
+              _ptr(residual), 0 if residual is None else residual.stride(0), m, n, k, _stream(a))
+    return c
+
+
 def gemm_grouped(op: str, items: list, *, any_k: bool = False) -> list:
     """Up to three GEMMs of layout `op` with one k in one fh_gemm_bf16_grouped
     call: each item is (a, b, residual, out) with gemm()'s meaning (residual

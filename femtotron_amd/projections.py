@@ -34,8 +34,9 @@ GEMM (``torch.mm`` on hipBLASLt/rocBLAS), by policy:
 * ``"library"``: always the library.
 
 k need not be a multiple of 64 (fh_gemm_bf16_any_k: a weight gradient's k is the
-token count of a batch, of any length).  Operands the kernel does not take
-(fp32, k below 64, ...) go to the library under every policy.  ``gemm_dispatch_counts()`` tells tests and
+token count of a batch, of any length).  Small fp32 products run on fh_gemm_f32
+(ops.gemm_f32_supported).  Operands the kernels do not take (larger fp32 ones,
+k below 64, ...) go to the library under every policy.  ``gemm_dispatch_counts()`` tells tests and
 the benchmark which path ran.
 """
 from __future__ import annotations
@@ -104,6 +105,11 @@ def _choose_hand(op: str, a: torch.Tensor, b: torch.Tensor, table: str | None = 
     return use
 
 
+def _small_f32(op: str, a: torch.Tensor, b: torch.Tensor) -> bool:
+    """Whether an fp32 product runs on fh_gemm_f32 (counted as hand-written)."""
+    return a.dtype == torch.float32 and _policy[0] != "library" and ops.gemm_f32_supported(op, a, b) and _count(True)
+
+
 def _count(hand: bool) -> bool:
     """Count one GEMM as hand-written or library; returns `hand`."""
     with _lock:
@@ -117,6 +123,8 @@ def _use_hand(op: str, a: torch.Tensor, b: torch.Tensor) -> bool:
 
 def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """x [T, in] @ w[out, in]^T."""
+    if _small_f32("nt", x, w):
+        return ops.gemm_f32("nt", x, w)
     if _use_hand("nt", x, w):
         return ops.gemm("nt", x, w, any_k=True)
     return torch.mm(x, w.t())
@@ -139,6 +147,8 @@ def linear_residual(x: torch.Tensor, w: torch.Tensor, residual: torch.Tensor) ->
     """residual + to_dtype(x @ w^T), written into `residual`'s memory (the
     hand-written GEMM's residual epilogue; otherwise the library GEMM followed
     by fh_add into `residual`)."""
+    if residual.is_contiguous() and _small_f32("nt", x, w):
+        return ops.gemm_f32("nt", x, w, residual=residual, out=residual)
     if _count(residual.is_contiguous() and _choose_hand("nt", x, w, "nt_res")):
         return ops.gemm("nt", x, w, residual=residual, out=residual, any_k=True)
     m = torch.mm(x, w.t())
@@ -149,6 +159,8 @@ def linear_residual(x: torch.Tensor, w: torch.Tensor, residual: torch.Tensor) ->
 
 def linear_dgrad(dy: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """dy [T, out] @ w [out, in]."""
+    if _small_f32("nn", dy, w):
+        return ops.gemm_f32("nn", dy, w)
     if _use_hand("nn", dy, w):
         return ops.gemm("nn", dy, w, any_k=True)
     return torch.mm(dy, w)
@@ -156,6 +168,8 @@ def linear_dgrad(dy: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
 
 def linear_wgrad(dy: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
     """dy [T, out]^T @ x [T, in]: the [out, in] weight gradient."""
+    if _small_f32("tn", dy, x):
+        return ops.gemm_f32("tn", dy, x)
     if _use_hand("tn", dy, x):
         return ops.gemm("tn", dy, x, any_k=True)
     return torch.mm(dy.t(), x)

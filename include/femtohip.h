@@ -430,6 +430,14 @@ size_t fh_gemm_bf16_grouped_any_k_workspace_size(int op, int count, const fh_gem
 int fh_gemm_bf16_grouped_any_k(int op, int count, const fh_gemm_problem* problems, int64_t k, void* workspace,
                                hipStream_t stream);
 
+/* The same three products in fp32 (fp32 models), C = A B (+ residual, which may
+ * be C itself): fp32 products and sums in a fixed order.  For small products:
+ * one workgroup per 32 x 32 outputs, operands read through the caches.  Where k
+ * is an operand's contiguous index: k and its leading dimension multiples of 4,
+ * 16-byte aligned.  m < 2^20, n < 2^24. */
+int fh_gemm_f32(int op, const void* a, int64_t lda, const void* b, int64_t ldb, void* c, int64_t ldc,
+                const void* residual, int64_t ldr, int64_t m, int64_t n, int64_t k, hipStream_t stream);
+
 /* The q/k/v projection with the rotary embedding in its epilogue: C = A B^T
  * (FH_GEMM_NT, no residual) and then, on columns [0, rot_cols) of C (the q and
  * k heads of head_dim columns each), the rotation of fh_rope_fwd -- bit for

@@ -290,6 +290,32 @@ def test_mid_tiles_match_and_add_the_residual(op, m, n, k, pad):
     assert torch.equal(ops.gemm(op, a, b, residual=r, out=r), want)
 
 
+@pytest.mark.parametrize("op", ["nt", "nn", "tn"])
+@pytest.mark.parametrize("m,n,k", [(256, 256, 256), (1, 8, 4), (33, 40, 20), (31, 72, 132), (256, 264, 688),
+                                   (300, 256, 64), (8, 520, 248)])
+def test_small_f32_product(op, m, n, k):
+    """fh_gemm_f32 at tile, chunk and wave edges (k of the weight gradient odd too), operands followed by NaNs:
+    within k * 2^-24 of the sum of absolute products of the fp64 result; the residual added to the fp32 result."""
+    for kk in ((min(k, 256), min(k, 256) - 1) if op == "tn" else (k,)):
+        g = torch.Generator(device=DEV).manual_seed(m + n + kk)
+        shapes = {"nt": ((m, kk), (n, kk)), "nn": ((m, kk), (kk, n)), "tn": ((kk, m), (kk, n))}[op]
+        ops_ = []
+        for rows, cols in shapes:
+            buf = torch.full((rows + 40, cols + 40 + (-cols) % 4), float("nan"), device=DEV)
+            buf[:rows, :cols] = torch.randn(rows, cols, device=DEV, generator=g)
+            ops_.append(buf[:rows, :cols])
+        a, b = ops_
+        assert ops.gemm_f32_supported(op, a, b)
+        c = ops.gemm_f32(op, a, b)
+        ref, absref = _ref(op, a, b, torch.float64)
+        assert bool(((c.double() - ref).abs() <= (kk + 2) * 2.0 ** -24 * absref).all())
+        r = torch.randn(m, n, device=DEV, generator=g)
+        want = r + c
+        assert torch.equal(ops.gemm_f32(op, a, b, residual=r, out=r), want)
+    with pytest.raises(ValueError):
+        ops.gemm_f32(op, a.to(BF), b.to(BF))
+
+
 def _guarded(rows, cols, g):
     """A [rows, cols] operand inside a larger NaN-filled buffer: what a read past it would meet."""
     buf = torch.full((rows + 64, cols + 64), float("nan"), device=DEV, dtype=BF)
