@@ -40,6 +40,16 @@ class FhGemmProblem(ctypes.Structure):
                 ("residual", _V), ("ldr", _I64), ("m", _I64), ("n", _I64)]
 
 
+class FhLayer(ctypes.Structure):
+    """fh_layer of include/femtohip.h."""
+    _fields_ = [("dt", c_int), ("cos_per_token", ctypes.c_int32), ("batch", _I64), ("seq_len", _I64),
+                ("hidden", _I64), ("n_heads", _I64), ("n_kv_heads", _I64), ("head_dim", _I64), ("ffn", _I64),
+                ("eps1", _F), ("eps2", _F), ("scale", _F), ("reserved", _F), ("cos", _V), ("sin", _V),
+                ("wqkv", _V), ("wo", _V), ("wgu", _V), ("wd", _V), ("w1", _V), ("w2", _V)]
+
+
+FH_LAYER_DWQKV, FH_LAYER_DWO, FH_LAYER_DWGU, FH_LAYER_DWD = 1, 2, 4, 8
+
 # name -> (restype, argtypes); mirrors include/femtohip.h exactly.
 SIGNATURES: dict[str, tuple] = {
     "fh_abi_version": (c_int, []),
@@ -83,6 +93,9 @@ SIGNATURES: dict[str, tuple] = {
     "fh_embedding_fwd": (c_int, [c_int, _V, _V, _V, _I64, _I64, _I64, _V]),
     "fh_embedding_bwd_workspace_size": (c_size_t, [_I64, _I64]),
     "fh_embedding_bwd": (c_int, [c_int, _V, _V, _V, _I64, _I64, _I64, _I64, _V, _V]),
+    "fh_layer_workspace_size": (c_size_t, [POINTER(FhLayer), c_int]),
+    "fh_layer_fwd": (c_int, [POINTER(FhLayer), _V, _V, _V, _V]),
+    "fh_layer_bwd": (c_int, [POINTER(FhLayer), _V, _V, _V, _V, _V, _V, _V, _V, _V, c_int, _V, _V]),
     "fh_adamw_step": (c_int, [c_int, _V, _V, c_int, _I64, FhAdamHyper, _F, _V, _V]),
 }
 

@@ -36,9 +36,9 @@ from dataclasses import dataclass
 
 import torch
 
-from . import ops
-from .projections import (linear, linear_dgrad, linear_residual, linear_rope, linear_wgrad, linear_wgrad_group,
-                          linear_wgrad_into)
+from . import _lib, ops
+from .projections import (count_hand, gemm_policy, linear, linear_dgrad, linear_residual, linear_rope, linear_wgrad,
+                          linear_wgrad_group, linear_wgrad_into)
 from .weight_packing import packed
 
 
@@ -323,6 +323,76 @@ def layer_backward(dout2: torch.Tensor, x2: torch.Tensor, cos: torch.Tensor, sin
     return dx, (dwq, dwk, dwv, dwo, dwg, dwu, dwd, dw1, dw2)
 
 
+# The layer as one call per direction (fh_layer_fwd / fh_layer_bwd): while its
+# intermediates are small its kernels end before Python has issued the next ones.
+# Forward and backward op by op and in one call each, wall time, bf16: 688 and 377
+# us (2048 wide, ffn 8192, 256 tokens), 722 and 716 (1000 tokens), 647 and 318 (256
+# wide, 256 tokens), 642 and 457 (1024 wide, 2048 tokens).  Past this workspace
+# the kernels are the time (2048 wide at 1000 tokens, 231 MiB: level already), and
+# op by op an intermediate's memory is reused once it is read.
+ONE_CALL_MAX_BYTES = 256 << 20
+# fp32: every product runs on fh_gemm_f32, which is made for small ones: 630 and
+# 206 us (256 wide, ffn 688, 256 tokens), 683 and 304 (1024 tokens), 834 and 716 at
+# the largest of these sizes; beyond, the library's larger tiles are faster.
+ONE_CALL_F32_HIDDEN, ONE_CALL_F32_FFN, ONE_CALL_F32_TOKENS = 512, 2048, 1024
+
+
+def _one_call(x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, shp: LayerShape, w: tuple,
+              dout: torch.Tensor | None = None):
+    """(argument block, workspace bytes, the tensors it points into) if the
+    layer's forward (or, given dout, its recompute and backward) runs as one
+    call, else None.  It runs what the default settings run: the hand-written
+    GEMMs, weight gradients in order on the current stream."""
+    B, S, H = x.shape
+    T = B * S
+    if gemm_policy() != "hand" or _use_side_stream or T == 0:
+        return None
+    if x.dtype == torch.bfloat16:
+        # 64: the least k of the GEMMs (k = T in the weight gradients)
+        if min(T, H, shp.ffn, shp.hq) < 64 or H % 8 or shp.ffn % 8:
+            return None
+    elif H > ONE_CALL_F32_HIDDEN or shp.ffn > ONE_CALL_F32_FFN or T > ONE_CALL_F32_TOKENS or H % 4 or shp.ffn % 4:
+        return None
+    # The intermediates alone (no products' workspace): skip the rest where they are too large.
+    if T * (4 * H + 3 * shp.ffn) * x.element_size() > ONE_CALL_MAX_BYTES:
+        return None
+    if dout is not None and (dout.dtype != x.dtype or dout.device != x.device or dout.shape != x.shape
+                             or dout.data_ptr() % 16):
+        return None
+    wq, wk, wv, wo, wg, wu, wd, w1, w2 = w
+    call = ops.layer_args(B, S, shp, x, cos, sin, _cat_rows(wq, wk, wv), wo, _cat_rows(wg, wu), wd, w1, w2)
+    if call is None:
+        return None
+    nbytes = ops.layer_workspace_size(call[0], dout is not None)
+    if nbytes == 0 or nbytes > ONE_CALL_MAX_BYTES:
+        return None
+    return call[0], nbytes, call[1]
+
+
+def _one_call_backward(call, x: torch.Tensor, dout: torch.Tensor, shp: LayerShape, w: tuple):
+    """layer_backward's results from fh_layer_bwd."""
+    args, nbytes, _alive = call
+    wq, wk, wv, wo, wg, wu, wd, w1, w2 = w
+    grads, accumulate = [], 0
+    for bit, group, rows, cols in ((_lib.FH_LAYER_DWQKV, (wq, wk, wv), shp.hq + 2 * shp.hkv, shp.hidden),
+                                   (_lib.FH_LAYER_DWO, (wo,), shp.hidden, shp.hq),
+                                   (_lib.FH_LAYER_DWGU, (wg, wu), 2 * shp.ffn, shp.hidden),
+                                   (_lib.FH_LAYER_DWD, (wd,), shp.hidden, shp.ffn)):
+        g = grad_target(*group)
+        if g is not None and g.data_ptr() % 16 == 0:
+            accumulate |= bit
+        else:
+            g = torch.empty(rows, cols, dtype=x.dtype, device=x.device)
+        grads.append(g)
+    grads += [torch.empty_like(w1), torch.empty_like(w2)]
+    dx = ops.layer_bwd(args, nbytes, x, dout, grads, accumulate)
+    count_hand(11)
+    dwqkv, dwo, dwgu, dwd, dw1, dw2 = (None if accumulate & (1 << i) and i < 4 else g for i, g in enumerate(grads))
+    dwq, dwk, dwv = split_rows(dwqkv, shp.hq, shp.hkv, shp.hkv)
+    dwg, dwu = split_rows(dwgu, shp.ffn, shp.ffn)
+    return dx, (dwq, dwk, dwv, dwo, dwg, dwu, dwd, dw1, dw2)
+
+
 class FusedDecoderLayerFunction(torch.autograd.Function):
     """autograd node for one checkpointed decoder layer.
 
@@ -334,7 +404,12 @@ class FusedDecoderLayerFunction(torch.autograd.Function):
     def forward(ctx, x, cos, sin, shp, wq, wk, wv, wo, wg, wu, wd, w1, w2):
         B, S, H = x.shape
         w = (wq, wk, wv, wo, wg, wu, wd, w1, w2)
-        out = layer_forward(x.reshape(B * S, H), cos, sin, shp, B, S, w, keep=False)
+        call = _one_call(x, cos, sin, shp, w)
+        if call is not None:
+            out = ops.layer_fwd(call[0], call[1], x)
+            count_hand(4)
+        else:
+            out = layer_forward(x.reshape(B * S, H), cos, sin, shp, B, S, w, keep=False)
         ctx.save_for_backward(x, cos, sin, *w)
         ctx.shp = shp
         return out.view(B, S, H)
@@ -344,9 +419,13 @@ class FusedDecoderLayerFunction(torch.autograd.Function):
         x, cos, sin, *w = ctx.saved_tensors
         shp = ctx.shp
         B, S, H = x.shape
-        x2 = x.reshape(B * S, H)
+        dout = dout.contiguous()
         with torch.no_grad():
-            acts = layer_forward(x2, cos, sin, shp, B, S, tuple(w), keep=True)
-            dx, dws = layer_backward(dout.contiguous().view(B * S, H), x2, cos, sin, shp, B, S,
-                                     tuple(w), acts)
+            call = _one_call(x, cos, sin, shp, tuple(w), dout)
+            if call is not None:
+                dx, dws = _one_call_backward(call, x, dout, shp, tuple(w))
+            else:
+                x2 = x.reshape(B * S, H)
+                acts = layer_forward(x2, cos, sin, shp, B, S, tuple(w), keep=True)
+                dx, dws = layer_backward(dout.view(B * S, H), x2, cos, sin, shp, B, S, tuple(w), acts)
         return (dx.view(B, S, H), None, None, None, *dws)

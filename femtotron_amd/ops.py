@@ -51,7 +51,9 @@ def _rowmajor(t: torch.Tensor, name: str) -> int:
 
 
 def _stream(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    """The current stream of t's device (the raw handle: building a
+    torch.cuda.Stream object costs more than the launch's other host work)."""
+    return torch._C._cuda_getCurrentRawStream(t.device.index)
 
 
 def _ptr(t: torch.Tensor | None):
@@ -365,6 +367,52 @@ def embedding_bwd(dy: torch.Tensor, ids: torch.Tensor, vocab: int,
     _lib.call("fh_embedding_bwd", _dtype_code(dy), _ptr(dy), _ptr(ids), _ptr(dw), n, vocab, hidden,
               -1 if padding_idx is None else int(padding_idx), _ptr(ws), _stream(dy))
     return dw
+
+
+# ------------------------------------------------------------- decoder layer
+def layer_args(batch: int, seq_len: int, shp, x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, *ws: torch.Tensor):
+    """(fh_layer argument block, the tensors it points into) of a layer of shape
+    `shp` (fused_layer.LayerShape) and weights wqkv, wo, wgu, wd, w1, w2; None
+    where an operand is not what the layer calls take: x's device and dtype,
+    contiguous, 16-byte aligned, of the shape's sizes.  The block holds raw
+    pointers: the caller keeps the tensors alive and uses it at once."""
+    H, hq, F_ = shp.hidden, shp.hq, shp.ffn
+    sizes = ((hq + 2 * shp.hkv, H), (H, hq), (2 * F_, H), (H, F_), (H,), (H,))
+    dt, dev = x.dtype, x.device
+    for w, size in zip(ws, sizes):
+        if w.dtype != dt or w.device != dev or w.shape != size or not w.is_contiguous() or w.data_ptr() % 16:
+            return None
+    if not x.is_cuda or dt not in _DT or not x.is_contiguous() or x.data_ptr() % 16:
+        return None
+    if not cos.dtype == sin.dtype == dt or not cos.device == sin.device == dev:
+        return None
+    cos2, sin2, per_token = _rope_tables("layer", cos, sin, shp.head_dim, seq_len, batch * seq_len)
+    args = _lib.FhLayer(_DT[dt], per_token, batch, seq_len, H, shp.n_heads, shp.n_kv_heads, shp.head_dim, F_,
+                        shp.eps1, shp.eps2, shp.scale, 0.0, cos2.data_ptr(), sin2.data_ptr(),
+                        *(w.data_ptr() for w in ws))
+    return args, (cos2, sin2, *ws)
+
+
+def layer_workspace_size(args: _lib.FhLayer, backward: bool) -> int:
+    return _lib.lib().fh_layer_workspace_size(ctypes.byref(args), int(backward))
+
+
+def layer_fwd(args: _lib.FhLayer, nbytes: int, x: torch.Tensor) -> torch.Tensor:
+    """fh_layer_fwd on the x of layer_args, with a workspace of nbytes."""
+    out = torch.empty_like(x)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
+    _lib.call("fh_layer_fwd", ctypes.byref(args), x.data_ptr(), out.data_ptr(), ws.data_ptr(), _stream(x))
+    return out
+
+
+def layer_bwd(args: _lib.FhLayer, nbytes: int, x: torch.Tensor, dout: torch.Tensor, grads: list,
+              accumulate: int) -> torch.Tensor:
+    """fh_layer_bwd on contiguous, 16-byte aligned x and dout; grads: the dwqkv, dwo, dwgu, dwd, dw1, dw2 buffers.  Returns dx."""
+    dx = torch.empty_like(x)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
+    _lib.call("fh_layer_bwd", ctypes.byref(args), x.data_ptr(), dout.data_ptr(), dx.data_ptr(),
+              *(g.data_ptr() for g in grads), accumulate, ws.data_ptr(), _stream(x))
+    return dx
 
 
 # ------------------------------------------------------------- GEMM

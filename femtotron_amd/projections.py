@@ -117,6 +117,12 @@ def _count(hand: bool) -> bool:
     return hand
 
 
+def count_hand(n: int) -> None:
+    """Count n GEMMs that a one-call layer (fh_layer_fwd / fh_layer_bwd) ran hand-written."""
+    with _lock:
+        _counts["hand"] += n
+
+
 def _use_hand(op: str, a: torch.Tensor, b: torch.Tensor) -> bool:
     return _count(_choose_hand(op, a, b))
 

@@ -454,6 +454,44 @@ int fh_gemm_bf16_rope(const void* a, int64_t lda, const void* b, int64_t ldb, vo
                       int64_t head_dim, int64_t seq_len, const void* cos, const void* sin,
                       int cos_per_token, hipStream_t stream);
 
+/* ------------------------------------------------------------------------
+ * One activation-checkpointed decoder layer (modeling_llama.py:284-325) in one
+ * call per direction: the launches of the entry points above, in the order of
+ * femtotron_amd/fused_layer.py, for batches whose kernels are shorter than a
+ * Python host needs to issue them.  FH_F32 products run on fh_gemm_f32 (small
+ * layers).  All weights row-major and packed: wqkv [q; k; v rows, hidden], wgu
+ * [gate; up rows, hidden].  cos/sin as in fh_rope_fwd.  Requirements of the
+ * entry points apply (FH_BF16: batch * seq_len >= 64).
+ *   fwd: out = layer(x); x, out [batch * seq_len, hidden].
+ *   bwd: recomputes the forward from x, then dx and the weight gradients for
+ *        dout.  `accumulate`: FH_LAYER_* bits of the bf16 gradients to add into
+ *        (their buffers hold the gradients so far, fh_gemm_bf16's residual == C);
+ *        the others are overwritten.
+ * workspace: fh_layer_workspace_size bytes (backward: 0 or 1), 16-byte aligned.
+ */
+typedef struct fh_layer {
+  fh_dtype dt;
+  int32_t cos_per_token;
+  int64_t batch, seq_len, hidden, n_heads, n_kv_heads, head_dim, ffn;
+  float eps1, eps2, scale, reserved;
+  const void* cos;
+  const void* sin;
+  const void* wqkv;
+  const void* wo;
+  const void* wgu;
+  const void* wd;
+  const void* w1;
+  const void* w2;
+} fh_layer;
+
+enum { FH_LAYER_DWQKV = 1, FH_LAYER_DWO = 2, FH_LAYER_DWGU = 4, FH_LAYER_DWD = 8 };
+
+size_t fh_layer_workspace_size(const fh_layer* layer, int backward);
+int fh_layer_fwd(const fh_layer* layer, const void* x, void* out, void* workspace, hipStream_t stream);
+int fh_layer_bwd(const fh_layer* layer, const void* x, const void* dout, void* dx, void* dwqkv, void* dwo,
+                 void* dwgu, void* dwd, void* dw1, void* dw2, int accumulate, void* workspace,
+                 hipStream_t stream);
+
 #ifdef __cplusplus
 }  /* extern "C" */
 #endif
