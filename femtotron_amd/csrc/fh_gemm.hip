@@ -79,7 +79,7 @@ namespace {
 constexpr int kTm = 256, kTn = 256, kTk = 64;  // block tile and stage depth
 constexpr int kSubBytes = kTk * 128;           // KO sub-tile: [64 k x 64] bf16
 
-enum Epi { EPI_STORE = 0, EPI_RESIDUAL = 1, EPI_PARTIAL = 2, EPI_ROPE = 3, EPI_STREAM = 4, EPI_GROUP = 5 };
+enum Epi { EPI_STORE = 0, EPI_RESIDUAL = 1, EPI_PARTIAL = 2, EPI_ROPE = 3, EPI_STREAM = 4, EPI_GROUP = 5, EPI_ACC = 6 };
 
 // The rotary embedding of EPI_ROPE: columns [0, rot_cols) of C are heads of
 // hd columns (hd a power of two dividing the 256-column tile, so no head
@@ -110,7 +110,8 @@ struct GemmArgs {
   const uint16_t* b;
   uint16_t* c;
   const uint16_t* r;  // residual (EPI_RESIDUAL)
-  float* part;        // fp32 slice partials (EPI_PARTIAL)
+  float* part;        // fp32 slice partials (EPI_PARTIAL); the running fp32 sum (EPI_ACC)
+  int add;            // EPI_ACC: part holds the sum so far
   int64_t lda, ldb, ldc, ldr;
   int m, n;
   int tiles_m, tiles_n, tiles;
@@ -339,7 +340,8 @@ __device__ __forceinline__ GemmArgs for_tile(const GemmArgs& g, int& t) {
 
 // One tile t over k-steps s_begin .. s_begin + nst - 1.  The result goes to C
 // (bf16, with the EPI epilogue) or, for EPI_PARTIAL and for EPI_STREAM with
-// to_part, as fp32 to pdst (the tile's origin, row stride pld).  EPI_STREAM
+// to_part, as fp32 to pdst (the tile's origin, row stride pld).  EPI_ACC: the
+// fp32 sum of the product and, with g.add, of pdst, to pdst or rounded to C.  EPI_STREAM
 // ends with a barrier, as the workgroup's next tile reuses the LDS ring.
 // RAGGED: k may be no multiple of 64.
 template <bool A_KO, bool B_KO, int EPI, bool RAGGED, int W>
@@ -491,7 +493,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, char* ring, int t, 
   wait_lds();
   bar();
 
-  if (EPI == EPI_PARTIAL || (EPI == EPI_STREAM && to_part)) {
+  if (EPI == EPI_PARTIAL || EPI == EPI_ACC || (EPI == EPI_STREAM && to_part)) {
     // The fp32 tile goes through LDS in two halves of W rows ([W rows x 2 W
     // columns], 16-byte chunk c of row r stored at chunk c ^ (r % 16)); the
     // lanes of a wave then store the chunks of 128 / W whole rows.
@@ -516,6 +518,36 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, char* ring, int t, 
       wait_lds();
       bar();
       const int chunk = lane % CH, col = n0 + 4 * chunk;
+      if constexpr (EPI == EPI_ACC) {
+        // The sum so far is read 16 rows at a time, all in flight together.
+        constexpr int NB = 16;
+#pragma unroll 1
+        for (int q0 = 0; q0 < W / 4 / RI; q0 += NB) {
+          const int r0 = W / 4 * wave + RI * q0 + lane / CH;
+          float4 old[NB];
+#pragma unroll
+          for (int u = 0; u < NB; ++u) {
+            const int r = r0 + RI * u;
+            old[u] = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (g.add && m0 + W * half + r < g.m && col < g.n)
+              old[u] = *reinterpret_cast<const float4*>(pdst + static_cast<int64_t>(W * half + r) * pld + 4 * chunk);
+          }
+#pragma unroll
+          for (int u = 0; u < NB; ++u) {
+            const int r = r0 + RI * u, mrow = m0 + W * half + r;
+            const float4 v = *reinterpret_cast<const float4*>(ring + r * RB + ((chunk ^ (r & 15)) << 4));
+            const float4 o = make_float4(old[u].x + v.x, old[u].y + v.y, old[u].z + v.z, old[u].w + v.w);
+            if (mrow >= g.m || col >= g.n) continue;
+            if (g.c != nullptr)
+              *reinterpret_cast<uint2*>(g.c + mrow * g.ldc + col) = make_uint2(pk_bf16(o.x, o.y), pk_bf16(o.z, o.w));
+            else
+              *reinterpret_cast<float4*>(pdst + static_cast<int64_t>(W * half + r) * pld + 4 * chunk) = o;
+          }
+        }
+        wait_lds();
+        bar();
+        continue;
+      }
 #pragma unroll 4
       for (int q2 = 0; q2 < W / 4 / RI; ++q2) {
         const int r = W / 4 * wave + RI * q2 + lane / CH;
@@ -867,7 +899,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     const int s_begin = slice * g.steps_per_slice;
     int m0, n0;
     tile_origin(g, t, m0, n0);
-    float* pdst = EPI == EPI_PARTIAL
+    float* pdst = EPI == EPI_PARTIAL || EPI == EPI_ACC
                       ? g.part + static_cast<int64_t>(slice) * g.m * g.n + static_cast<int64_t>(m0) * g.n + n0
                       : nullptr;
     gemm_tile<A_KO, B_KO, EPI, RAGGED, 128>(g, ring, t, s_begin, min(g.total_steps - s_begin, g.steps_per_slice), pdst,
@@ -1506,6 +1538,26 @@ extern "C" size_t fh_gemm_bf16_grouped_any_k_workspace_size(int op, int count, c
 extern "C" int fh_gemm_bf16_grouped_any_k(int op, int count, const fh_gemm_problem* problems, int64_t k,
                                           void* workspace, hipStream_t stream) {
   return group_impl(op, count, problems, k, true, workspace, stream);
+}
+
+// A 32000 x 2048 weight gradient of 4096 tokens into a running 262 MB sum: 575 us as
+// a library product with beta = 1, 481 here (446 without a sum to add, 470 rounding
+// it into C; the plain bf16 product 394).  The sum's traffic is not hidden: it runs
+// at the end of a tile, one workgroup per CU.
+extern "C" int fh_gemm_bf16_acc(const void* a, int64_t lda, const void* b, int64_t ldb, float* acc, int add, void* c,
+                                int64_t ldc, int64_t m, int64_t n, int64_t k, hipStream_t stream) {
+  GemmArgs g;
+  if (int e = gemm_setup(FH_GEMM_TN, a, lda, b, ldb, c ? c : acc, c ? ldc : n, nullptr, 0, m, n, k, true, g)) return e;
+  FH_REQUIRE(acc && aligned16(acc), "gemm_bf16_acc: acc must be 16-byte aligned");
+  g.c = static_cast<uint16_t*>(c);
+  g.part = acc;
+  g.add = add != 0;
+  g.steps_per_slice = g.total_steps;
+  g.grid = g.tiles;
+  const dim3 grid((static_cast<unsigned>(g.tiles) + 7) / 8 * 8), block(256);
+  if (g.repeat > 0) hipLaunchKernelGGL((k_gemm<true, true, EPI_ACC, true>), grid, block, 0, stream, g);
+  else hipLaunchKernelGGL((k_gemm<true, true, EPI_ACC, false>), grid, block, 0, stream, g);
+  return check_launch("fh_gemm_bf16_acc");
 }
 
 extern "C" int fh_gemm_bf16_rope(const void* a, int64_t lda, const void* b, int64_t ldb, void* c, int64_t ldc,

@@ -9,13 +9,13 @@ Reference loss head (femtotron/model/llama.py:91-111, femtotron/model/base.py:20
 It materialises the logits in the model dtype and twice more in fp32 (the
 ``.float()`` copy and the log-softmax), ~0.38 MB per token at V = 32000, which
 is the largest activation term of a checkpointed step.  Here the rows are
-processed in chunks of at most ~256 MB of logits: per chunk one library GEMM
+processed in chunks of at most 1 GiB of logits: per chunk one GEMM
 forms the logits, ``fh_ce_fwd_bwd`` computes the fp32 row losses and overwrites
 the chunk with its gradient (softmax - onehot) / n_valid in the model dtype (the
 rounding point of the reference's ``.float()`` backward), and two GEMMs turn it
 into the chunk's input gradient (dlogits @ W, in the model dtype like the
 reference) and its weight-gradient contribution (dlogits^T @ hidden,
-accumulated across chunks in fp32 and rounded once).  Both gradients are
+accumulated in fp32, across chunks too, and rounded once).  Both gradients are
 computed in the forward and scaled by the incoming gradient in the backward, so
 nothing of size [tokens, V] outlives a chunk.
 
@@ -29,9 +29,22 @@ from __future__ import annotations
 import torch
 
 from . import ops
+from .projections import _choose_hand
 
 IGNORE_INDEX = -100
-CHUNK_BYTES = 256 << 20  # logits bytes per chunk
+# Logits bytes per chunk.  Each chunk past the first reads and each before the
+# last writes the fp32 sum of the weight gradient (8 bytes per weight: a third to
+# half of that product's own time at 256 MB of a 32000- or 128256-token vocabulary),
+# and a single chunk needs no sum, which at 4 bytes per weight is itself the
+# larger part of the head's memory for a large vocabulary.  Forward and backward
+# in chunks of 256 MB, 512 MB and 1 GB: 16384 x 2048 hidden states and a vocabulary of
+# 32000 5582, 5219 and 5023 us with a peak of 766, 751 and 1001 MB; 8192 x 4096 and
+# 128256 27.7, 23.0 and 20.4 ms, 3320, 2505 and 3006 MB.
+CHUNK_BYTES = 1 << 30
+# The logits run hand-written up to this width, where a tile is few stages long:
+# 16384 x 32000 352 us against the library's 426 at 256 wide, 508 against 613 at
+# 512, 848 against 842 at 1024, and 1544 against 1497 at 2048.
+LOGITS_HAND_MAX_HIDDEN = 1024
 
 
 def shift_labels(labels: torch.Tensor, ignore_index: int = IGNORE_INDEX) -> torch.Tensor:
@@ -50,6 +63,43 @@ def supported(hidden: torch.Tensor, weight: torch.Tensor) -> bool:
             and weight.shape[0] % 8 == 0 and not torch.is_autocast_enabled())
 
 
+def _logits(x_c: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
+    if x_c.size(1) <= LOGITS_HAND_MAX_HIDDEN and _choose_hand("nt", x_c, weight):
+        return ops.gemm("nt", x_c, weight, any_k=True)
+    return torch.mm(x_c, weight.t())
+
+
+def _input_grad(dlogits: torch.Tensor, weight: torch.Tensor, out: torch.Tensor) -> None:
+    """out = dlogits @ weight.  Hand-written where supported: 4096 x 2048 x 32000 392
+    us against the library's 439, 1024 x 2048 x 32000 119 against 298."""
+    if _choose_hand("nn", dlogits, weight) and out.is_contiguous() and out.data_ptr() % 16 == 0:
+        ops.gemm("nn", dlogits, weight, out=out, any_k=True)
+    else:
+        torch.mm(dlogits, weight, out=out)
+
+
+def _weight_grad(dlogits: torch.Tensor, x_c: torch.Tensor, dw32: torch.Tensor | None, first: bool, last: bool):
+    """(dw or None, the running fp32 sum or None) after this chunk: dw appears
+    with the last one.  A chunk that does not run hand-written (fp32, a width that is
+    no multiple of 8, fewer than 64 rows) leaves the rounding to the caller."""
+    V, H = dlogits.size(1), x_c.size(1)
+    if _choose_hand("tn", dlogits, x_c):
+        if first and last:
+            return ops.gemm("tn", dlogits, x_c, any_k=True), None
+        dw = torch.empty(V, H, dtype=x_c.dtype, device=x_c.device) if last else None
+        if first:
+            dw32 = torch.empty(V, H, dtype=torch.float32, device=x_c.device)
+        ops.gemm_acc(dlogits, x_c, dw32, add=not first, out=dw)
+        return dw, dw32
+    if first:
+        dw32 = torch.zeros(V, H, dtype=torch.float32, device=x_c.device)
+    if x_c.dtype == torch.float32:
+        dw32.addmm_(dlogits.t(), x_c)
+    else:
+        torch.addmm(dw32, dlogits.t(), x_c, out_dtype=torch.float32, out=dw32)
+    return None, dw32
+
+
 class FusedLinearCrossEntropy(torch.autograd.Function):
     """loss = mean over non-ignored rows of CE(hidden2 @ weight^T, targets).
     Saved for backward: the input gradient [N, H] and the weight gradient."""
@@ -63,24 +113,23 @@ class FusedLinearCrossEntropy(torch.autograd.Function):
         inv_count = (1.0 / n_valid).reshape(1)  # inf when nothing is valid -> NaN loss, as torch
         need_dx, need_dw = ctx.needs_input_grad[0], ctx.needs_input_grad[1]
         dx = torch.empty_like(hidden2) if need_dx else None
-        dw32 = torch.zeros(V, H, dtype=torch.float32, device=dev) if need_dw else None
+        dw = dw32 = None
         loss_sum = torch.zeros((), dtype=torch.float32, device=dev)
         chunk = max(256, (CHUNK_BYTES // (V * hidden2.element_size())) // 256 * 256)
         for r0 in range(0, N, chunk):
             r1 = min(N, r0 + chunk)
             x_c = hidden2[r0:r1]
-            logits = torch.mm(x_c, weight.t())
+            logits = _logits(x_c, weight)
             loss_rows = ops.ce_fwd_bwd_(logits, targets[r0:r1], inv_count, IGNORE_INDEX)
             loss_sum += loss_rows.sum()
             if need_dx:
-                torch.mm(logits, weight, out=dx[r0:r1])
+                _input_grad(logits, weight, dx[r0:r1])
             if need_dw:
-                if hidden2.dtype == torch.float32:
-                    dw32.addmm_(logits.t(), x_c)
-                else:
-                    torch.addmm(dw32, logits.t(), x_c, out_dtype=torch.float32, out=dw32)
+                dw, dw32 = _weight_grad(logits, x_c, dw32, r0 == 0, r1 == N)
             del logits
-        ctx.save_for_backward(dx, dw32.to(weight.dtype) if need_dw else None)
+        if need_dw and dw is None:  # no rows, or the library's last chunk
+            dw = torch.zeros_like(weight) if dw32 is None else dw32.to(weight.dtype)
+        ctx.save_for_backward(dx, dw)
         return loss_sum * inv_count[0]
 
     @staticmethod

@@ -495,6 +495,24 @@ def gemm(op: str, a: torch.Tensor, b: torch.Tensor, *, residual: torch.Tensor | 
     return c
 
 
+def gemm_acc(a: torch.Tensor, b: torch.Tensor, acc: torch.Tensor, *, add: bool,
+             out: torch.Tensor | None = None) -> None:
+    """acc (fp32 [m, n], contiguous) = a[k,m]^T @ b[k,n] (+ acc, with `add`), in
+    fp32; with `out` (bf16 [m, n]) the sum is rounded into `out` instead and acc
+    only read (fh_gemm_bf16_acc)."""
+    _require_gpu(a, b, acc, out)
+    if not gemm_any_k_supported("tn", a, b):
+        raise ValueError(f"gemm_acc: unsupported operands {tuple(a.shape)} {a.stride()} x {tuple(b.shape)} {b.stride()}")
+    m, n, k = gemm_dims("tn", a, b)
+    if acc.dtype != torch.float32 or acc.shape != (m, n) or not acc.is_contiguous() or acc.data_ptr() % 16:
+        raise ValueError(f"gemm_acc: acc must be an aligned, contiguous fp32 [{m}, {n}] tensor")
+    if out is not None and (out.dtype != torch.bfloat16 or out.shape != (m, n) or out.stride(1) != 1
+                            or out.stride(0) % 8 or out.data_ptr() % 16):
+        raise ValueError(f"gemm_acc: out must be a 16-byte aligned bf16 [{m}, {n}] view, row stride % 8 == 0")
+    _lib.call("fh_gemm_bf16_acc", _ptr(a), a.stride(0), _ptr(b), b.stride(0), _ptr(acc), int(add), _ptr(out),
+              0 if out is None else out.stride(0), m, n, k, _stream(a))
+
+
 # fh_gemm_f32 takes products of at most this many outputs and k (weight
 # gradients: k of at most 256).  There the library runs some shapes as one tile
 # on one CU (256 x 256 x 688 160 us against 8, 256 x 256 x 512 'nn' 118 against 8)

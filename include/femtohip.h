@@ -438,6 +438,13 @@ int fh_gemm_bf16_grouped_any_k(int op, int count, const fh_gemm_problem* problem
 int fh_gemm_f32(int op, const void* a, int64_t lda, const void* b, int64_t ldb, void* c, int64_t ldc,
                 const void* residual, int64_t ldr, int64_t m, int64_t n, int64_t k, hipStream_t stream);
 
+/* A weight gradient of tokens that come in chunks: acc [m, n] (fp32, row-major,
+ * no padding) = a[k, m]^T b[k, n] (+ acc, with add).  With c (bf16, ldc) the sum
+ * is rounded into c instead and acc only read.  Any k of at least 64; the other
+ * requirements of fh_gemm_bf16's FH_GEMM_TN.  No workspace. */
+int fh_gemm_bf16_acc(const void* a, int64_t lda, const void* b, int64_t ldb, float* acc, int add, void* c,
+                     int64_t ldc, int64_t m, int64_t n, int64_t k, hipStream_t stream);
+
 /* The q/k/v projection with the rotary embedding in its epilogue: C = A B^T
  * (FH_GEMM_NT, no residual) and then, on columns [0, rot_cols) of C (the q and
  * k heads of head_dim columns each), the rotation of fh_rope_fwd -- bit for

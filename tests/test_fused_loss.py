@@ -187,3 +187,31 @@ def test_fused_loss_lowers_peak_activation_memory():
     p_stock = peak(False)
     p_fused = peak(True)
     assert p_fused < 0.5 * p_stock, f"fused {p_fused / 2**20:.0f} MiB vs stock {p_stock / 2**20:.0f} MiB"
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("N,H,V,rows", [(512, 256, 1024, 512),   # one chunk
+                                        (700, 256, 1024, 256),   # three, the last of 188 rows
+                                        (530, 264, 1000, 256),   # the last of 18: fewer than a hand-written product takes
+                                        (520, 100, 1000, 256),   # a width that the hand-written products do not take
+                                        (40, 2056, 1024, 256)])  # a wide one, and few rows
+def test_loss_head_in_chunks_matches_fp64(monkeypatch, dtype, N, H, V, rows):
+    """Loss and both gradients against fp64 with the logits and their gradient rounded where the head rounds them:
+    every product sums in fp32 and rounds once, so only those roundings and the output's are left (bf16 2^-8 each)."""
+    import femtotron_amd.fused_loss as fl
+    monkeypatch.setattr(fl, "CHUNK_BYTES", rows * V * dtype.itemsize)
+    g = torch.Generator().manual_seed(N + H)
+    x = torch.randn(N, H, generator=g).to(dtype).to(DEV).requires_grad_(True)
+    w = (torch.randn(V, H, generator=g) * H ** -0.5).to(dtype).to(DEV).requires_grad_(True)
+    labels = _labels(1, N, V, 3)[0].to(DEV)
+    loss = fl.FusedLinearCrossEntropy.apply(x, w, labels)
+    loss.backward()
+    x64, w64 = (t.detach().double().requires_grad_(True) for t in (x, w))
+    want = F.cross_entropy(x64 @ w64.t(), labels, ignore_index=IGNORE_INDEX)
+    want.backward()
+    # relative to the tensor's norm: roundings are independent, so their sums grow no faster than the norm
+    tol = 1e-5 if dtype == torch.float32 else 3 * 2.0 ** -8
+    assert abs(loss.item() - want.item()) <= tol * abs(want.item())
+    for got, ref in ((x.grad, x64.grad), (w.grad, w64.grad)):
+        assert float((got.double() - ref).norm() / ref.norm()) < tol

@@ -418,3 +418,39 @@ def test_gemm_rope_rejects_bad_arguments():
     st = lib.fh_gemm_bf16_rope(x.data_ptr(), 128, x.data_ptr(), 128, x.data_ptr(), 128, 256, 128, 128,
                                128, 64, 100, c64.data_ptr(), c64.data_ptr(), 0, None)
     assert st == 1 and b"multiple of seq_len" in lib.fh_last_error()
+
+
+@pytest.mark.parametrize("m,n,k", [(256, 256, 64), (8, 8, 65), (264, 520, 200), (512, 256, 1024), (1000, 72, 127)])
+@pytest.mark.parametrize("add", [False, True])
+@pytest.mark.parametrize("rounded", [False, True])
+def test_weight_gradient_into_an_fp32_sum(m, n, k, add, rounded):
+    """fh_gemm_bf16_acc at tile and k edges: the fp32 sum (k products in fp32: 2^-24 k of their absolute sum) or its
+    one rounding to bf16 (2^-8 more); the sum's neighbours, and with `out` the sum itself, keep their values."""
+    g = torch.Generator().manual_seed(m + n + k)
+    a, b = (torch.randn(k, d, generator=g).bfloat16().to(DEV) for d in (m, n))
+    buf = torch.randn(m * n + 64, generator=g).to(DEV)
+    acc = buf[32:32 + m * n].view(m, n)
+    before = buf.clone()
+    old = acc.double() if add else torch.zeros(m, n, dtype=torch.float64, device=DEV)
+    out = torch.full((m, n + 8), -7.0, dtype=torch.bfloat16, device=DEV)[:, :n] if rounded else None
+    ops.gemm_acc(a, b, acc, add=add, out=out)
+    want = old + a.double().t() @ b.double()
+    lim = 2.0 ** -24 * (k + 1) * (old.abs() + a.double().abs().t() @ b.double().abs())
+    if rounded:
+        assert torch.equal(buf, before)
+        assert bool(((out.double() - want).abs() <= lim + 2.0 ** -8 * want.abs()).all())
+        assert bool((out.as_strided((m, 8), (n + 8, 1), n) == -7.0).all())
+    else:
+        assert bool(((acc.double() - want).abs() <= lim).all())
+        before[32:32 + m * n] = buf[32:32 + m * n]
+        assert torch.equal(buf, before)
+
+
+def test_weight_gradient_into_an_fp32_sum_refuses_other_operands():
+    a, b = torch.zeros(64, 16, device=DEV).bfloat16(), torch.zeros(64, 8, device=DEV).bfloat16()
+    acc, out = torch.zeros(16, 8, device=DEV), torch.zeros(16, 8, device=DEV).bfloat16()
+    for bad in (dict(a=a[:32], b=b[:32]), dict(a=a.float()), dict(acc=acc.double()), dict(acc=acc.t()),
+                dict(acc=torch.zeros(129, device=DEV)[1:].view(16, 8)), dict(out=out.float()), dict(out=out[:8])):
+        args = dict(a=a, b=b, acc=acc, out=out) | bad
+        with pytest.raises(ValueError):
+            ops.gemm_acc(args["a"], args["b"], args["acc"], add=True, out=args["out"])
