@@ -496,20 +496,22 @@ extern "C" int fh_embedding_bwd(fh_dtype dt, const void* dy, const int64_t* ids,
     hipLaunchKernelGGL(k_embed_keys, dim3(static_cast<unsigned>((wide + kEmbThreads - 1) / kEmbThreads)),
                        dim3(kEmbThreads), 0, stream, ids, n_tokens, vocab, padding_idx, keys[0], vals[0],
                        seg_start, seg_end);
-    const int tiles = static_cast<int>((n_tokens + kTile - 1) / kTile);
-    const int passes = radix_passes(vocab);
-    for (int p = 0; p < passes; ++p) {
-      hipLaunchKernelGGL(k_radix_hist, dim3(tiles), dim3(kEmbThreads), 0, stream, keys[cur], n_tokens,
-                         8 * p, hist, tiles);
-      hipLaunchKernelGGL(k_radix_scan, dim3(1), dim3(1024), 0, stream, hist,
-                         static_cast<int64_t>(tiles) * kBins);
-      hipLaunchKernelGGL(k_radix_scatter, dim3(tiles), dim3(kEmbThreads), 0, stream, keys[cur],
-                         vals[cur], keys[cur ^ 1], vals[cur ^ 1], n_tokens, 8 * p, hist, tiles);
-      cur ^= 1;
+    if (n_tokens > 0) {
+      const int tiles = static_cast<int>((n_tokens + kTile - 1) / kTile);
+      const int passes = radix_passes(vocab);
+      for (int p = 0; p < passes; ++p) {
+        hipLaunchKernelGGL(k_radix_hist, dim3(tiles), dim3(kEmbThreads), 0, stream, keys[cur], n_tokens,
+                           8 * p, hist, tiles);
+        hipLaunchKernelGGL(k_radix_scan, dim3(1), dim3(1024), 0, stream, hist,
+                           static_cast<int64_t>(tiles) * kBins);
+        hipLaunchKernelGGL(k_radix_scatter, dim3(tiles), dim3(kEmbThreads), 0, stream, keys[cur],
+                           vals[cur], keys[cur ^ 1], vals[cur ^ 1], n_tokens, 8 * p, hist, tiles);
+        cur ^= 1;
+      }
+      hipLaunchKernelGGL(k_embed_bounds, dim3(static_cast<unsigned>((n_tokens + kEmbThreads - 1) / kEmbThreads)),
+                         dim3(kEmbThreads), 0, stream, keys[cur], n_tokens, static_cast<uint32_t>(vocab),
+                         seg_start, seg_end);
     }
-    hipLaunchKernelGGL(k_embed_bounds, dim3(static_cast<unsigned>((n_tokens + kEmbThreads - 1) / kEmbThreads)),
-                       dim3(kEmbThreads), 0, stream, keys[cur], n_tokens, static_cast<uint32_t>(vocab),
-                       seg_start, seg_end);
   }
   // A row of kHotTokens tokens needs that many.
   const int64_t hot_parts = (hidden + kRowsPerBlock * kHotCols - 1) / (kRowsPerBlock * kHotCols);

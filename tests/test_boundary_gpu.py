@@ -88,6 +88,15 @@ def test_embedding_bwd_zipf_ids_ordered_exact(dtype, T, V, H):
     assert torch.equal(got, want32.to(dtype))
 
 
+@pytest.mark.parametrize("V", [524288, 524296])
+def test_embedding_bwd_no_tokens(V):
+    """No tokens: all rows zero, with the ids grouped in one launch and sorted."""
+    from femtotron_amd import ops
+    dy = torch.empty(0, 8, dtype=torch.bfloat16, device=DEV)
+    got = ops.embedding_bwd(dy, torch.empty(0, dtype=torch.int64, device=DEV), V)
+    assert got.shape == (V, 8) and not got.any()
+
+
 def test_embedding_bwd_tinyllama_vs_torch_and_deterministic():
     """TinyLlama step shape (16384 tokens, V = 32000, H = 2048, bf16): within one
     bf16 ulp of torch's F.embedding backward on the GPU and of the fp64 sums;
