@@ -1345,7 +1345,9 @@ __global__ __launch_bounds__(256) void k_attn_fwd_f32(
       for (int e = 0; e < 4; ++e)
         if (16 * t + 4 * c + e < hi) mloc = fmaxf(mloc, x[t][e] * scale_log2);
     const float mn = fmaxf(m, col_max(mloc));
-    const float alpha = fast_exp2(m - mn);
+    // Scores of -inf only (so far): weights 0, not exp2(-inf + inf).
+    const float ms = mn == -INFINITY ? 0.f : mn;
+    const float alpha = fast_exp2(m - ms);
     m = mn;
     l *= alpha;
 #pragma unroll
@@ -1354,7 +1356,7 @@ __global__ __launch_bounds__(256) void k_attn_fwd_f32(
     for (int t = 0; t < 2; ++t)
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        x[t][e] = 16 * t + 4 * c + e < hi ? fast_exp2(fmaf(x[t][e], scale_log2, -mn)) : 0.f;
+        x[t][e] = 16 * t + 4 * c + e < hi ? fast_exp2(fmaf(x[t][e], scale_log2, -ms)) : 0.f;
         l += x[t][e];
       }
     wsum_f32<HD>(oacc, x, vp + static_cast<int64_t>(k0) * ldv, ldv, S - 1 - k0, k0 + 31 > q0, 0, hi, r, c);

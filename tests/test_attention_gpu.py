@@ -171,6 +171,29 @@ def test_attention_fp32_masked_rows_do_not_leak(hd, bad):
 
 
 @pytest.mark.parametrize("hd", [32, 64, 128])
+def test_attention_fp32_overflowed_scores_weigh_nothing(hd):
+    """Scores of -inf in a whole key block (keys 0-31, whose products overflow) are
+    weights of 0 for the queries that see other keys as well: their outputs are
+    attention over keys 32 .. i (fp32 sums of at most 77 terms: 1e-5 of the peak)."""
+    ops = _ops()
+    S, nh, cut = 77, 2, 32
+    hq = nh * hd
+    buf, _ = _inputs(1, S, nh, nh, hd, torch.float32, 5)
+    buf[:, :hq] = buf[:, :hq].abs() + 0.1
+    buf[:cut, hq:2 * hq] = -3e38
+    q, k, v = (buf[:, i * hq:(i + 1) * hq] for i in range(3))
+    g = buf.to(DEV)
+    o, _ = ops.attn_fwd(g[:, :hq], g[:, hq:2 * hq], g[:, 2 * hq:], 1, S, nh, nh, hd, hd ** -0.5)
+    want = torch.empty(S - cut, hq, dtype=torch.float64)
+    seen = torch.ones(S - cut, S - cut, dtype=torch.bool).tril()
+    for h in range(nh):
+        qh, kh, vh = (t[cut:, h * hd:(h + 1) * hd].double() for t in (q, k, v))
+        p = torch.softmax((qh @ kh.t() * hd ** -0.5).masked_fill(~seen, -float("inf")), -1)
+        want[:, h * hd:(h + 1) * hd] = p @ vh
+    assert float((o[cut:].cpu().double() - want).abs().max() / want.abs().max()) < 1e-5
+
+
+@pytest.mark.parametrize("hd", [32, 64, 128])
 def test_attention_ragged_tiles_stay_inside_their_sequence(hd):
     """Tiles that run past S load clamped rows of their own sequence, never the
     next one: with every q/k/v/dO value of sequence 1 set to NaN, sequence 0's
