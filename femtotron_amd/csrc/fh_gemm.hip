@@ -278,6 +278,11 @@ template <int W>
 constexpr int kSlotOf = 2 * W * 128;
 constexpr int kSlot = kSlotOf<128>;
 constexpr int kRing = 5;  // operand slots in LDS (160 KB, or 80 KB for W = 64)
+// Stages from a load to its use in the 128 x 128 tile where a CU has one workgroup
+// (2 everywhere else), and the ring that takes: two slots per stage and a free one.
+constexpr int kDeep = 4;
+template <int D>
+constexpr int kRingOf = 2 * D + 1;
 
 // Zeroes the first `n` of the 64 k's of this wave's quarter of an operand's
 // stage, which has landed (lane i filled 16-byte slot i of each 1 KB run, with
@@ -297,7 +302,11 @@ __device__ __forceinline__ void wait_vm_n() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
-__device__ __forceinline__ int mod5(int v) { return v >= 5 ? v - 5 : v; }
+template <int R>
+__device__ __forceinline__ int mod_ring(int v) {
+  return v >= R ? v - R : v;
+}
+__device__ __forceinline__ int mod5(int v) { return mod_ring<kRing>(v); }
 
 // Origin of tile t: tiles run in groups of 1024 rows (GM m-tiles), n-major inside a
 // group, so consecutive tiles (and the workgroups of one XCD) share B columns
@@ -343,8 +352,8 @@ __device__ __forceinline__ GemmArgs for_tile(const GemmArgs& g, int& t) {
 // to_part, as fp32 to pdst (the tile's origin, row stride pld).  EPI_ACC: the
 // fp32 sum of the product and, with g.add, of pdst, to pdst or rounded to C.  EPI_STREAM
 // ends with a barrier, as the workgroup's next tile reuses the LDS ring.
-// RAGGED: k may be no multiple of 64.
-template <bool A_KO, bool B_KO, int EPI, bool RAGGED, int W>
+// RAGGED: k may be no multiple of 64.  D: stages from a load to its use.
+template <bool A_KO, bool B_KO, int EPI, bool RAGGED, int W, int D = 2>
 __device__ __forceinline__ void gemm_tile(const GemmArgs& g, char* ring, int t, int s_begin, int nst,
                                           float* pdst, int64_t pld, bool to_part) {
   constexpr int F = W / 16, RUNS = W / 16;  // fragments per operand and k32 step; loads per operand and stage
@@ -416,17 +425,17 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, char* ring, int t, 
     else acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[buf][i], fa[buf][j], acc[i][j], 0, 0, 0);
   };
 
-  // Operand u (A of stage x: u = 2x, B: 2x+1) lives in ring slot u % 5.
-  // Prologue: stages 0 and 1, wait for stage 0, read its step-0 fragments.
+  // Operand u (A of stage x: u = 2x, B: 2x+1) lives in ring slot u % R, R = 2 D + 1.
+  // Prologue: stages 0 to D - 1, wait for stage 0, read its step-0 fragments.
+  constexpr int R = kRingOf<D>;
 #pragma unroll
-  for (int jj = 0; jj < RUNS; ++jj) dma(OpA(), 0, 0, jj);
+  for (int st = 0; st < D; ++st) {
 #pragma unroll
-  for (int jj = 0; jj < RUNS; ++jj) dma(OpB(), 0, 1, jj);
+    for (int jj = 0; jj < RUNS; ++jj) dma(OpA(), st, 2 * st, jj);
 #pragma unroll
-  for (int jj = 0; jj < RUNS; ++jj) dma(OpA(), 1, 2, jj);
-#pragma unroll
-  for (int jj = 0; jj < RUNS; ++jj) dma(OpB(), 1, 3, jj);
-  wait_vm_n<2 * RUNS>();
+    for (int jj = 0; jj < RUNS; ++jj) dma(OpB(), st, 2 * st + 1, jj);
+  }
+  wait_vm_n<2 * RUNS * (D - 1)>();
   // The stage that repeats k's, if this range ends with it (-1: none).
   [[maybe_unused]] const int xr = g.repeat > 0 && s_begin + nst == g.total_steps ? nst - 1 : -1;
   [[maybe_unused]] auto zero = [&](int sa, int sb) __attribute__((always_inline)) {
@@ -443,38 +452,49 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, char* ring, int t, 
     __builtin_amdgcn_sched_barrier(0);
   }
 
-  // Stage x (A in slot s, B in s+1; stage x+1 in s+2, s+3; s+4 free):
+  // Stage x (A in slot s, B in s+1; stage x+1 in s+2, s+3; ...; s+2D free):
   //   step 0: its MFMAs on buffer 0 while step 1's fragments are read into
-  //     buffer 1 (one read per F / 2 MFMAs) and A(x+2) is loaded into s+4;
-  //   then each wave waits for its reads and for every load but A(x+2)'s
-  //   (stage x+1 complete in LDS), and the barrier: stage x's slots are
+  //     buffer 1 (one read per F / 2 MFMAs) and A(x+D) is loaded into s+2D;
+  //   then each wave waits for its reads and for every load up to stage x+1's
+  //   (complete in LDS), and the barrier: stage x's slots are
   //   read no more;
   //   step 1: its MFMAs on buffer 1 while the next stage's step-0 fragments
-  //     are read into buffer 0 and B(x+2) is loaded into slot s.
+  //     are read into buffer 0 and B(x+D) is loaded into slot s.
+  // D > 2: the last D stages (LOAD false) load nothing, as that many re-loads would
+  // be most of a short slice's traffic; `left` stages after x+1 are then in flight.
   int s = 0;
-  for (int x = 0; x < nst; ++x) {
-    const int sB = mod5(s + 1), nA = mod5(s + 2), nB = mod5(s + 3), fA = mod5(s + 4);
+  auto stage = [&](auto load_tag, int x) __attribute__((always_inline)) {
+    constexpr bool LOAD = decltype(load_tag)::value;
+    const int sB = mod_ring<R>(s + 1), nA = mod_ring<R>(s + 2), nB = mod_ring<R>(s + 3), fA = mod_ring<R>(s + 2 * D);
     // VALU writes of an accumulator (the zeroing before the loop) need wait
     // states before an MFMA reads it.
     if constexpr (W == 128) asm volatile("s_nop 4");
 #pragma unroll
     for (int p = 0; p < F * F; ++p) {
       if (p % (F / 2) == 0) rd1(s, sB, 1, 1, p / (F / 2));
-      if (p % F == 1) set_m0(ring0 + fA * SLOT + (p / F) * 1024);
-      if (p % F == 2) dma_m0(OpA(), x + 2, p / F);
+      if (LOAD && p % F == 1) set_m0(ring0 + fA * SLOT + (p / F) * 1024);
+      if (LOAD && p % F == 2) dma_m0(OpA(), x + D, p / F);
       mf1(0, p);
       __builtin_amdgcn_sched_barrier(0);
     }
     wait_lds();
-    wait_vm_n<RUNS>();
+    if constexpr (LOAD) {
+      wait_vm_n<RUNS + 2 * RUNS * (D - 2)>();
+    } else {
+      static_assert(LOAD || D == 4, "the waits below are those of four stages");
+      const int left = nst - 2 - x;
+      if (left >= 2) wait_vm_n<4 * RUNS>();
+      else if (left == 1) wait_vm_n<2 * RUNS>();
+      else wait_vm();
+    }
     if constexpr (RAGGED)
       if (x + 1 == xr) zero(nA, nB);
     bar();
 #pragma unroll
     for (int p = 0; p < F * F; ++p) {
       if (p % (F / 2) == 0) rd1(nA, nB, 0, 0, p / (F / 2));
-      if (p % F == 1) set_m0(ring0 + s * SLOT + (p / F) * 1024);
-      if (p % F == 2) dma_m0(OpB(), x + 2, p / F);
+      if (LOAD && p % F == 1) set_m0(ring0 + s * SLOT + (p / F) * 1024);
+      if (LOAD && p % F == 2) dma_m0(OpB(), x + D, p / F);
       mf1(1, p);
       __builtin_amdgcn_sched_barrier(0);
     }
@@ -485,6 +505,13 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, char* ring, int t, 
     // reads the accumulators.
     if constexpr (W == 128)
       if (x == nst - 1) asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7");
+  };
+  if constexpr (D == 2) {
+    for (int x = 0; x < nst; ++x) stage(std::true_type(), x);
+  } else {
+    int x = 0;
+    for (; x < nst - D; ++x) stage(std::true_type(), x);
+    for (; x < nst; ++x) stage(std::false_type(), x);
   }
   __builtin_amdgcn_sched_barrier(0);
   // The re-loads past the end and the last stale fragment reads complete
@@ -910,16 +937,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
 // The 128 x 128 tile: W = 64, so a workgroup needs 80 KB of LDS and half the
 // registers, and two run on a CU.  One tile, or one K slice of it
 // (EPI_PARTIAL), per workgroup; EPI_GROUP: the tiles of a group's problems.
-template <bool A_KO, bool B_KO, int EPI, bool RAGGED>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_gemm_mid(GemmArgs g) {
-  __shared__ __align__(16) char ring[kRing * kSlotOf<64>];
+template <bool A_KO, bool B_KO, int EPI, bool RAGGED, int D>
+__device__ __forceinline__ void gemm_mid(const GemmArgs& g, char* ring) {
   const int nb8 = gridDim.x >> 3;
   const int lid = (blockIdx.x & 7) * nb8 + (blockIdx.x >> 3);
   if (lid >= g.grid) return;
   if constexpr (EPI == EPI_GROUP) {
     int t = lid;
     const GemmArgs pg = for_tile(g, t);
-    gemm_tile<A_KO, B_KO, EPI, RAGGED, 64>(pg, ring, t, 0, g.total_steps, nullptr, 0, false);
+    gemm_tile<A_KO, B_KO, EPI, RAGGED, 64, D>(pg, ring, t, 0, g.total_steps, nullptr, 0, false);
   } else {
     const int slice = lid / g.tiles, t = lid - slice * g.tiles;
     const int s_begin = slice * g.steps_per_slice;
@@ -928,10 +954,26 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     float* pdst = EPI == EPI_PARTIAL
                       ? g.part + static_cast<int64_t>(slice) * g.m * g.n + static_cast<int64_t>(m0) * g.n + n0
                       : nullptr;
-    gemm_tile<A_KO, B_KO, EPI, RAGGED, 64>(g, ring, t, s_begin, min(g.total_steps - s_begin, g.steps_per_slice), pdst,
+    gemm_tile<A_KO, B_KO, EPI, RAGGED, 64, D>(g, ring, t, s_begin, min(g.total_steps - s_begin, g.steps_per_slice), pdst,
                                            g.n, EPI == EPI_PARTIAL);
   }
 }
+
+template <bool A_KO, bool B_KO, int EPI, bool RAGGED>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_gemm_mid(GemmArgs g) {
+  __shared__ __align__(16) char ring[kRing * kSlotOf<64>];
+  gemm_mid<A_KO, B_KO, EPI, RAGGED, 2>(g, ring);
+}
+
+// The same with loads kDeep stages ahead, for launches of at most one workgroup per
+// CU.  Its 144 KB of LDS are the launch's dynamic LDS: seeing one workgroup per
+// CU, the compiler would move the accumulators to AGPRs and copy them at every stage.
+template <bool A_KO, bool B_KO, int EPI, bool RAGGED>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_gemm_deep(GemmArgs g) {
+  extern __shared__ __align__(16) char deep_ring[];
+  gemm_mid<A_KO, B_KO, EPI, RAGGED, kDeep>(g, deep_ring);
+}
+constexpr size_t kDeepLds = kRingOf<kDeep> * kSlotOf<64>;
 
 // The persistent form (gemm_persist): G = gridDim.x workgroups, a multiple of
 // 8, at most the number of tiles.
@@ -1085,7 +1127,8 @@ constexpr int kMid = 128;  // tile of k_gemm_mid
 // and TN of three widths, 16 to 4096 tokens, each timed in 256 x 256 tiles and in
 // 128 x 128 tiles over 1 to 8 slices): stages per CU times a stage's time, a
 // cost per tile and per launch, and for K slices writing and re-reading the
-// partials.  A 128 x 128 stage takes 0.41-0.56 us for a quarter of the work of
+// partials.  A 128 x 128 stage takes 0.41-0.56 us (0.37-0.57 in k_gemm_deep, fitted
+// to 200 more products) for a quarter of the work of
 // the 256 x 256 stage's 1.18 (LDS reads per MFMA double), so the small tiles win
 // only where the large ones leave CUs idle or split K: 256 x 11264 x 2048 32 ->
 // 20 us, 512 x 2048 x 2048 28 -> 14, 999 x 2048 x 2048 31 -> 19, 256 x 2048 x
@@ -1103,8 +1146,28 @@ double reduce_us(int64_t m, int64_t n, int64_t slices) {
   return slices > 1 ? kReduceFixed + kReducePerMB * static_cast<double>(slices) * m * n * 4e-6 : 0.0;
 }
 
-double mid_us(int op, int64_t tiles, int64_t m, int64_t n, int64_t per, int64_t slices, int cus) {
-  return static_cast<double>(ceil_div(tiles * slices, cus)) * per * kMidStage[op] + kMidFixed +
+// Whether a launch of 128 x 128 tiles (`per` stages each) runs with loads kDeep
+// stages ahead (k_gemm_deep): no CU has a second workgroup whose MFMAs would fill the
+// wait for a load, the operands are well past one XCD's 4 MB of L2, whose latency two
+// stages cover, and there are stages enough to set against filling four.  Stages of
+// 0.41-0.56 us become 0.37-0.46 (0.57 from about 200 on, where the workgroups no
+// longer share blocks in L2): 256 x 11264 x 2048 21.1 -> 18.3 us, 512 x 2048 x 2048
+// 19.2 -> 16.2 (NN 21.2 -> 16.6), 1024 x 4096 x 4096 NN 42.3 -> 33.8, 16 x 28672 x 4096
+// 63.5 -> 49.0, that is 4.8 TB/s.  With 4 stages, or most of it in L2 (256-wide
+// models: 256 x 256 x 688 8.9 -> 9.4, 2002 x 256 x 1376 14.6 -> 15.4), it would lose.
+bool mid_deep(int64_t workgroups, int64_t per, int64_t m, int64_t n, int64_t steps) {
+  return workgroups <= device_cus() && per >= 8 && (m + n) * steps * (kTk * 2) > (int64_t(8) << 20);
+}
+
+double deep_stage_us(int op, int64_t per) {
+  const double base[3] = {0.37, 0.38, 0.44};  // NT, NN, TN
+  return base[op] + 5e-4 * static_cast<double>(std::min<int64_t>(per, 96)) +
+         1.2e-3 * static_cast<double>(std::max<int64_t>(0, std::min<int64_t>(per, 224) - 96));
+}
+
+double mid_us(int op, int64_t tiles, int64_t m, int64_t n, int64_t steps, int64_t per, int64_t slices, int cus) {
+  const double stage = mid_deep(tiles * slices, per, m, n, steps) ? deep_stage_us(op, per) : kMidStage[op];
+  return static_cast<double>(ceil_div(tiles * slices, cus)) * per * stage + kMidFixed +
          kMidTile * static_cast<double>(tiles * slices) / cus + reduce_us(m, n, slices);
 }
 
@@ -1139,7 +1202,7 @@ GemmPlan gemm_plan(int op, int64_t m, int64_t n, int64_t k) {
   double bound = kMidMargin * p.us;
   for (int s = 1; s <= 8 && (s == 1 || s <= k / 256); ++s) {
     const int64_t mper = ceil_div(steps, s), ms = ceil_div(steps, mper);
-    const double us = mid_us(op, mid_tiles, m, n, mper, ms, cus);
+    const double us = mid_us(op, mid_tiles, m, n, steps, mper, ms, cus);
     if (us < bound - 1e-9) {
       bound = us;
       p = GemmPlan{static_cast<int>(ms), false, true, us};
@@ -1200,7 +1263,14 @@ void launch_mid(const GemmArgs& g, unsigned blocks, bool partial, hipStream_t st
   const dim3 grid(blocks), block(256);
   if (g.grouped)
     hipLaunchKernelGGL((k_gemm_mid<A_KO, B_KO, EPI_GROUP, RAGGED>), grid, block, 0, stream, g);
-  else if (partial)
+  else if (mid_deep(g.grid, g.steps_per_slice, g.m, g.n, g.total_steps)) {
+    if (partial)
+      hipLaunchKernelGGL((k_gemm_deep<A_KO, B_KO, EPI_PARTIAL, RAGGED>), grid, block, kDeepLds, stream, g);
+    else if (g.r != nullptr)
+      hipLaunchKernelGGL((k_gemm_deep<A_KO, B_KO, EPI_RESIDUAL, RAGGED>), grid, block, kDeepLds, stream, g);
+    else
+      hipLaunchKernelGGL((k_gemm_deep<A_KO, B_KO, EPI_STORE, RAGGED>), grid, block, kDeepLds, stream, g);
+  } else if (partial)
     hipLaunchKernelGGL((k_gemm_mid<A_KO, B_KO, EPI_PARTIAL, RAGGED>), grid, block, 0, stream, g);
   else if (g.r != nullptr)
     hipLaunchKernelGGL((k_gemm_mid<A_KO, B_KO, EPI_RESIDUAL, RAGGED>), grid, block, 0, stream, g);

@@ -291,6 +291,24 @@ def test_mid_tiles_match_and_add_the_residual(op, m, n, k, pad):
 
 
 @pytest.mark.parametrize("op", ["nt", "nn", "tn"])
+@pytest.mark.parametrize("m,n,k", [
+    (264, 8200, 512), (264, 8200, 520), (256, 8200, 584), (264, 8200, 640), (1000, 3976, 1160),  # whole K, 8 to 19 stages
+    (264, 2056, 2056), (136, 2056, 5000), (16, 4104, 4104), (520, 1032, 2888), (8, 2048, 11264),  # K slices
+])
+def test_mid_tiles_four_stages_ahead(op, m, n, k):
+    """At most one workgroup per CU and operands past one XCD's L2: four stages in flight, slices of eight stages and
+    more (the last one shorter, its last k ragged), operands followed by NaNs."""
+    g = torch.Generator(device=DEV).manual_seed(m + k)
+    shapes = {"nt": ((m, k), (n, k)), "nn": ((m, k), (k, n)), "tn": ((k, m), (k, n))}[op]
+    a, b = (_guarded(*s, g) for s in shapes)
+    c = ops.gemm(op, a, b, any_k=True)
+    _check(op, a, b, c)
+    r = torch.randn(m, n, device=DEV, generator=g).to(BF)
+    want = (r.float() + c.float()).to(BF)
+    assert torch.equal(ops.gemm(op, a, b, residual=r, out=r, any_k=True), want)
+
+
+@pytest.mark.parametrize("op", ["nt", "nn", "tn"])
 @pytest.mark.parametrize("m,n,k", [(256, 256, 256), (1, 8, 4), (33, 40, 20), (31, 72, 132), (256, 264, 688),
                                    (300, 256, 64), (8, 520, 248)])
 def test_small_f32_product(op, m, n, k):
