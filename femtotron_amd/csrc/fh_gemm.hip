@@ -38,9 +38,10 @@
 //     immediates.
 // Outputs that 256 x 256 tiles would spread over few CUs run in 128 x 128 tiles
 // (k_gemm_mid, chosen by gemm_plan): the same stages and ring with a quarter of
-// the wave's outputs, 80 KB of LDS and two workgroups per CU.  The GEMMs of a
-// 2048-wide layer at 256 tokens 430 -> 265 us of kernel time, at 999 tokens 606 ->
-// 476 us.
+// the wave's outputs, 80 KB of LDS and two workgroups per CU; or, for launches of
+// at most one workgroup per CU, four stages in flight in 144 KB (k_gemm_deep).  The
+// GEMMs of a 2048-wide layer at 256 tokens 430 -> 242 us of kernel time, at 999 tokens
+// 606 -> 454 us.
 // The MFMA is issued as (B fragment, A fragment), so each lane's four
 // accumulator values are consecutive along n (C's contiguous index).  The finished tile goes through LDS so that
 // every global store writes whole rows.
