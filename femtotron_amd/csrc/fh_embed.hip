@@ -290,10 +290,18 @@ __global__ __launch_bounds__(kGroupThreads) void k_embed_group(const int64_t* __
 // (2 per lane) with the rows of up to kHotDepth tokens in flight, the additions
 // still one after the other in token order: 58-62 us there.  (One wave per row and
 // 1024 threads per workgroup, the tokens read as scalars: 132 us.)
+//
+// A hot workgroup looks through hot_ids consecutive ids and sums its frequent ones
+// one after the other: 64 of them where the vocabulary gives workgroups enough, as
+// few of whose ids are frequent, fewer (down to one) in a small vocabulary, whose
+// ids may all be: fh_embedding_bwd halves them until there are kHotWaves waves.
+// With 64 throughout, uniform ids of a small vocabulary were 32 waves' work at
+// V = 1024, H = 256 (16384 tokens: 91 us, now 17; one wave per row 40) and 64 at
+// V = 64, H = 2048 (4096 tokens: 203 us, now 11; one wave per row 64).
 constexpr int kRowChunks = 4;
 constexpr int kHotTokens = 8;
-constexpr int kHotIds = kWave;      // ids that a hot workgroup looks through
 constexpr int kHotCols = 2 * kWave;  // columns that a wave sums of a hot row
+constexpr int64_t kHotWaves = 4096;  // 16 per CU
 template <typename T>
 constexpr int kHotDepth = sizeof(T) == 2 ? 64 : 32;
 
@@ -350,25 +358,26 @@ __device__ __forceinline__ void hot_columns(const T* __restrict__ dy, const uint
   else *reinterpret_cast<float2*>(dst + c) = make_float2(a0, a1);
 }
 
-// Workgroups [0, hot_blocks): hot_blocks / hot_parts groups of kHotIds ids, and
-// for each group hot_parts workgroups of kRowsPerBlock column slices; then one
-// wave per row.
+// Workgroups [0, hot_blocks): hot_blocks / hot_parts groups of hot_ids (at most 64)
+// ids, and for each group hot_parts workgroups of kRowsPerBlock column slices; then
+// one wave per row.
 template <typename T>
 __global__ __launch_bounds__(kEmbThreads) void k_embed_rows(const T* __restrict__ dy,
                                                             const uint32_t* __restrict__ tok,
                                                             const uint32_t* __restrict__ seg_start,
                                                             const uint32_t* __restrict__ seg_end,
                                                             T* __restrict__ dw, int64_t vocab,
-                                                            int64_t hidden, int hot_blocks, int hot_parts) {
+                                                            int64_t hidden, int hot_blocks, int hot_parts,
+                                                            int hot_ids) {
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int block = blockIdx.x;
   if (block < hot_blocks) {
-    const int64_t v0 = static_cast<int64_t>(block / hot_parts) * kHotIds;
+    const int64_t v0 = static_cast<int64_t>(block / hot_parts) * hot_ids;
     const int64_t c0 = static_cast<int64_t>(block % hot_parts * kRowsPerBlock + wave) * kHotCols;
     if (c0 >= hidden) return;
     uint32_t lo = 0, len = 0;
-    if (v0 + lane < vocab) {
+    if (lane < hot_ids && v0 + lane < vocab) {
       lo = seg_start[v0 + lane];
       len = seg_end[v0 + lane] - lo;
     }
@@ -515,14 +524,16 @@ extern "C" int fh_embedding_bwd(fh_dtype dt, const void* dy, const int64_t* ids,
   }
   // A row of kHotTokens tokens needs that many.
   const int64_t hot_parts = (hidden + kRowsPerBlock * kHotCols - 1) / (kRowsPerBlock * kHotCols);
-  const int64_t hot_blocks = n_tokens >= kHotTokens ? (vocab + kHotIds - 1) / kHotIds * hot_parts : 0;
+  int64_t hot_ids = kWave;
+  while (hot_ids > 1 && (vocab + hot_ids - 1) / hot_ids * hot_parts * kRowsPerBlock < kHotWaves) hot_ids /= 2;
+  const int64_t hot_blocks = n_tokens >= kHotTokens ? (vocab + hot_ids - 1) / hot_ids * hot_parts : 0;
   const int64_t blocks = hot_blocks + (vocab + kRowsPerBlock - 1) / kRowsPerBlock;
   FH_REQUIRE(blocks <= 0x7fffffff, "embedding_bwd: vocab * hidden too large");
   auto rows = [&](auto tag) {
     using T = decltype(tag);
     hipLaunchKernelGGL(k_embed_rows<T>, dim3(static_cast<unsigned>(blocks)), dim3(kEmbThreads), 0, stream,
                        static_cast<const T*>(dy), vals[cur], seg_start, seg_end, static_cast<T*>(dweight), vocab,
-                       hidden, static_cast<int>(hot_blocks), static_cast<int>(hot_parts));
+                       hidden, static_cast<int>(hot_blocks), static_cast<int>(hot_parts), static_cast<int>(hot_ids));
   };
   if (dt == FH_BF16) rows(uint16_t{});
   else rows(float{});
