@@ -1538,20 +1538,20 @@ int group_setup(int op, int count, const fh_gemm_problem* probs, int64_t k, bool
   return FH_OK;
 }
 
-// The problems' own workspace where they run one by one; else the stream form's
-// segment slots where its tiles allow it (the 128 x 128 tiles need none, but the
-// size stays one of a group's sizes).
+// The stream form's segment slots, nothing for the 128 x 128 tiles, and the most that
+// one of the problems needs where they run one by one.
 size_t group_workspace(int op, int count, const fh_gemm_problem* problems, int64_t k) {
-  int64_t tiles = 0;
   size_t most = 0;
   for (int i = 0; i < count; ++i) {
     const int64_t m = problems[i].m, n = problems[i].n;
     if (m <= 0 || n <= 0) return 0;
-    tiles += ceil_div(m, kTm) * ceil_div(n, kTn);
     most = std::max(most, gemm_workspace(op, m, n, k));
   }
-  if (group_form(op, count, problems, k) == GroupForm::kSeparate) return most;
-  return stream_allowed(tiles, ceil_div(k, kTk)) ? stream_workspace_bytes() : 0;
+  switch (group_form(op, count, problems, k)) {
+    case GroupForm::kStream: return stream_workspace_bytes();
+    case GroupForm::kMid: return 0;
+    default: return most;
+  }
 }
 
 int group_impl(int op, int count, const fh_gemm_problem* problems, int64_t k, bool any_k, void* workspace,

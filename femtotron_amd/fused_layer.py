@@ -325,12 +325,14 @@ def layer_backward(dout2: torch.Tensor, x2: torch.Tensor, cos: torch.Tensor, sin
 
 # The layer as one call per direction (fh_layer_fwd / fh_layer_bwd): while its
 # intermediates are small its kernels end before Python has issued the next ones.
-# Forward and backward op by op and in one call each, wall time, bf16: 688 and 377
-# us (2048 wide, ffn 8192, 256 tokens), 722 and 716 (1000 tokens), 647 and 318 (256
-# wide, 256 tokens), 642 and 457 (1024 wide, 2048 tokens).  Past this workspace
-# the kernels are the time (2048 wide at 1000 tokens, 231 MiB: level already), and
-# op by op an intermediate's memory is reused once it is read.
-ONE_CALL_MAX_BYTES = 256 << 20
+# Forward and backward op by op and in one call each, wall time, bf16, weights
+# packed: 778 and 446 us (2048 wide, ffn 5632, 256 tokens), 745 and 580 (999),
+# 745 and 685 (1100, a workspace of 133 MiB), 843 and 849 (1300, 225 MiB); 715 and
+# 380 (256 wide, ffn 688, 1024 tokens), 742 and 583 (16384, 189 MiB), 1268 and 1258
+# (32768, 323 MiB).  Past this workspace the kernels are the time, and op by op an
+# intermediate's memory is reused once it is read (1300 tokens: a backward's peak
+# of 182 MiB against 313).
+ONE_CALL_MAX_BYTES = 192 << 20
 # fp32: every product runs on fh_gemm_f32, which is made for small ones: 630 and
 # 206 us (256 wide, ffn 688, 256 tokens), 683 and 304 (1024 tokens), 834 and 716 at
 # the largest of these sizes; beyond, the library's larger tiles are faster.

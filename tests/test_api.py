@@ -215,6 +215,28 @@ def test_library_validates_arguments_on_host():
     assert L.fh_gemm_bf16_workspace_size(_lib.FH_GEMM_NT, 64, 64, 96) == 0
 
 
+def _group_workspace(shapes, k):
+    from femtotron_amd import _lib
+    probs = (_lib.FhGemmProblem * len(shapes))()
+    for i, (m, n) in enumerate(shapes):
+        probs[i] = _lib.FhGemmProblem(None, m, None, n, None, n, None, 0, m, n)
+    return _lib.lib().fh_gemm_bf16_grouped_any_k_workspace_size(_lib.FH_GEMM_TN, len(shapes), probs, k)
+
+
+def test_a_group_in_small_tiles_asks_for_no_workspace():
+    """The weight gradients of a 2048-wide layer: few tokens run in 128 x 128 tiles, which
+    write their outputs alone; the stream form has its segment slots (128 MiB on 256 CUs).
+    A one-call backward over 256 tokens holds its intermediates (19 MiB) and K slices."""
+    from femtotron_amd import _lib
+    if not _lib.LIB_PATH.exists():
+        pytest.skip("libfemtohip.so not built")
+    shapes = [(2048, 5632), (2048, 2048), (2560, 2048)]
+    assert _group_workspace(shapes, 256) == _group_workspace(shapes, 999) == 0
+    assert _group_workspace(shapes, 16384) > 0
+    layer = _lib.FhLayer(_lib.FH_BF16, 0, 1, 256, 2048, 32, 4, 64, 5632, 1e-5, 1e-5, 0.125, 0.0, *[None] * 8)
+    assert _lib.lib().fh_layer_workspace_size(ctypes.byref(layer), 1) < 40 << 20
+
+
 def test_linear_weight_accepts_tensor_parallel_wrappers_at_world_size_1():
     """The dispatcher takes femtotron's Column/RowParallelLinear at one rank
     (tensor_parallel/linear.py:42-64, 170-191: weight, bias, world_size,

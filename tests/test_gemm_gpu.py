@@ -184,23 +184,24 @@ def test_residual_epilogue_rounds_like_the_unfused_add(op, m, n, k):
     assert torch.equal(inplace, fused)
 
 
-@pytest.mark.parametrize("op,shapes,k,one_launch", [
+@pytest.mark.parametrize("op,shapes,k,form", [
     # the layer's q/k/v, o and down weight gradients at config 3: 80 + 64 + 176
     # tiles, one stream launch (a whole round, then 64 tail tiles in XCD slabs)
-    ("tn", [(2560, 2048), (2048, 2048), (2048, 5632)], 16384, True),
-    ("tn", [(2560, 2048), (2048, 2048), (2048, 5632)], 256, True),       # 4 k-steps
-    ("tn", [(6144, 4096), (4096, 4096), (4096, 14336)], 1024, True),     # config 4's: six whole rounds, no tail
-    ("tn", [(520, 264), (1032, 776)], 8192, False),                      # ragged, too few tiles: one call each
-    ("tn", [(2600, 2056), (2048, 2048), (2048, 5640)], 4096, True),      # ragged edge tiles in one launch
-    ("nn", [(4096, 2048), (4096, 2560)], 2048, True),                    # the other layouts: 128 + 160 tiles
-    ("nt", [(4096, 2048), (4104, 2568)], 2048, True),
+    ("tn", [(2560, 2048), (2048, 2048), (2048, 5632)], 16384, "stream"),
+    ("tn", [(2560, 2048), (2048, 2048), (2048, 5632)], 256, "mid"),      # few tokens: 128 x 128 tiles
+    ("tn", [(6144, 4096), (4096, 4096), (4096, 14336)], 1024, "stream"),  # config 4's: six whole rounds, no tail
+    ("tn", [(6144, 4096), (4096, 4096), (4096, 14336)], 256, "stream"),  # 4 k-steps
+    ("tn", [(520, 264), (1032, 776)], 8192, "separate"),                 # ragged, too few tiles: one call each
+    ("tn", [(2600, 2056), (2048, 2048), (2048, 5640)], 4096, "stream"),  # ragged edge tiles in one launch
+    ("nn", [(4096, 2048), (4096, 2560)], 2048, "stream"),                # the other layouts: 128 + 160 tiles
+    ("nt", [(4096, 2048), (4104, 2568)], 2048, "stream"),
 ])
-def test_grouped_matches_each_product_and_accumulates(op, shapes, k, one_launch):
+def test_grouped_matches_each_product_and_accumulates(op, shapes, k, form):
     """fh_gemm_bf16_grouped: every problem within the product's bound, bitwise
     repeatable, and with residual == C the accumulating epilogue
     to_bf16(R + to_bf16(A^T B)) bit for bit (whole tiles in the GEMM, split ones
     in the fixup); a group whose tiles do not fill a round runs as separate
-    fh_gemm_bf16 calls."""
+    fh_gemm_bf16 calls, or in 128 x 128 tiles, which need no workspace."""
     g = torch.Generator(device=DEV).manual_seed(k + len(shapes))
     ops_ = [_operands(op, m, n, k, g) for m, n in shapes]
     probs = (_lib.FhGemmProblem * len(shapes))()
@@ -209,8 +210,9 @@ def test_grouped_matches_each_product_and_accumulates(op, shapes, k, one_launch)
     code = {"nt": _lib.FH_GEMM_NT, "nn": _lib.FH_GEMM_NN, "tn": _lib.FH_GEMM_TN}[op]
     ws = _lib.lib().fh_gemm_bf16_grouped_workspace_size(code, len(shapes), probs, k)
     cus = torch.cuda.get_device_properties(0).multi_processor_count // 8 * 8
+    one_launch = form != "separate"
     if one_launch:
-        assert ws == 2 * cus * 256 * 256 * 4
+        assert ws == (2 * cus * 256 * 256 * 4 if form == "stream" else 0)
     outs = ops.gemm_grouped(op, [(a, b, None, None) for a, b in ops_])
     for (a, b), c in zip(ops_, outs):
         _check(op, a, b, c, exact=True)
