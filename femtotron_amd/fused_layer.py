@@ -190,7 +190,8 @@ def grad_target(*params: torch.Tensor) -> torch.Tensor | None:
     buffer (as autograd leaves them after a first backward, which stores the
     row views of the GEMM output), and no gradient hooks on the parameters
     (their AccumulateGrad step is what the in-place accumulation skips).
-    None otherwise."""
+    None otherwise, and where the buffer is not 16-byte aligned, as the GEMM's
+    epilogue needs it (gradients that are views into a flat buffer)."""
     if not _accumulate_in_gemm:
         return None
     gs = []
@@ -200,7 +201,8 @@ def grad_target(*params: torch.Tensor) -> torch.Tensor | None:
                 or p._backward_hooks or getattr(p, "_post_accumulate_grad_hooks", None)):
             return None
         gs.append(g)
-    return packed(*gs)
+    target = packed(*gs)
+    return target if target is not None and target.data_ptr() % 16 == 0 else None
 
 
 class _WgradStream:
@@ -381,7 +383,7 @@ def _one_call_backward(call, x: torch.Tensor, dout: torch.Tensor, shp: LayerShap
                                    (_lib.FH_LAYER_DWGU, (wg, wu), 2 * shp.ffn, shp.hidden),
                                    (_lib.FH_LAYER_DWD, (wd,), shp.hidden, shp.ffn)):
         g = grad_target(*group)
-        if g is not None and g.data_ptr() % 16 == 0:
+        if g is not None:
             accumulate |= bit
         else:
             g = torch.empty(rows, cols, dtype=x.dtype, device=x.device)

@@ -215,6 +215,25 @@ def test_library_validates_arguments_on_host():
     assert L.fh_gemm_bf16_workspace_size(_lib.FH_GEMM_NT, 64, 64, 96) == 0
 
 
+def test_gradients_accumulate_in_the_gemm_only_where_it_can_write_them():
+    """grad_target: adjacent bf16 gradients as one tensor, none where the buffer is not
+    16-byte aligned (the GEMM refuses such an output; autograd adds into it)."""
+    import torch
+
+    from femtotron_amd.fused_layer import grad_target
+    flat = torch.zeros(3 * 64 + 8, dtype=torch.bfloat16)
+    assert flat.data_ptr() % 16 == 0
+    ps = [torch.nn.Parameter(torch.zeros(8, 8, dtype=torch.bfloat16)) for _ in range(3)]
+    for shift in (0, 1, 4, 8):
+        for i, p in enumerate(ps):
+            p.grad = flat[shift + 64 * i:shift + 64 * (i + 1)].view(8, 8)
+        got = grad_target(*ps)
+        if shift % 8:
+            assert got is None
+        else:
+            assert got.shape == (24, 8) and got.data_ptr() == ps[0].grad.data_ptr()
+
+
 def _group_workspace(shapes, k):
     from femtotron_amd import _lib
     probs = (_lib.FhGemmProblem * len(shapes))()

@@ -358,3 +358,42 @@ def test_gradient_accumulation_in_the_gemm_equals_autograds(packed):
                            position_embeddings=(cos, sin)).backward(
         randn((1, 128, c["hidden"]), 6).to(DEV, torch.bfloat16))
     assert torch.equal(wo.grad, ref[0].self_attn.o_proj.weight.grad)
+
+
+@pytest.mark.parametrize("one_call", [True, False], ids=["one_call", "op_by_op"])
+@pytest.mark.parametrize("T", [128, 333])
+def test_a_gradient_buffer_that_is_not_aligned_is_left_to_autograd(monkeypatch, T, one_call):
+    """.grad tensors that are views at an odd element of a flat buffer (the GEMM's epilogue writes 16-byte rows):
+    autograd adds into them, the bits of an aligned gradient's, in the layer, the MLP and the attention alone."""
+    from femtotron_amd import fuse_attention, fused_layer
+    c, bf = CFG3, torch.bfloat16
+    hd = c["hidden"] // c["heads"]
+    cos, sin = ot.rope_cos_sin(T, hd, c["theta"], bf, device=DEV)
+    if not one_call:
+        monkeypatch.setattr(fused_layer, "ONE_CALL_MAX_BYTES", 0)
+
+    def run(shift, part):
+        layer = _stack(c, 1, 710, True)[0]
+        for names in (("q", "k", "v"), ("o",), ("gate", "up"), ("down",)):
+            ws = [getattr(layer.self_attn if n in "qkvo" else layer.mlp, n + "_proj").weight for n in names]
+            flat = torch.zeros(sum(w.numel() for w in ws) + 8, device=DEV, dtype=bf)
+            at = shift
+            for w in ws:
+                w.grad = flat[at:at + w.numel()].view(w.shape).fill_(0.25)
+                at += w.numel()
+                assert w.grad.data_ptr() % 16 == 2 * shift
+        for i in range(2):
+            x = randn((1, T, c["hidden"]), 5 + i).to(DEV, bf).requires_grad_(True)
+            if part == "attention":
+                fuse_attention(layer)
+                y, _ = layer.self_attn(hidden_states=x, position_embeddings=(cos, sin), attention_mask=None)
+            elif part == "mlp":
+                y = _wrapped(layer.mlp, True)(x)
+            else:
+                y = _wrapped(layer, True)(x, attention_mask=None, position_embeddings=(cos, sin))
+            y.backward(randn((1, T, c["hidden"]), 15 + i).to(DEV, bf))
+        return [p.grad.clone() for p in layer.parameters() if p.grad is not None]
+
+    for part in ("layer", "mlp", "attention") if not one_call else ("layer",):
+        for a, b in zip(run(0, part), run(1, part)):
+            assert torch.equal(a, b)
