@@ -363,14 +363,16 @@ def _one_call(x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, shp: LayerS
     if dout is not None and (dout.dtype != x.dtype or dout.device != x.device or dout.shape != x.shape
                              or dout.data_ptr() % 16):
         return None
-    wq, wk, wv, wo, wg, wu, wd, w1, w2 = w
-    call = ops.layer_args(B, S, shp, x, cos, sin, _cat_rows(wq, wk, wv), wo, _cat_rows(wg, wu), wd, w1, w2)
-    if call is None:
+    args = ops.layer_args(B, S, shp, x.dtype)
+    if args is None:
         return None
-    nbytes = ops.layer_workspace_size(call[0], dout is not None)
+    # The size before the operands: weights that are not packed are copied together.
+    nbytes = ops.layer_workspace_size(args, dout is not None)
     if nbytes == 0 or nbytes > ONE_CALL_MAX_BYTES:
         return None
-    return call[0], nbytes, call[1]
+    wq, wk, wv, wo, wg, wu, wd, w1, w2 = w
+    alive = ops.layer_operands(args, shp, x, cos, sin, _cat_rows(wq, wk, wv), wo, _cat_rows(wg, wu), wd, w1, w2)
+    return None if alive is None else (args, nbytes, alive)
 
 
 def _one_call_backward(call, x: torch.Tensor, dout: torch.Tensor, shp: LayerShape, w: tuple):

@@ -370,27 +370,36 @@ def embedding_bwd(dy: torch.Tensor, ids: torch.Tensor, vocab: int,
 
 
 # ------------------------------------------------------------- decoder layer
-def layer_args(batch: int, seq_len: int, shp, x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, *ws: torch.Tensor):
-    """(fh_layer argument block, the tensors it points into) of a layer of shape
-    `shp` (fused_layer.LayerShape) and weights wqkv, wo, wgu, wd, w1, w2; None
-    where an operand is not what the layer calls take: x's device and dtype,
-    contiguous, 16-byte aligned, of the shape's sizes.  The block holds raw
-    pointers: the caller keeps the tensors alive and uses it at once."""
+def layer_args(batch: int, seq_len: int, shp, dtype: torch.dtype) -> _lib.FhLayer | None:
+    """The sizes of an fh_layer argument block, of a layer of shape `shp`
+    (fused_layer.LayerShape), which layer_workspace_size reads; None for a dtype
+    that the layer calls do not take.  layer_operands adds the pointers."""
+    if dtype not in _DT:
+        return None
+    return _lib.FhLayer(_DT[dtype], 0, batch, seq_len, shp.hidden, shp.n_heads, shp.n_kv_heads, shp.head_dim, shp.ffn,
+                        shp.eps1, shp.eps2, shp.scale)
+
+
+def layer_operands(args: _lib.FhLayer, shp, x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, *ws: torch.Tensor):
+    """Points the block of layer_args at the operands of x's layer, with weights
+    wqkv, wo, wgu, wd, w1, w2, and returns the tensors that it then points into;
+    None where an operand is not what the layer calls take: x's device and dtype,
+    contiguous, 16-byte aligned, of the shape's sizes.  The caller keeps the
+    tensors alive and uses the block at once."""
     H, hq, F_ = shp.hidden, shp.hq, shp.ffn
     sizes = ((hq + 2 * shp.hkv, H), (H, hq), (2 * F_, H), (H, F_), (H,), (H,))
     dt, dev = x.dtype, x.device
     for w, size in zip(ws, sizes):
         if w.dtype != dt or w.device != dev or w.shape != size or not w.is_contiguous() or w.data_ptr() % 16:
             return None
-    if not x.is_cuda or dt not in _DT or not x.is_contiguous() or x.data_ptr() % 16:
+    if not x.is_cuda or not x.is_contiguous() or x.data_ptr() % 16:
         return None
     if not cos.dtype == sin.dtype == dt or not cos.device == sin.device == dev:
         return None
-    cos2, sin2, per_token = _rope_tables("layer", cos, sin, shp.head_dim, seq_len, batch * seq_len)
-    args = _lib.FhLayer(_DT[dt], per_token, batch, seq_len, H, shp.n_heads, shp.n_kv_heads, shp.head_dim, F_,
-                        shp.eps1, shp.eps2, shp.scale, 0.0, cos2.data_ptr(), sin2.data_ptr(),
-                        *(w.data_ptr() for w in ws))
-    return args, (cos2, sin2, *ws)
+    cos2, sin2, per_token = _rope_tables("layer", cos, sin, shp.head_dim, args.seq_len, args.batch * args.seq_len)
+    args.cos_per_token, args.cos, args.sin = per_token, cos2.data_ptr(), sin2.data_ptr()
+    args.wqkv, args.wo, args.wgu, args.wd, args.w1, args.w2 = (w.data_ptr() for w in ws)
+    return (cos2, sin2, *ws)
 
 
 def layer_workspace_size(args: _lib.FhLayer, backward: bool) -> int:
@@ -398,7 +407,7 @@ def layer_workspace_size(args: _lib.FhLayer, backward: bool) -> int:
 
 
 def layer_fwd(args: _lib.FhLayer, nbytes: int, x: torch.Tensor) -> torch.Tensor:
-    """fh_layer_fwd on the x of layer_args, with a workspace of nbytes."""
+    """fh_layer_fwd on the x of layer_operands, with a workspace of nbytes."""
     out = torch.empty_like(x)
     ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
     _lib.call("fh_layer_fwd", ctypes.byref(args), x.data_ptr(), out.data_ptr(), ws.data_ptr(), _stream(x))

@@ -256,6 +256,28 @@ def test_a_group_in_small_tiles_asks_for_no_workspace():
     assert _lib.lib().fh_layer_workspace_size(ctypes.byref(layer), 1) < 40 << 20
 
 
+def test_one_call_layer_copies_no_weights_before_its_size_fits(monkeypatch):
+    """Weights that are not packed are copied together for the one-call layer only once
+    its workspace is known to fit: a layer of 1500 tokens (2048 wide) whose intermediates
+    pass the first estimate and whose workspace does not."""
+    import torch
+
+    from femtotron_amd import _lib, fused_layer
+    if not _lib.LIB_PATH.exists():
+        pytest.skip("libfemtohip.so not built")
+    copies = []
+    monkeypatch.setattr(fused_layer, "_cat_rows", lambda *ws: copies.append(len(ws)) or torch.cat(ws))
+    shp = fused_layer.LayerShape(2048, 32, 4, 64, 5632, 1e-5, 1e-5, 0.125)
+    T, bf = 1500, torch.bfloat16
+    x, table = torch.empty(1, T, 2048, dtype=bf), torch.empty(1, T, 64, dtype=bf)
+    rows = ((2048, 2048), (256, 2048), (256, 2048), (2048, 2048), (5632, 2048), (5632, 2048), (2048, 5632), (2048,), (2048,))
+    w = tuple(torch.empty(*r, dtype=bf) for r in rows)
+    assert T * (4 * 2048 + 3 * 5632) * 2 < fused_layer.ONE_CALL_MAX_BYTES
+    assert fused_layer._one_call(x, table, table, shp, w, x) is None and copies == []
+    # a size that fits reaches the operands, which the layer calls do not take from host memory
+    assert fused_layer._one_call(x[:, :256], table[:, :256], table[:, :256], shp, w) is None and copies == [3, 2]
+
+
 def test_linear_weight_accepts_tensor_parallel_wrappers_at_world_size_1():
     """The dispatcher takes femtotron's Column/RowParallelLinear at one rank
     (tensor_parallel/linear.py:42-64, 170-191: weight, bias, world_size,
