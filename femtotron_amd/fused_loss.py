@@ -9,9 +9,9 @@ Reference loss head (femtotron/model/llama.py:91-111, femtotron/model/base.py:20
 It materialises the logits in the model dtype and twice more in fp32 (the
 ``.float()`` copy and the log-softmax), ~0.38 MB per token at V = 32000, which
 is the largest activation term of a checkpointed step.  Here the rows are
-processed in chunks of at most 1 GiB of logits: per chunk one GEMM
-forms the logits, ``fh_ce_fwd_bwd`` computes the fp32 row losses and overwrites
-the chunk with its gradient (softmax - onehot) / n_valid in the model dtype (the
+processed in chunks of 256 MB of logits (more where that needs no more memory,
+CHUNK_BYTES below): per chunk one GEMM forms the logits, ``fh_ce_fwd_bwd``
+computes the fp32 row losses and overwrites the chunk with its gradient (softmax - onehot) / n_valid in the model dtype (the
 rounding point of the reference's ``.float()`` backward), and two GEMMs turn it
 into the chunk's input gradient (dlogits @ W, in the model dtype like the
 reference) and its weight-gradient contribution (dlogits^T @ hidden,
@@ -29,18 +29,22 @@ from __future__ import annotations
 import torch
 
 from . import ops
-from .projections import _choose_hand
+from .projections import _choose_hand, gemm_policy
 
 IGNORE_INDEX = -100
-# Logits bytes per chunk.  Each chunk past the first reads and each before the
-# last writes the fp32 sum of the weight gradient (8 bytes per weight: a third to
-# half of that product's own time at 256 MB of a 32000- or 128256-token vocabulary),
-# and a single chunk needs no sum, which at 4 bytes per weight is itself the
-# larger part of the head's memory for a large vocabulary.  Forward and backward
-# in chunks of 256 MB, 512 MB and 1 GB: 16384 x 2048 hidden states and a vocabulary of
-# 32000 5582, 5219 and 5023 us with a peak of 766, 751 and 1001 MB; 8192 x 4096 and
-# 128256 27.7, 23.0 and 20.4 ms, 3320, 2505 and 3006 MB.
-CHUNK_BYTES = 1 << 30
+# Logits bytes per chunk, at least.  Beside them lies the fp32 sum of the weight
+# gradient (twice W, the bf16 gradient's bytes), from the first chunk to the last: the
+# head takes 2 W + CHUNK_BYTES, or the 3 W of rounding the sum where that is more, and
+# the products' K slices (64 MB at most here).  In that room (_chunk_rows) a chunk
+# grows to W for a large vocabulary, and one chunk takes all rows where their logits
+# and the gradient alone, with no sum, fit: each chunk past the first reads and each
+# before the last writes the sum, a third to half of that product's own time at 256
+# MB.  Forward and backward, and the peak over the inputs: 16384 x 2048 hidden states
+# and a vocabulary of 32000 5.71 ms and 628 MiB (in one chunk 5.06 and 1189; library
+# products in 256 MB chunks 6.21 and 564), 4096 x 2048 and 32000 1.46 and 391 (library
+# 1.73 and 516), 8192 x 4096 and 128256 19.4 and 3070, in one chunk (library 34.3 and
+# 3070; in 1 GiB chunks with the sum 20.3 and 4072).
+CHUNK_BYTES = 256 << 20
 # The logits run hand-written up to this width, where a tile is few stages long:
 # 16384 x 32000 352 us against the library's 426 at 256 wide, 508 against 613 at
 # 512, 848 against 842 at 1024, and 1544 against 1497 at 2048.
@@ -78,17 +82,40 @@ def _input_grad(dlogits: torch.Tensor, weight: torch.Tensor, out: torch.Tensor) 
         torch.mm(dlogits, weight, out=out)
 
 
-def _weight_grad(dlogits: torch.Tensor, x_c: torch.Tensor, dw32: torch.Tensor | None, first: bool, last: bool):
+def _peak_bytes(weight: torch.Tensor) -> int:
+    """Bytes that the logits, the fp32 sum and the bf16 gradient may take together."""
+    w = weight.numel() * weight.element_size()
+    return max(2 * w + CHUNK_BYTES, 3 * w)
+
+
+def _chunk_rows(hidden2: torch.Tensor, weight: torch.Tensor, need_dw: bool) -> int:
+    """Rows per chunk (CHUNK_BYTES above)."""
+    N, H = hidden2.shape
+    row = weight.size(0) * weight.element_size()
+    w = row * H
+    sums = need_dw and weight.dtype == torch.bfloat16  # fp32: the sum is the gradient itself
+    # One chunk needs no sum if its product runs hand-written.
+    if (sums and gemm_policy() == "hand" and N >= 64 and H % 8 == 0 and hidden2.data_ptr() % 16 == 0
+            and w + N * row <= _peak_bytes(weight)):
+        return N
+    return max(256, max(CHUNK_BYTES, w if sums else 0) // row // 256 * 256)
+
+
+def _weight_grad(dlogits: torch.Tensor, x_c: torch.Tensor, dw32: torch.Tensor | None, first: bool, last: bool,
+                 peak: int):
     """(dw or None, the running fp32 sum or None) after this chunk: dw appears
-    with the last one.  A chunk that does not run hand-written (fp32, a width that is
-    no multiple of 8, fewer than 64 rows) leaves the rounding to the caller."""
+    with the last one.  A last chunk that does not run hand-written (fp32, a width
+    that is no multiple of 8, fewer than 64 rows), or leaves no room for dw beside
+    its logits, leaves the rounding to the caller."""
     V, H = dlogits.size(1), x_c.size(1)
     if _choose_hand("tn", dlogits, x_c):
         if first and last:
             return ops.gemm("tn", dlogits, x_c, any_k=True), None
-        dw = torch.empty(V, H, dtype=x_c.dtype, device=x_c.device) if last else None
+        dw = None
         if first:
             dw32 = torch.empty(V, H, dtype=torch.float32, device=x_c.device)
+        elif last and 6 * dw32.numel() + 2 * dlogits.numel() <= peak:
+            dw = torch.empty(V, H, dtype=x_c.dtype, device=x_c.device)
         ops.gemm_acc(dlogits, x_c, dw32, add=not first, out=dw)
         return dw, dw32
     if first:
@@ -115,7 +142,7 @@ class FusedLinearCrossEntropy(torch.autograd.Function):
         dx = torch.empty_like(hidden2) if need_dx else None
         dw = dw32 = None
         loss_sum = torch.zeros((), dtype=torch.float32, device=dev)
-        chunk = max(256, (CHUNK_BYTES // (V * hidden2.element_size())) // 256 * 256)
+        chunk = _chunk_rows(hidden2, weight, need_dw)
         for r0 in range(0, N, chunk):
             r1 = min(N, r0 + chunk)
             x_c = hidden2[r0:r1]
@@ -125,7 +152,7 @@ class FusedLinearCrossEntropy(torch.autograd.Function):
             if need_dx:
                 _input_grad(logits, weight, dx[r0:r1])
             if need_dw:
-                dw, dw32 = _weight_grad(logits, x_c, dw32, r0 == 0, r1 == N)
+                dw, dw32 = _weight_grad(logits, x_c, dw32, r0 == 0, r1 == N, _peak_bytes(weight))
             del logits
         if need_dw and dw is None:  # no rows, or the library's last chunk
             dw = torch.zeros_like(weight) if dw32 is None else dw32.to(weight.dtype)

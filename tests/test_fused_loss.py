@@ -145,8 +145,8 @@ def test_fused_loss_bf16_matches_stock_loss_head():
     apply_activation_checkpointing(model, get_ac_policy("llama_decoder_layer"), checkpoint_fn=fused_checkpoint)
     ids = torch.randint(0, CFG3["vocab"], (2, 1024), generator=torch.Generator().manual_seed(7)).to(DEV)
     res = []
-    old = fl.CHUNK_BYTES
-    fl.CHUNK_BYTES = 64 << 20  # 1024 rows per chunk at V = 32000: exercise chunking
+    old = fl._chunk_rows
+    fl._chunk_rows = lambda *a: 1024  # exercise chunking
     try:
         for fused in (True, False):
             for p in model.parameters():
@@ -155,7 +155,7 @@ def test_fused_loss_bf16_matches_stock_loss_head():
             loss.backward()
             res.append((loss.detach().float(), {n: p.grad.float() for n, p in model.named_parameters()}))
     finally:
-        fl.CHUNK_BYTES = old
+        fl._chunk_rows = old
     (lf, gf), (lr, gr) = res
     assert abs(lf.item() - lr.item()) <= 1e-3 * abs(lr.item())
     for n in gr:
@@ -200,7 +200,7 @@ def test_loss_head_in_chunks_matches_fp64(monkeypatch, dtype, N, H, V, rows):
     """Loss and both gradients against fp64 with the logits and their gradient rounded where the head rounds them:
     every product sums in fp32 and rounds once, so only those roundings and the output's are left (bf16 2^-8 each)."""
     import femtotron_amd.fused_loss as fl
-    monkeypatch.setattr(fl, "CHUNK_BYTES", rows * V * dtype.itemsize)
+    monkeypatch.setattr(fl, "_chunk_rows", lambda *a: rows)
     g = torch.Generator().manual_seed(N + H)
     x = torch.randn(N, H, generator=g).to(dtype).to(DEV).requires_grad_(True)
     w = (torch.randn(V, H, generator=g) * H ** -0.5).to(dtype).to(DEV).requires_grad_(True)
@@ -215,3 +215,27 @@ def test_loss_head_in_chunks_matches_fp64(monkeypatch, dtype, N, H, V, rows):
     assert abs(loss.item() - want.item()) <= tol * abs(want.item())
     for got, ref in ((x.grad, x64.grad), (w.grad, w64.grad)):
         assert float((got.double() - ref).norm() / ref.norm()) < tol
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N,H,V", [(16384, 256, 32000),   # the logits, 1000 MiB, are the larger part
+                                   (9000, 2048, 32000),   # two chunks and a remainder
+                                   (8192, 1024, 32000),   # all rows in one chunk would not fit, by little
+                                   (1100, 1024, 128256)])  # one chunk, no sum
+def test_loss_head_peak_memory(N, H, V):
+    """Peak of the bf16 head over its inputs: the input gradient, the fp32 sum of the weight gradient and 256 MB of
+    logits, or the sum and the gradient it is rounded to where those are more, and the K slices of a product."""
+    import femtotron_amd.fused_loss as fl
+    g = torch.Generator(device=DEV).manual_seed(N)
+    x = torch.randn(1, N, H, device=DEV, generator=g).bfloat16().requires_grad_(True)
+    w = (torch.randn(V, H, device=DEV, generator=g) * 0.02).bfloat16().requires_grad_(True)
+    labels = torch.randint(0, V, (1, N), device=DEV, generator=g)
+    for _ in range(2):  # the second step finds the library's own workspace there
+        x.grad = w.grad = None
+        torch.cuda.synchronize()
+        torch.cuda.reset_peak_memory_stats()
+        base = torch.cuda.memory_allocated()
+        fl.fused_causal_lm_loss(x, w, labels).backward()
+    peak = torch.cuda.max_memory_allocated() - base
+    room = 2 * N * H + max(4 * V * H + (256 << 20), 6 * V * H) + (64 << 20)
+    assert peak <= room + (4 << 20), f"{peak / 2**20:.0f} MiB, {room / 2**20:.0f} MiB expected"
