@@ -1583,16 +1583,39 @@ size_t split_offset(int64_t batch, int64_t seq_len, int64_t n_heads) {
 // of LDS), two of the head_dim-128 kernel.
 constexpr int64_t kDkdvBlocks = 256;
 
-// The smallest split of the group's heads (a divisor of the group) that gives
-// `want` workgroups, or the largest that the workspace holds.
-int head_split(int64_t blocks, int64_t want, int64_t group, int64_t floats_per_split, size_t room) {
+// Key blocks of a sequence in the dK/dV kernels, and the floats of one part's sums.
+int64_t dkdv_key_blocks(int64_t seq_len, int64_t head_dim) {
+  const int64_t keys = head_dim <= 64 ? DkdvFusedTiles<64>::NWH * 32 : DkdvTiles<128>::NKS * 32;
+  return (seq_len + keys - 1) / keys;
+}
+int64_t split_part_floats(int64_t batch, int64_t seq_len, int64_t n_kv_heads, int64_t head_dim) {
+  return 2 * batch * seq_len * n_kv_heads * head_dim;
+}
+
+// Workgroups that a kv head's query heads are split over in the bf16 backward (1:
+// no split): the smallest divisor of the group that fills the chip, or the largest
+// whose sums the workspace holds.
+int head_split(int64_t batch, int64_t seq_len, int64_t n_heads, int64_t n_kv_heads, int64_t head_dim) {
+  const int64_t nkb = dkdv_key_blocks(seq_len, head_dim), group = n_heads / n_kv_heads;
+  const int64_t blocks = (head_dim <= 64 ? (nkb + 1) / 2 : nkb) * batch * n_kv_heads;
+  const int64_t want = head_dim <= 64 ? kDkdvBlocks : 2 * kDkdvBlocks;
+  const int64_t part = split_part_floats(batch, seq_len, n_kv_heads, head_dim);
+  const int64_t room = static_cast<int64_t>(split_floats(batch, seq_len, n_heads));
   int64_t n = 1;
   for (int64_t d = 2; d <= group && blocks * n < want; ++d)
-    if (group % d == 0 && d * floats_per_split <= static_cast<int64_t>(room)) n = d;
+    if (group % d == 0 && d * part <= room) n = d;
   return static_cast<int>(n);
 }
 
 }  // namespace
+
+extern "C" size_t fh_attn_bwd_call_workspace_size(fh_dtype dt, int64_t batch, int64_t seq_len, int64_t n_heads,
+                                                  int64_t n_kv_heads, int64_t head_dim) {
+  if (batch <= 0 || seq_len <= 0 || check_dims(dt, Dims{batch, seq_len, n_heads, n_kv_heads, head_dim})) return 0;
+  const int n = dt == FH_BF16 ? head_split(batch, seq_len, n_heads, n_kv_heads, head_dim) : 1;
+  const size_t parts = n > 1 ? static_cast<size_t>(n) * split_part_floats(batch, seq_len, n_kv_heads, head_dim) : 0;
+  return (split_offset(batch, seq_len, n_heads) + parts) * sizeof(float);
+}
 
 extern "C" size_t fh_attn_bwd_workspace_size(int64_t batch, int64_t seq_len, int64_t n_heads) {
   if (batch <= 0 || seq_len <= 0 || n_heads <= 0) return 0;
@@ -1734,23 +1757,21 @@ int attn_bwd_impl(fh_dtype dt, const void* q, int64_t ldq, const void* k, int64_
       const auto kdk = static_cast<uint16_t*>(dk);
       const auto kdv = static_cast<uint16_t*>(dv);
       // Few workgroups: the group's heads split over several (HeadSplit).
-      const int64_t per_split = 2 * batch * seq_len * n_kv_heads * HD, kvb = batch * n_kv_heads;
-      const size_t room = split_floats(batch, seq_len, n_heads);
-      HeadSplit hs{delta + split_offset(batch, seq_len, n_heads), 1};
+      const int64_t kvb = batch * n_kv_heads, nkb = dkdv_key_blocks(seq_len, HD);
+      const HeadSplit hs{delta + split_offset(batch, seq_len, n_heads),
+                         head_split(batch, seq_len, n_heads, n_kv_heads, HD)};
       if constexpr (HD <= 64) {
         using DT = DkdvFusedTiles<HD>;
-        const int64_t nkb = (seq_len + DT::NWH * 32 - 1) / (DT::NWH * 32), pairs = (nkb + 1) / 2;
-        hs.n = head_split(pairs * kvb, kDkdvBlocks, group, per_split, room);
+        static_assert(DT::NWH == DkdvFusedTiles<64>::NWH, "dkdv_key_blocks");
         // One key block per workgroup where all of them still run at once.
         const bool paired = nkb * kvb * hs.n > kDkdvBlocks;
-        const dim3 gk(static_cast<unsigned>(paired ? pairs : nkb), static_cast<unsigned>(kvb * hs.n));
+        const dim3 gk(static_cast<unsigned>(paired ? (nkb + 1) / 2 : nkb), static_cast<unsigned>(kvb * hs.n));
         hipLaunchKernelGGL((k_attn_bwd_dkdv_fused<HD>), gk, dim3(DT::NT), 0, stream, kq, ldq, kk,
                            ldk, kvp, ldv, kg, lddo, nl2, delta, kdk, lddk, kdv, lddv, S, nh, nkv,
                            group, scale * kLog2e, scale, rb, hs, paired);
       } else {
         using DT = DkdvTiles<HD>;
-        const int64_t nkb = (seq_len + DT::NKS * 32 - 1) / (DT::NKS * 32);
-        hs.n = head_split(nkb * kvb, 2 * kDkdvBlocks, group, per_split, room);
+        static_assert(DT::NKS == DkdvTiles<128>::NKS, "dkdv_key_blocks");
         const dim3 gk(static_cast<unsigned>(nkb), static_cast<unsigned>(kvb * hs.n));
         hipLaunchKernelGGL((k_attn_bwd_dkdv<HD>), gk, dim3(DT::NT), 0, stream, kq, ldq, kk, ldk,
                            kvp, ldv, kg, lddo, nl2, delta, kdk, lddk, kdv, lddv, S, nh, nkv, group,

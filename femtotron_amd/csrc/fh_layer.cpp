@@ -124,7 +124,7 @@ BwdPlan bwd_plan(const fh_layer& l) {
     ws = std::max(ws, fh_gemm_bf16_grouped_any_k_workspace_size(FH_GEMM_TN, 3, g, z.T));
   }
   ws = std::max(ws, fh_rmsnorm_bwd_workspace_size(z.T, z.H));
-  ws = std::max(ws, fh_attn_bwd_workspace_size(l.batch, l.seq_len, l.n_heads));
+  ws = std::max(ws, fh_attn_bwd_call_workspace_size(l.dt, l.batch, l.seq_len, l.n_heads, l.n_kv_heads, l.head_dim));
   b.ws = ar.take(ws);
   b.total = ar.at;
   return b;

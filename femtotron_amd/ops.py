@@ -287,7 +287,7 @@ def attn_bwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: torch.Tensor,
     _same_dtype(q, k, v, o, dout, dq, dk, dv)
     if lse.dtype != torch.float32 or not lse.is_contiguous() or lse.numel() != batch * n_heads * seq_len:
         raise ValueError("attn_bwd: lse must be contiguous fp32 [batch, n_heads, seq_len]")
-    ws_bytes = _lib.lib().fh_attn_bwd_workspace_size(batch, seq_len, n_heads)
+    ws_bytes = _lib.lib().fh_attn_bwd_call_workspace_size(_dtype_code(q), batch, seq_len, n_heads, n_kv_heads, head_dim)
     ws = torch.empty(max(ws_bytes, 4) // 4, dtype=torch.float32, device=q.device)
     args = (_dtype_code(q), _ptr(q), _rowmajor(q, "q"), _ptr(k), _rowmajor(k, "k"),
             _ptr(v), _rowmajor(v, "v"), _ptr(o), _rowmajor(o, "o"), _ptr(dout),

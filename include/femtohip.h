@@ -213,8 +213,12 @@ int fh_attn_fwd_rope(fh_dtype dt, const void* q, int64_t ldq, const void* k, int
                      const void* sin, int cos_per_token, hipStream_t stream);
 
 /* Bytes of workspace fh_attn_bwd needs: per query, fp32, rowsum(dO*O) and the
- * lse in log2 units; for short batches also the fp32 partial sums of dK and dV
- * over parts of a kv head's query heads (at most 32 MB). */
+ * lse in log2 units; for short FH_BF16 batches with grouped kv heads also the fp32
+ * partial sums of dK and dV over parts of a kv head's query heads (at most 32 MB).
+ * _call_: what one call of these sizes needs (0 for sizes it refuses); the other:
+ * enough for either dtype and any number of kv heads. */
+size_t fh_attn_bwd_call_workspace_size(fh_dtype dt, int64_t batch, int64_t seq_len, int64_t n_heads,
+                                       int64_t n_kv_heads, int64_t head_dim);
 size_t fh_attn_bwd_workspace_size(int64_t batch, int64_t seq_len, int64_t n_heads);
 
 /* Gradients of fh_attn_fwd given o, lse and dout: writes dq, dk, dv (each

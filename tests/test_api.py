@@ -256,6 +256,27 @@ def test_a_group_in_small_tiles_asks_for_no_workspace():
     assert _lib.lib().fh_layer_workspace_size(ctypes.byref(layer), 1) < 40 << 20
 
 
+def test_attention_backward_asks_for_what_the_call_uses():
+    """fp32 and one query head per kv head never split the heads: two floats per query
+    (rounded up to 16 bytes); a split call's sums lie within the size that holds for any."""
+    from femtotron_amd import _lib
+    if not _lib.LIB_PATH.exists():
+        pytest.skip("libfemtohip.so not built")
+    L = _lib.lib()
+    call, most = L.fh_attn_bwd_call_workspace_size, L.fh_attn_bwd_workspace_size
+    for B, S in ((1, 256), (1, 333), (3, 333), (4, 512), (1, 4096)):
+        for hd in (32, 64, 128):
+            least = -(-2 * B * S * 32 // 4) * 16
+            assert call(_lib.FH_F32, B, S, 32, 4, hd) == least
+            assert call(_lib.FH_BF16, B, S, 32, 32, hd) == least
+            for nkv in (1, 4, 16):
+                got = call(_lib.FH_BF16, B, S, 32, nkv, hd)
+                assert least <= got <= most(B, S, 32)
+                assert (got - least) % (2 * B * S * nkv * hd * 4) == 0
+    assert call(_lib.FH_BF16, 1, 256, 32, 4, 64) > most(1, 4096, 32) // 16  # split
+    assert call(_lib.FH_BF16, 1, 256, 32, 5, 64) == call(_lib.FH_BF16, 1, 256, 32, 4, 48) == 0
+
+
 def test_one_call_layer_copies_no_weights_before_its_size_fits(monkeypatch):
     """Weights that are not packed are copied together for the one-call layer only once
     its workspace is known to fit: a layer of 1500 tokens (2048 wide) whose intermediates
