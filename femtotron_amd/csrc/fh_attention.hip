@@ -1594,7 +1594,12 @@ int64_t split_part_floats(int64_t batch, int64_t seq_len, int64_t n_kv_heads, in
 
 // Workgroups that a kv head's query heads are split over in the bf16 backward (1:
 // no split): the smallest divisor of the group that fills the chip, or the largest
-// whose sums the workspace holds.
+// whose sums the workspace holds, if that is worth adding the sums: the items (query
+// tile and head) of the first key block that a workgroup is spared, against a launch,
+// its loop over the parts and their bytes (microseconds, fitted to 173 sizes of four
+// head counts, 1 to 8 sequences of 16 to 4096 tokens; dQ included).  Split without
+// this test, the shortest lost to a workgroup per kv head: 1 x 16 tokens, 8 / 4 heads
+// of 32 8.7 -> 13.2 us, 8 x 64 9.3 -> 11.9, 8 x 64, 32 / 4 heads of 64 17.5 -> 20.6.
 int head_split(int64_t batch, int64_t seq_len, int64_t n_heads, int64_t n_kv_heads, int64_t head_dim) {
   const int64_t nkb = dkdv_key_blocks(seq_len, head_dim), group = n_heads / n_kv_heads;
   const int64_t blocks = (head_dim <= 64 ? (nkb + 1) / 2 : nkb) * batch * n_kv_heads;
@@ -1604,7 +1609,10 @@ int head_split(int64_t batch, int64_t seq_len, int64_t n_heads, int64_t n_kv_hea
   int64_t n = 1;
   for (int64_t d = 2; d <= group && blocks * n < want; ++d)
     if (group % d == 0 && d * part <= room) n = d;
-  return static_cast<int>(n);
+  const int64_t tile = head_dim <= 64 ? DkdvFusedTiles<64>::BQ : DkdvTiles<128>::BQ;
+  const double items = static_cast<double>(group * ((seq_len + tile - 1) / tile)) * (1.0 - 1.0 / static_cast<double>(n));
+  const double sums = 2.9 + 0.5 * static_cast<double>(n) + 1.6e-6 * static_cast<double>(n * part);
+  return (head_dim <= 64 ? 1.1 : 1.28) * items > sums ? static_cast<int>(n) : 1;
 }
 
 }  // namespace

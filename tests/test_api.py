@@ -274,6 +274,11 @@ def test_attention_backward_asks_for_what_the_call_uses():
                 assert least <= got <= most(B, S, 32)
                 assert (got - least) % (2 * B * S * nkv * hd * 4) == 0
     assert call(_lib.FH_BF16, 1, 256, 32, 4, 64) > most(1, 4096, 32) // 16  # split
+    for B, S, nh, nkv, hd in ((1, 16, 8, 4, 32), (8, 64, 8, 4, 32), (8, 64, 32, 4, 64), (8, 64, 32, 8, 128)):
+        # a few items per workgroup: their sums would take longer than they do
+        assert call(_lib.FH_BF16, B, S, nh, nkv, hd) == -(-2 * B * S * nh // 4) * 16
+    for B, S, nh, nkv, hd in ((1, 161, 3, 1, 64), (1, 61, 5, 1, 128), (2, 129, 6, 1, 32), (1, 333, 32, 8, 128)):
+        assert call(_lib.FH_BF16, B, S, nh, nkv, hd) > -(-2 * B * S * nh // 4) * 16
     assert call(_lib.FH_BF16, 1, 256, 32, 5, 64) == call(_lib.FH_BF16, 1, 256, 32, 4, 48) == 0
 
 
