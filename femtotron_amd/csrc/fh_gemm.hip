@@ -1262,9 +1262,13 @@ void launch_persist(int op, const GemmArgs& g, hipStream_t stream) {
 template <bool A_KO, bool B_KO, bool RAGGED>
 void launch_mid(const GemmArgs& g, unsigned blocks, bool partial, hipStream_t stream) {
   const dim3 grid(blocks), block(256);
-  if (g.grouped)
-    hipLaunchKernelGGL((k_gemm_mid<A_KO, B_KO, EPI_GROUP, RAGGED>), grid, block, 0, stream, g);
-  else if (mid_deep(g.grid, g.steps_per_slice, g.m, g.n, g.total_steps)) {
+  if constexpr (A_KO && B_KO) {  // groups of small tiles are weight gradients (group_form)
+    if (g.grouped) {
+      hipLaunchKernelGGL((k_gemm_mid<true, true, EPI_GROUP, RAGGED>), grid, block, 0, stream, g);
+      return;
+    }
+  }
+  if (mid_deep(g.grid, g.steps_per_slice, g.m, g.n, g.total_steps)) {
     if (partial)
       hipLaunchKernelGGL((k_gemm_deep<A_KO, B_KO, EPI_PARTIAL, RAGGED>), grid, block, kDeepLds, stream, g);
     else if (g.r != nullptr)
