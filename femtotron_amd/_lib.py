@@ -84,6 +84,7 @@ SIGNATURES: dict[str, tuple] = {
     "fh_gemm_bf16": (c_int, [c_int, _V, _I64, _V, _I64, _V, _I64, _V, _I64, _I64, _I64, _I64, _V, _V]),
     "fh_gemm_bf16_any_k_workspace_size": (c_size_t, [c_int, _I64, _I64, _I64]),
     "fh_gemm_bf16_any_k": (c_int, [c_int, _V, _I64, _V, _I64, _V, _I64, _V, _I64, _I64, _I64, _I64, _V, _V]),
+    "fh_gemm_bf16_form": (c_char_p, [c_int, _I64, _I64, _I64, c_int]),
     "fh_gemm_f32": (c_int, [c_int, _V, _I64, _V, _I64, _V, _I64, _V, _I64, _I64, _I64, _I64, _V]),
     "fh_gemm_bf16_acc": (c_int, [_V, _I64, _V, _I64, _V, c_int, _V, _I64, _I64, _I64, _I64, _V]),
     "fh_gemm_bf16_rope": (c_int, [_V, _I64, _V, _I64, _V, _I64, _I64, _I64, _I64, _I64, _I64, _I64,

@@ -1393,6 +1393,18 @@ void use_mid_tiles(GemmArgs& g) {
   g.tiles = tile0;
 }
 
+// Whether whole-K 256 x 256 tiles run in the persistent form.  With the residual
+// epilogue: the forward (NT) layout only.
+bool use_persist(int op, const GemmArgs& g, const GemmPlan& plan) {
+#if FH_GEMM_PERSIST
+  return !plan.mid && !plan.stream && plan.slices == 1 && (g.r == nullptr || op == FH_GEMM_NT) &&
+         g.rope.cos == nullptr && g.total_steps >= 2 && g.m % kTm == 0 && g.n % kTn == 0 &&
+         g.lda < (int64_t(1) << 24) && g.ldb < (int64_t(1) << 24) && g.tiles > stream_grid();
+#else
+  return false;
+#endif
+}
+
 // Launches the GEMM of g in the stream form (segment slots in `workspace`,
 // split tiles summed by k_gemm_fixup) or over the plan's K slices (partials in
 // `workspace`, summed by k_gemm_reduce, when there is more than one).
@@ -1414,17 +1426,12 @@ int gemm_run(int op, GemmArgs& g, const GemmPlan& plan, void* workspace, hipStre
     return FH_OK;
   }
   g.steps_per_slice = (g.total_steps + slices - 1) / slices;
-#if FH_GEMM_PERSIST
-  // The residual epilogue in this form: the forward (NT) layout only.
-  if (!plan.mid && slices == 1 && (g.r == nullptr || op == FH_GEMM_NT) && g.rope.cos == nullptr && g.total_steps >= 2 &&
-      g.m % kTm == 0 && g.n % kTn == 0 && g.lda < (int64_t(1) << 24) && g.ldb < (int64_t(1) << 24) &&
-      g.tiles > stream_grid()) {
+  if (use_persist(op, g, plan)) {
     g.grid = stream_grid();
     if (g.repeat > 0) launch_persist<true>(op, g, stream);
     else launch_persist<false>(op, g, stream);
     return FH_OK;
   }
-#endif
   const int64_t logical = static_cast<int64_t>(g.tiles) * slices;
   FH_REQUIRE(logical <= 0x7ffffff0, "gemm_bf16: grid too large");
   g.grid = static_cast<int>(logical);
@@ -1473,6 +1480,22 @@ extern "C" int fh_gemm_bf16_any_k(int op, const void* a, int64_t lda, const void
                                   int64_t ldc, const void* residual, int64_t ldr, int64_t m, int64_t n,
                                   int64_t k, void* workspace, hipStream_t stream) {
   return gemm_impl(op, a, lda, b, ldb, c, ldc, residual, ldr, m, n, k, true, workspace, stream, "fh_gemm_bf16_any_k");
+}
+
+extern "C" const char* fh_gemm_bf16_form(int op, int64_t m, int64_t n, int64_t k, int residual) {
+  GemmArgs g;
+  alignas(16) static const char aligned[16] = {};  // stands for the operands, which are not read
+  void* p = const_cast<char*>(aligned);
+  const int64_t pad_m = (m + 7) / 8 * 8, pad_k = (k + 7) / 8 * 8;
+  if (gemm_setup(op, p, op == FH_GEMM_TN ? pad_m : pad_k, p, op == FH_GEMM_NT ? pad_k : n, p, n, residual ? p : nullptr,
+                 n, m, n, k, true, g))
+    return nullptr;
+  const GemmPlan plan = gemm_plan(op, m, n, k);
+  if (plan.stream) return "stream";
+  if (!plan.mid) return plan.slices > 1 ? "split" : use_persist(op, g, plan) ? "persist" : "tile";
+  const int64_t tiles = ceil_div(m, kMid) * ceil_div(n, kMid), per = ceil_div(g.total_steps, plan.slices);
+  if (mid_deep(tiles * plan.slices, per, m, n, g.total_steps)) return plan.slices > 1 ? "deep split" : "deep";
+  return plan.slices > 1 ? "mid split" : "mid";
 }
 
 namespace {

@@ -391,6 +391,13 @@ int fh_gemm_bf16_any_k(int op, const void* a, int64_t lda, const void* b, int64_
                        int64_t ldc, const void* residual, int64_t ldr, int64_t m, int64_t n,
                        int64_t k, void* workspace, hipStream_t stream);
 
+/* The form in which fh_gemm_bf16_any_k (and fh_gemm_bf16) runs a product of these
+ * sizes (leading dimensions below 2^24), with or without a residual: 256 x 256 tiles
+ * as "tile", "split" (K slices), "persist" or "stream"; 128 x 128 tiles as "mid" or
+ * "mid split", with loads four stages ahead "deep" or "deep split".  NULL for sizes
+ * it refuses. */
+const char* fh_gemm_bf16_form(int op, int64_t m, int64_t n, int64_t k, int residual);
+
 /* Up to three GEMMs of one layout and one k in one launch: problem i is
  * fh_gemm_bf16(op, a, lda, b, ldb, c, ldc, residual, ldr, m, n, k) of its
  * fields, with the same roundings, requirements and residual rules.  The

@@ -213,6 +213,10 @@ def test_library_validates_arguments_on_host():
     assert L.fh_gemm_bf16_workspace_size(_lib.FH_GEMM_TN, 512, 512, 16384) > 0
     assert L.fh_gemm_bf16_workspace_size(_lib.FH_GEMM_NT, 16384, 2048, 2048) == 0
     assert L.fh_gemm_bf16_workspace_size(_lib.FH_GEMM_NT, 64, 64, 96) == 0
+    # the form of a product, from its sizes
+    assert L.fh_gemm_bf16_form(_lib.FH_GEMM_NT, 16384, 11264, 2048, 0) == b"persist"
+    assert L.fh_gemm_bf16_form(_lib.FH_GEMM_TN, 2048, 2048, 999, 1) == b"mid"
+    assert L.fh_gemm_bf16_form(_lib.FH_GEMM_NT, 64, 64, 100, 0) is None
 
 
 def test_gradients_accumulate_in_the_gemm_only_where_it_can_write_them():

@@ -272,15 +272,23 @@ def test_gemm_rejects_unsupported_operands():
         ops.gemm("nt", x, x, out=wide[:, :128])
 
 
+def _form(op, m, n, k, resid):
+    code = {"nt": _lib.FH_GEMM_NT, "nn": _lib.FH_GEMM_NN, "tn": _lib.FH_GEMM_TN}[op]
+    return _lib.lib().fh_gemm_bf16_form(code, m, n, k, int(resid)).decode()
+
+
 @pytest.mark.parametrize("op", ["nt", "nn", "tn"])
-@pytest.mark.parametrize("m,n,k,pad", [
-    (128, 128, 64, 0), (8, 128, 128, 8), (136, 120, 192, 0),     # one 128 x 128 tile and its edges, one to three stages
-    (256, 11264, 2048, 0), (1000, 2048, 2048, 0),                # whole K, two workgroups on some CUs
-    (256, 2048, 5632, 0), (16, 2048, 11264, 64), (512, 264, 16384, 0),  # K slices
+@pytest.mark.parametrize("m,n,k,pad,form", [
+    (128, 128, 64, 0, "mid"), (8, 128, 128, 8, "mid"), (136, 120, 192, 0, "mid"),  # one 128 x 128 tile and its edges, one to three stages
+    (4096, 2048, 256, 0, "mid"),                                            # whole K, two workgroups per CU
+    (256, 256, 2048, 0, "mid split"), (512, 768, 2048, 8, "mid split"),     # K slices
+    (256, 11264, 2048, 0, "deep"), (1000, 2048, 2048, 0, "deep"),           # whole K, four stages ahead
+    (256, 2048, 5632, 0, "deep split"), (16, 2048, 11264, 64, "deep split"), (512, 264, 16384, 0, "deep split"),
 ])
-def test_mid_tiles_match_and_add_the_residual(op, m, n, k, pad):
+def test_mid_tiles_match_and_add_the_residual(op, m, n, k, pad, form):
     """Sizes that run in 128 x 128 tiles: the product within its bound, repeatable, the residual bit-identical to
     the rounded product plus the residual, in place too."""
+    assert _form(op, m, n, k, False) == _form(op, m, n, k, True) == form
     g = torch.Generator(device=DEV).manual_seed(m + 3 * n + 7 * k)
     a, b = _operands(op, m, n, k, g, pad)
     c = ops.gemm(op, a, b)
@@ -300,6 +308,7 @@ def test_mid_tiles_match_and_add_the_residual(op, m, n, k, pad):
 def test_mid_tiles_four_stages_ahead(op, m, n, k):
     """At most one workgroup per CU and operands past one XCD's L2: four stages in flight, slices of eight stages and
     more (the last one shorter, its last k ragged), operands followed by NaNs."""
+    assert _form(op, m, n, k, False) == _form(op, m, n, k, True) == ("deep" if n > 3000 and m > 16 else "deep split")
     g = torch.Generator(device=DEV).manual_seed(m + k)
     shapes = {"nt": ((m, k), (n, k)), "nn": ((m, k), (k, n)), "tn": ((k, m), (k, n))}[op]
     a, b = (_guarded(*s, g) for s in shapes)
@@ -347,19 +356,21 @@ def _guarded(rows, cols, g):
 @pytest.mark.parametrize("m,n,k,form", [
     # 128 x 128 tiles: two to four stages, K slices of which the last ends ragged
     (264, 520, 72, "mid"), (512, 768, 120, "mid"), (4352, 4096, 184, "mid"), (512, 768, 2056, "mid split"),
-    (128, 136, 712, "mid split"), (8, 8, 72, "mid"),
+    (128, 136, 712, "mid"), (128, 136, 1160, "mid split"), (8, 8, 72, "mid"),
     # 256 x 256 tiles
     (2000, 14336, 520, "tile"), (1000, 28672, 2056, "tile"),
     (1000, 4096, 14344, "split"), (1032, 4104, 14344, "split"),           # the last slice ends ragged
-    (8192, 4096, 1032, "persist"), (10240, 2048, 1000, "persist"),        # the next tile's stages loaded ahead
+    (8192, 4096, 1032, "persist"), (12288, 2048, 1000, "persist"),        # the next tile's stages loaded ahead
     (4104, 4088, 2056, "stream"), (10240, 2048, 4104, "stream"),          # a segment ends ragged
 ])
 @pytest.mark.parametrize("resid", [False, True])
 def test_any_k_matches_fp64_product(op, m, n, k, form, resid):
-    """k not a multiple of 64 (a multiple of 8, and for 'tn' an odd one): every form of the kernels (`form`: the
-    one that most layouts take at these sizes), operands followed by NaNs, against the fp64 product within the rounding bound; with a residual bit-identical to the
-    rounded product plus the residual."""
+    """k not a multiple of 64 (a multiple of 8, and for 'tn' an odd one): every form of the kernels, operands
+    followed by NaNs, against the fp64 product within the rounding bound; with a residual bit-identical to the
+    rounded product plus the residual (the persistent form's epilogue: 'nt' alone)."""
     for kk in ((k, k + 1, k - 7) if op == "tn" else (k,)):
+        assert _form(op, m, n, kk, False) == form
+        assert _form(op, m, n, kk, True) == ("tile" if form == "persist" and op != "nt" else form)
         g = torch.Generator(device=DEV).manual_seed(m + kk)
         shapes = {"nt": ((m, kk), (n, kk)), "nn": ((m, kk), (kk, n)), "tn": ((kk, m), (kk, n))}[op]
         a, b = (_guarded(*s, g) for s in shapes)
@@ -382,8 +393,15 @@ def test_grouped_any_k_matches_each_product(shapes, k):
     items = [(_guarded(k, m, g), _guarded(k, n, g), None, None) for m, n in shapes]
     with pytest.raises(ValueError):
         ops.gemm_grouped("tn", items)
-    for (a, b, _, _), c in zip(items, ops.gemm_grouped("tn", items, any_k=True)):
+    outs = ops.gemm_grouped("tn", items, any_k=True)
+    for (a, b, _, _), c in zip(items, outs):
         _check("tn", a, b, c)
+    # into kept gradients: the rounded product added and rounded again, bit for bit
+    rs = [torch.randn(c.shape, device=DEV, generator=g).to(BF) for c in outs]
+    want = [(r.float() + c.float()).to(BF) for r, c in zip(rs, outs)]
+    kept = ops.gemm_grouped("tn", [(a, b, r, r) for (a, b, _, _), r in zip(items, rs)], any_k=True)
+    for r, got, w in zip(rs, kept, want):
+        assert got.data_ptr() == r.data_ptr() and torch.equal(r, w)
 
 
 def test_any_k_rejects_what_it_cannot_read():
