@@ -12,7 +12,7 @@ from ctypes import POINTER, c_char_p, c_float, c_int, c_int64, c_size_t, c_void_
 from pathlib import Path
 
 LIB_PATH = Path(__file__).resolve().parent / "libfemtohip.so"
-ABI_VERSION = 6
+ABI_VERSION = 7
 
 FH_BF16 = 0
 FH_F32 = 1

@@ -40,7 +40,7 @@
 extern "C" {
 #endif
 
-#define FH_ABI_VERSION 6
+#define FH_ABI_VERSION 7
 
 typedef enum fh_dtype {
   FH_BF16 = 0, /* bfloat16 storage, fp32 arithmetic */

@@ -188,6 +188,23 @@ def test_library_exports_every_declared_symbol():
     assert _lib.lib().fh_abi_version() == _lib.ABI_VERSION
 
 
+# The declarations (sha256 of the header without comments and spaces) of an ABI version: a
+# change of either raises FH_ABI_VERSION, so that a stale library is refused.
+ABI_DECLARATIONS = (7, "dc9b32ad0af3a261")
+
+
+def test_abi_version_is_raised_with_the_declarations():
+    import hashlib
+
+    from femtotron_amd import _lib
+    text = re.sub(r"/\*.*?\*/", "", (ROOT / "include" / "femtohip.h").read_text(), flags=re.S)
+    version = int(re.search(r"#define FH_ABI_VERSION (\d+)", text).group(1))
+    text = re.sub(r"#define FH_ABI_VERSION \d+", "", text)
+    digest = hashlib.sha256(re.sub(r"\s+", "", text).encode()).hexdigest()[:16]
+    assert (version, digest) == ABI_DECLARATIONS, "declarations changed: raise FH_ABI_VERSION and record both"
+    assert _lib.ABI_VERSION == version
+
+
 def test_library_validates_arguments_on_host():
     """Invalid arguments are rejected before any HIP call (works without a GPU)."""
     from femtotron_amd import _lib
