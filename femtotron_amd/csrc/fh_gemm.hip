@@ -1178,7 +1178,7 @@ GemmPlan gemm_plan(int op, int64_t m, int64_t n, int64_t k) {
   const double per_slice = 48.0 * static_cast<double>(m) * n / (655360.0 * static_cast<double>(k));
   int best = 1;
   double best_cost = 1e30;
-  for (int s = 1; s <= 8 && s <= k / 256; ++s) {
+  for (int s = 1; s <= 8 && (s == 1 || s <= k / 256); ++s) {
     const double rounds = static_cast<double>((tiles * s + cus - 1) / cus);
     const double cost = rounds / s + (s > 1 ? per_slice * s : 0.0);
     if (cost < best_cost - 1e-9) {

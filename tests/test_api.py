@@ -255,6 +255,19 @@ def test_gradients_accumulate_in_the_gemm_only_where_it_can_write_them():
             assert got.shape == (24, 8) and got.data_ptr() == ps[0].grad.data_ptr()
 
 
+@pytest.mark.parametrize("m,n", [(11264, 2048), (6144, 4096), (4096, 14336), (4096, 11008), (28672, 4096)])
+def test_a_few_stages_are_not_split_over_the_chip(m, n):
+    """Weight gradients of 193 to 255 tokens (four stages, the last one ragged) run as those
+    of 192 and 256 do, in whole tiles: the stream form's segments would cost more than they."""
+    from femtotron_amd import _lib
+    if not _lib.LIB_PATH.exists():
+        pytest.skip("libfemtohip.so not built")
+    form = _lib.lib().fh_gemm_bf16_form
+    assert form(_lib.FH_GEMM_TN, m, n, 192, 0) == form(_lib.FH_GEMM_TN, m, n, 256, 0) == b"persist"
+    for k in (193, 200, 255):
+        assert form(_lib.FH_GEMM_TN, m, n, k, 0) == b"persist"
+
+
 def _group_workspace(shapes, k):
     from femtotron_amd import _lib
     probs = (_lib.FhGemmProblem * len(shapes))()
