@@ -101,23 +101,32 @@ def _chunk_rows(hidden2: torch.Tensor, weight: torch.Tensor, need_dw: bool) -> i
     return max(256, max(CHUNK_BYTES, w if sums else 0) // row // 256 * 256)
 
 
+def _acc_by_hand(V: int, H: int) -> bool:
+    """Whether a chunk's product is added to the fp32 sum by fh_gemm_bf16_acc: from 192
+    tiles of 256 x 256 on, as it splits no k and fewer leave CUs idle.  Hand-written and
+    library: 4096 x 32000 x 2048 481 and 575 us, x 512 level, x 256 103 and 83; 8192 x
+    1024 x 256 151 and 49 (the head of 140000 tokens 3.35 and 1.5 ms)."""
+    return V * H >= 192 * 256 * 256
+
+
 def _weight_grad(dlogits: torch.Tensor, x_c: torch.Tensor, dw32: torch.Tensor | None, first: bool, last: bool,
                  peak: int):
     """(dw or None, the running fp32 sum or None) after this chunk: dw appears
-    with the last one.  A last chunk that does not run hand-written (fp32, a width
-    that is no multiple of 8, fewer than 64 rows), or leaves no room for dw beside
-    its logits, leaves the rounding to the caller."""
+    with the last one.  A last chunk whose product is not added by hand (fp32, a
+    width that is no multiple of 8, fewer than 64 rows, few tiles), or that leaves no room for
+    dw beside its logits, leaves the rounding to the caller."""
     V, H = dlogits.size(1), x_c.size(1)
     if _choose_hand("tn", dlogits, x_c):
         if first and last:
             return ops.gemm("tn", dlogits, x_c, any_k=True), None
-        dw = None
-        if first:
-            dw32 = torch.empty(V, H, dtype=torch.float32, device=x_c.device)
-        elif last and 6 * dw32.numel() + 2 * dlogits.numel() <= peak:
-            dw = torch.empty(V, H, dtype=x_c.dtype, device=x_c.device)
-        ops.gemm_acc(dlogits, x_c, dw32, add=not first, out=dw)
-        return dw, dw32
+        if _acc_by_hand(V, H):
+            dw = None
+            if first:
+                dw32 = torch.empty(V, H, dtype=torch.float32, device=x_c.device)
+            elif last and 6 * dw32.numel() + 2 * dlogits.numel() <= peak:
+                dw = torch.empty(V, H, dtype=x_c.dtype, device=x_c.device)
+            ops.gemm_acc(dlogits, x_c, dw32, add=not first, out=dw)
+            return dw, dw32
     if first:
         dw32 = torch.zeros(V, H, dtype=torch.float32, device=x_c.device)
     if x_c.dtype == torch.float32:

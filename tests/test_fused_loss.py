@@ -196,11 +196,14 @@ def test_fused_loss_lowers_peak_activation_memory():
                                         (530, 264, 1000, 256),   # the last of 18: fewer than a hand-written product takes
                                         (520, 100, 1000, 256),   # a width that the hand-written products do not take
                                         (40, 2056, 1024, 256)])  # a wide one, and few rows
-def test_loss_head_in_chunks_matches_fp64(monkeypatch, dtype, N, H, V, rows):
+@pytest.mark.parametrize("by_hand", [True, False])
+def test_loss_head_in_chunks_matches_fp64(monkeypatch, dtype, N, H, V, rows, by_hand):
     """Loss and both gradients against fp64 with the logits and their gradient rounded where the head rounds them:
     every product sums in fp32 and rounds once, so only those roundings and the output's are left (bf16 2^-8 each)."""
     import femtotron_amd.fused_loss as fl
     monkeypatch.setattr(fl, "_chunk_rows", lambda *a: rows)
+    assert not fl._acc_by_hand(V, H)  # so small a vocabulary's sum is the library's
+    monkeypatch.setattr(fl, "_acc_by_hand", lambda *a: by_hand)
     g = torch.Generator().manual_seed(N + H)
     x = torch.randn(N, H, generator=g).to(dtype).to(DEV).requires_grad_(True)
     w = (torch.randn(V, H, generator=g) * H ** -0.5).to(dtype).to(DEV).requires_grad_(True)
@@ -215,6 +218,14 @@ def test_loss_head_in_chunks_matches_fp64(monkeypatch, dtype, N, H, V, rows):
     assert abs(loss.item() - want.item()) <= tol * abs(want.item())
     for got, ref in ((x.grad, x64.grad), (w.grad, w64.grad)):
         assert float((got.double() - ref).norm() / ref.norm()) < tol
+
+
+def test_a_chunk_is_added_by_hand_where_its_tiles_fill_the_chip():
+    """One tile of 256 x 256 per workgroup and no k split: a small vocabulary over many tokens (4 tiles over 131072
+    tokens: twice the head's time) stays with the library."""
+    import femtotron_amd.fused_loss as fl
+    assert fl._acc_by_hand(32000, 2048) and fl._acc_by_hand(128256, 256)
+    assert not fl._acc_by_hand(1024, 256) and not fl._acc_by_hand(32000, 256)
 
 
 @pytest.mark.gpu
