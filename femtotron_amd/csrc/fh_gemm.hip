@@ -1115,6 +1115,9 @@ int stream_grid() { return std::max(8, device_cus() / 8 * 8); }
 //     longer share operand blocks in L2 (TN 2048 x 5632 x 16384, 176 tiles:
 //     450 us against 361 us split in 4; 11264 x 2048, 352 tiles: 655-660
 //     against 685 us, 10240 x 2048: 644-666 against 754 us).
+//   A whole K is always a candidate, also with less than 256 k: four stages in the
+//   stream form cost more than the product (TN, 200 tokens: 11264 x 2048 60 us against
+//   26, 6144 x 4096 50 against 26, 4096 x 14336 76 against 49).
 struct GemmPlan {
   int slices;   // K slices of the split form
   bool stream;  // the stream form models faster

@@ -386,6 +386,18 @@ def test_any_k_matches_fp64_product(op, m, n, k, form, resid):
             assert torch.equal(ops.gemm(op, a, b, residual=r, out=r, any_k=True), want)
 
 
+@pytest.mark.parametrize("k", [65, 127, 129, 200, 255])
+def test_any_k_persistent_form_of_few_stages(k):
+    """Weight gradients of a ragged batch of few tokens: two to four stages per tile, the last one repeating k's, the
+    next tile's first stages loaded under them."""
+    g = torch.Generator(device=DEV).manual_seed(k)
+    a, b = _guarded(k, 11264, g), _guarded(k, 2048, g)
+    assert _form("tn", 11264, 2048, k, False) == "persist"
+    c = ops.gemm("tn", a, b, any_k=True)
+    _check("tn", a, b, c)
+    assert torch.equal(c, ops.gemm("tn", a, b, any_k=True))
+
+
 @pytest.mark.parametrize("k", [65, 127, 999, 2002])
 @pytest.mark.parametrize("shapes", [[(2560, 2048), (2048, 2048), (2048, 5632)], [(512, 256), (256, 256)]])
 def test_grouped_any_k_matches_each_product(shapes, k):
