@@ -147,8 +147,8 @@ __global__ __launch_bounds__(kWave) void k_clip_coef(const float* __restrict__ f
 // consecutive bytes (8 consecutive elements per thread are two 16-byte accesses at
 // a stride of 32), and what no kernel reads again before the next step (gradient,
 // master, m, v) moves non-temporally, which leaves L2 and the MALL to the
-// parameters.  Whole step, bf16 / fp32 parameters: 44 M 259 -> 220 / 320 -> 255 us,
-// 218 M 1225 -> 1179 / 1508 -> 1435, 923 M 5.24 -> 5.17 / 6.41 -> 6.19 ms (5.4-6.2
+// parameters.  Whole step, bf16 / fp32 parameters: 44 M 250 -> 223 / 318 -> 254 us,
+// 218 M 1223 -> 1172 / 1508 -> 1444, 923 M 5.24 -> 5.17 / 6.41 -> 6.19 ms (5.4-6.2
 // TB/s; a copy of 4 GiB reaches 4.7).  Non-temporal loads alone 255 / 308, stores
 // alone 260 / 316, the layout alone 260 / 316 us at 44 M.
 constexpr int kAdamQuads = static_cast<int>(kAdamChunk / (4 * kAdamThreads));

@@ -188,7 +188,8 @@ int fh_scale(fh_dtype dt, const void* x, void* out, int64_t n, const float* scal
  * j*head_dim.. of k/v/dk/dv; q head h reads kv head h / (n_heads/n_kv_heads).
  * head_dim in {32, 64, 128}; strides multiples of 8 and < 2^24; 16-byte
  * aligned bases.
- * FH_BF16 runs on MFMA (fp32 softmax/accumulation); FH_F32 in fp32 FMA.
+ * Both run on MFMA: FH_BF16 with fp32 softmax and accumulation, FH_F32 in fp32
+ * throughout.
  * lse: fp32 [batch, n_heads, seq_len], natural-log row log-sum-exp of the
  * scaled scores (nullable in the forward).
  */
