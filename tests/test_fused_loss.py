@@ -228,6 +228,28 @@ def test_a_chunk_is_added_by_hand_where_its_tiles_fill_the_chip():
     assert not fl._acc_by_hand(1024, 256) and not fl._acc_by_hand(32000, 256)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("need_dw", [True, False])
+def test_chunks_stay_within_their_room(dtype, need_dw):
+    """Logits beside the fp32 sum (or, in one chunk, the gradient alone): no more than 256 MB beside the sum, or than
+    rounding the sum; whole 256s of rows, at least 256; the fp32 head and one without a weight gradient as ever."""
+    import femtotron_amd.fused_loss as fl
+    for V in (1000, 1024, 32000, 128256, 1 << 20):
+        for H in (100, 256, 2048, 4096):
+            w = torch.empty(V, H, dtype=dtype, device="meta")
+            plain = max(256, (256 << 20) // (V * w.element_size()) // 256 * 256)
+            for N in (1, 63, 64, 300, 4096, 8192, 16385, 200000):
+                rows = fl._chunk_rows(torch.empty(N, H, dtype=dtype, device="meta"), w, need_dw)
+                W, L = V * H * 2, min(rows, N) * V * w.element_size()
+                if dtype == torch.float32 or not need_dw:
+                    assert rows == plain
+                elif rows == N and (N % 256 or rows != plain):  # all in one: no sum
+                    assert W + L <= max(2 * W + (256 << 20), 3 * W)
+                else:
+                    assert rows % 256 == 0 and rows >= plain
+                    assert 2 * W + L <= max(2 * W + (256 << 20), 3 * W) or rows == 256
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("N,H,V", [(16384, 256, 32000),   # the logits, 1000 MiB, are the larger part
                                    (9000, 2048, 32000),   # two chunks and a remainder
